@@ -90,7 +90,8 @@ def host_library(name: str, sources: list[str], compiler: str = "g++") -> str:
 
 # The kernel library's sources (every kernel hand-written: it links nothing
 # beyond the HIP runtime).
-KERNEL_SOURCES = ["rmsnorm.hip", "gemm.hip", "gemm_f32.hip", "rowops.hip", "bcast.hip"]
+KERNEL_SOURCES = ["rmsnorm.hip", "gemm.hip", "gemm_ring_n.hip", "gemm_ring_t.hip", "gemm_f32.hip",
+                  "rowops.hip", "bcast.hip"]
 KERNEL_LIBS: list[str] = []
 # The benchmark's own measurement probes (csrc/agk_bench.h): loaded by bench.py
 # only, not part of the product ABI.

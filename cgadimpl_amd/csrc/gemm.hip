@@ -12,13 +12,15 @@
 // (kscale multiplies the A operand as it is staged, rounding to bf16 as a
 // stored h would be; rowscale multiplies the fp32 accumulator.)
 //
-// Two kernels share the tile shape.  When K is a multiple of 64 and there is
-// no k-scale, the product runs on the direct-to-LDS kernel further below,
-// which stages whole 128-byte lines of either operand layout through two
-// 64-deep LDS stages without registers; otherwise the register-staged kernel
-// described here runs.
+// Three kernels.  A product without a k-scale runs on the direct-to-LDS kernel
+// further below (256 x 256 tiles, whole 128-byte lines of either operand layout
+// staged through two 64-deep LDS stages without registers) or, where those tiles
+// would leave CUs idle, on the ring kernel of gemm_ring.hpp (smaller tiles, more
+// bytes in flight); pick_shape chooses.  A k-scale, or a leading dimension too
+// large for the direct kernels' 31-bit offsets, takes the register-staged kernel
+// described here.
 //
-// Kernel shape.  A workgroup of 512 lanes (8 waves, 2 along M x 4 along N)
+// Register-staged kernel shape.  A workgroup of 512 lanes (8 waves, 2 along M x 4 along N)
 // computes a 256 x 256 tile of C; each wave owns 128 x 64 of it as 4 x 2
 // v_mfma_f32_32x32x16_bf16 accumulators (128 fp32 registers per lane).  K is
 // walked in steps of 64: the next step's A and B tiles are loaded from HBM /
@@ -48,50 +50,17 @@
 #include <atomic>
 
 #include "agk_rmsnorm.h"
+#include "gemm_common.hpp"
+#include "gemm_ring.hpp"
 
 namespace agk_gemm {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-constexpr int BM = 256, BN = 256, BK = 64;
+constexpr int BM = 256, BN = 256;
 constexpr int kThreads = 512;
 constexpr int kWavesN = 4;
 constexpr int WM = 128, WN = 64;            // per-wave tile
 constexpr int TM = WM / 32, TN = WN / 32;   // MFMA tiles per wave
-constexpr int kStride = BK;                 // bf16 per LDS row (128 bytes)
 constexpr int kStageElems = (BM + BN) * kStride;
-
-// LDS position of k-chunk c (8 bf16 = 16 bytes) of row `row`: chunks are
-// XOR-swizzled by the row's low bits, so the 8 lanes of a 16-byte fragment
-// read (8 consecutive rows, one chunk) and the 8-byte writes of the
-// transposing stager (rows 8 apart) land on different banks.
-__device__ __forceinline__ int lds_off(int row, int c) {
-    return row * kStride + ((c ^ (row & 7) ^ ((row >> 3) & 7)) << 3);
-}
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// fp32 -> bf16, round to nearest even (v_cvt_pk_bf16_f32: NaN stays NaN).
-__device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-    return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
-}
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
-}
-// lo16(a) | lo16(b) << 16 and hi16(a) | hi16(b) << 16 (v_perm_b32)
-__device__ __forceinline__ uint32_t lo_pair(uint32_t a, uint32_t b) {
-    return __builtin_amdgcn_perm(b, a, 0x05040100u);
-}
-__device__ __forceinline__ uint32_t hi_pair(uint32_t a, uint32_t b) {
-    return __builtin_amdgcn_perm(b, a, 0x07060302u);
-}
 
 // ---- operand staging --------------------------------------------------------
 // An operand tile is R = 256 rows (of A: m, of B: n) by BK = 64 k.
@@ -186,45 +155,6 @@ __device__ __forceinline__ void store_tile(const Stage<KCONTIG>& s, uint16_t* ld
             *reinterpret_cast<u32x2*>(lds + lds_off(r + 2 * w + 1, kq >> 3) + (kq & 7)) = odd;
         }
     }
-}
-
-__device__ __forceinline__ bf16x8 lds_frag(const uint16_t* lds, int row, int k) {
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lds + lds_off(row, k >> 3)));
-}
-
-// ---- tile order ----------------------------------------------------------------
-// Workgroups are dispatched round-robin over the 8 XCDs (workgroup L runs on
-// XCD L % 8), each XCD with its own L2.  The tile order below gives each XCD
-// a contiguous chunk of a grouped ordering (group_m m-tiles x all n-tiles,
-// column by column), so the ~32 workgroups resident on one XCD at a time
-// cover about group_m x 32 / group_m tiles and share their A row-panels and B
-// column-panels in that XCD's L2, instead of every neighbouring tile landing
-// on a different XCD.  group_m = 4 unless a measured order is known for the
-// shape (tuned_group_m).
-constexpr int kXcds = 8;
-constexpr int kGroupM = 4;
-
-__device__ __forceinline__ void tile_of(int L, int tiles_m, int tiles_n, int group_m, int& tm,
-                                        int& tn) {
-    const int T = tiles_m * tiles_n;
-    const int x = L % kXcds, s = L / kXcds;
-    const int q = T / kXcds, r = T % kXcds;  // XCDs below r get q + 1 tiles
-    const int g = x < r ? x * (q + 1) + s : r * (q + 1) + (x - r) * q + s;
-    const int per_group = group_m * tiles_n;
-    const int group = g / per_group;
-    const int gm0 = group * group_m;
-    const int gsize = tiles_m - gm0 < group_m ? tiles_m - gm0 : group_m;
-    const int in = g - group * per_group;
-    tm = gm0 + in % gsize;
-    tn = in / gsize;
-}
-
-// The product rounded to bf16, plus a bf16 bias term (then rounded again when
-// stored): `matmul(X, W^T) + b` with its two roundings, as a bf16 product and
-// a bf16 sum give them.
-__device__ __forceinline__ float with_bias(float v, uint16_t b) {
-    v = __uint_as_float(f32_to_bf16_bits(v) << 16);
-    return v + __uint_as_float(static_cast<uint32_t>(b) << 16);
 }
 
 // ---- the kernel ---------------------------------------------------------------
@@ -337,92 +267,15 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(
     }
 }
 
-// ---- direct-to-LDS kernel: both operands k-contiguous, K a multiple of 64 ----
+// ---- direct-to-LDS kernel -----------------------------------------------------
 // Staging without registers: buffer_load_dwordx4 ... lds writes lane l's 16
 // bytes to LDS at (wave-uniform base) + 16 * l, so one wave instruction fills
 // a contiguous kilobyte of LDS; each lane fetches the global chunk that belongs
 // at its position of the swizzled layout.  Rows past M or N are fetched from
-// the last valid row (never stored).  The epilogue store_c writes the wave's
-// 128 x 64 block of C.
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// GENERAL: rowscale, a column bias (bf16 output only) and accumulate
-// honoured; CHECK: rows past M and columns past N skipped.  store_c picks the
-// variant once per call (uniform values), so the common plain, interior store
-// has no per-element branches.
-template <bool OUT_F32, bool GENERAL, bool CHECK>
-__device__ __forceinline__ void store_c_impl(const f32x16 (&acc)[TM][TN], void* __restrict__ C,
-                                             int64_t ldc, int M, int N, int m0, int n0, int wm,
-                                             int wn, int lane, const float* __restrict__ rowscale,
-                                             const uint16_t* __restrict__ colbias,
-                                             int accumulate) {
-    const int col_l = lane & 31;
-    const int row_l = 4 * (lane >> 5);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int row = m0 + wm * WM + i * 32 + 8 * (e >> 2) + row_l + (e & 3);
-            if (CHECK && row >= M) continue;
-            float rs = 1.0f;
-            if constexpr (GENERAL) rs = rowscale ? rowscale[row] : 1.0f;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int col = n0 + wn * WN + j * 32 + col_l;
-                if (CHECK && col >= N) continue;
-                float v = acc[i][j][e];
-                if constexpr (GENERAL) {
-                    v *= rs;
-                    // accumulation rounds the product first (no fused multiply-add)
-                    asm volatile("" : "+v"(v));
-                }
-                if constexpr (OUT_F32) {
-                    float* p = static_cast<float*>(C) + static_cast<int64_t>(row) * ldc + col;
-                    if constexpr (GENERAL) {
-                        *p = accumulate ? *p + v : v;
-                    } else {
-                        // Plain fp32 stores are whole 128-byte lines per 32 lanes:
-                        // non-temporal, so a round's C tiles (64 MB) do not evict
-                        // the operand panels from L2 and stream out as they come.
-                        // Measured on dW at c5 (4096 x 11008 x 8192, one box, three
-                        // alternations): 557-561 -> 528-529 us.  bf16 outputs keep
-                        // ordinary stores: no gain there, and the RMSNorm backward
-                        // reads dh from the caches right after its product.
-                        __builtin_nontemporal_store(v, p);
-                    }
-                } else {
-                    uint16_t* p = static_cast<uint16_t*>(C) + static_cast<int64_t>(row) * ldc + col;
-                    if constexpr (GENERAL) {
-                        if (accumulate) v = __uint_as_float(static_cast<uint32_t>(*p) << 16) + v;
-                        if (colbias) v = with_bias(v, colbias[col]);
-                    }
-                    *p = static_cast<uint16_t>(f32_to_bf16_bits(v));
-                }
-            }
-        }
-    }
-}
-
-// bn: the columns the calling tile covers from n0 (BN, or BN / 2 for a half tile).
-template <bool OUT_F32>
-__device__ __forceinline__ void store_c(const f32x16 (&acc)[TM][TN], void* __restrict__ C,
-                                        int64_t ldc, int M, int N, int m0, int n0, int wm, int wn,
-                                        int lane, const float* __restrict__ rowscale,
-                                        const uint16_t* __restrict__ colbias, int accumulate,
-                                        int bn = BN) {
-    if (rowscale != nullptr || colbias != nullptr || accumulate) {
-        store_c_impl<OUT_F32, true, true>(acc, C, ldc, M, N, m0, n0, wm, wn, lane, rowscale,
-                                          colbias, accumulate);
-    } else if (m0 + BM <= M && n0 + bn <= N) {
-        store_c_impl<OUT_F32, false, false>(acc, C, ldc, M, N, m0, n0, wm, wn, lane, nullptr,
-                                            nullptr, 0);
-    } else {
-        store_c_impl<OUT_F32, false, true>(acc, C, ldc, M, N, m0, n0, wm, wn, lane, nullptr,
-                                           nullptr, 0);
-    }
-}
-
-// ---- direct-to-LDS kernel -----------------------------------------------------
+// the last valid row (never stored).  The epilogue store_block writes the wave's
+// block of C.  K % 64 k at the end of K are staged through registers with
+// zeros past K (stage_k_tail) and multiplied before the whole k-tiles.
+//
 // The same 256 x 256 tile, over 4 waves of 128 x 128 (2 x 2; 4 x 4 MFMA tiles
 // per wave, whose 256 accumulator registers live in AGPRs).  K is walked in
 // 64-deep tiles through two LDS stages of 64 KiB (32 KiB per operand), filled by
@@ -459,9 +312,6 @@ __device__ __forceinline__ void store_c(const f32x16 (&acc)[TM][TN], void* __res
 // of the tile each wave waits for its own loads and reads, then the barrier.
 constexpr int kDirectThreads = 256;
 constexpr int kTrRow = 256;               // bf16 per LDS row of a k-strided operand
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
 
 // Element offset of column col (a multiple of 4) of k-row k in a k-strided stage.
 __device__ __forceinline__ int tr_off(int k, int col) {
@@ -623,10 +473,14 @@ __device__ __forceinline__ void direct_step(const DirectStage& d, const uint16_t
 // One tile's k loop and store.  NB = 4: the 256 x 256 tile at (m0, n0), wave
 // (wm, wn) owning its 128 x 128 block; NB = 2: the 256 x 128 half of that tile
 // starting at column n0 + half_off, wave (wm, wn) owning a 128 x 64 block.
-// Both stage the tile's full 256 B columns (the same loads).
-template <bool OUT_F32, bool A_TR, bool B_TR, int NB>
+// Both stage the tile's full 256 B columns (the same loads).  TAIL: K is not a
+// multiple of 64; the last K % 64 k are multiplied first, staged through
+// registers into st1 (which tile 1's loads fill only after it).
+template <bool OUT_F32, bool A_TR, bool B_TR, int NB, bool TAIL>
 __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0, uint16_t* st1,
-                                            void* __restrict__ C, int64_t ldc, int M, int N,
+                                            const uint16_t* __restrict__ a0, int64_t lda,
+                                            int rows_a, const uint16_t* __restrict__ b0,
+                                            int64_t ldb, int rows_b, void* __restrict__ C, int64_t ldc, int M, int N,
                                             int K, int m0, int n0, int half_off, int wm, int wn,
                                             int lane, int wave,
                                             const float* __restrict__ rowscale,
@@ -640,12 +494,25 @@ __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0,
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    const int nk = K / BK;  // >= 1: K is a positive multiple of 64
+    const int nk = K / BK;  // >= 1
     const int frow = lane & 31;
     const int fk = (lane >> 5) * 8;  // MFMA operand lanes 32..63 hold k 8..15
     const int bc = half_off + wn * (NB * 32);  // the wave's first B column in the stage
+    if constexpr (TAIL) {
+        stage_k_tail<A_TR, BM>(st1, a0, lda, rows_a, nk * BK, K);
+        stage_k_tail<B_TR, BN>(st1 + BM * BK, b0, ldb, rows_b, nk * BK, K);
+    }
     direct_issue_a(d, st0, 0, wave);
     direct_issue_b(d, st0, 0, wave);
+    if constexpr (TAIL) {
+        stage_barrier<16>();  // the tail's LDS writes, every wave (tile 0 still in flight)
+        for (int s = 0; s * 16 < K - nk * BK; ++s) {
+            Frags<NB> f;
+            read_frags<A_TR, B_TR>(f, st1, s, wm, bc, frow, fk, lane);
+            mfma_sub(f, acc);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -664,7 +531,7 @@ __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0,
     mfma_sub(f1, acc);  // substep 3 of the last tile
 
     if constexpr (NB == 4) {
-        // the wave's 128 x 128 block leaves as two 128 x 64 halves (store_c's layout)
+        // the wave's 128 x 128 block leaves as two 128 x 64 halves
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             f32x16 part[TM][TN];
@@ -672,12 +539,12 @@ __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0,
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) part[i][j] = acc[i][h * TN + j];
-            store_c<OUT_F32>(part, C, ldc, M, N, m0, n0, wm, 2 * wn + h, lane, rowscale, colbias,
-                             accumulate);
+            store_block<OUT_F32>(part, C, ldc, M, N, m0 + wm * WM, n0 + (2 * wn + h) * WN, lane,
+                                 rowscale, colbias, accumulate);
         }
     } else {
-        store_c<OUT_F32>(acc, C, ldc, M, N, m0, n0 + half_off, wm, wn, lane, rowscale, colbias,
-                         accumulate, BN / 2);
+        store_block<OUT_F32>(acc, C, ldc, M, N, m0 + wm * WM, n0 + half_off + wn * WN, lane,
+                             rowscale, colbias, accumulate);
     }
 }
 
@@ -688,7 +555,7 @@ __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0,
 // (workgroup full_tiles + 2 h + q: half q of tile full_tiles + h), so that a
 // last round of few tiles runs on twice as many CUs for half as long.  Every
 // output element is summed in the same k order either way (bit-identical).
-template <bool OUT_F32, bool A_TR, bool B_TR>
+template <bool OUT_F32, bool A_TR, bool B_TR, bool TAIL>
 __global__ __launch_bounds__(kDirectThreads) void gemm_nt_direct_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
     void* __restrict__ C, int64_t ldc, int M, int N, int K, const float* __restrict__ rowscale,
@@ -713,17 +580,17 @@ __global__ __launch_bounds__(kDirectThreads) void gemm_nt_direct_kernel(
 
     const int rows_a = M - m0 < BM ? M - m0 : BM;
     const int rows_b = N - n0 < BN ? N - n0 : BN;
+    const uint16_t* a0 = A_TR ? A + m0 : A + static_cast<int64_t>(m0) * lda;
+    const uint16_t* b0 = B_TR ? B + n0 : B + static_cast<int64_t>(n0) * ldb;
     DirectStage d;
     // the resources span the bytes the tile's loads can address (their k
     // position is the scalar offset, always inside the operand)
     d.ra = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(A_TR ? A + m0 : A + static_cast<int64_t>(m0) * lda),
-        static_cast<short>(0),
+        const_cast<uint16_t*>(a0), static_cast<short>(0),
         static_cast<int>(A_TR ? ((K - 1) * lda + rows_a) * 2 : ((rows_a - 1) * lda + K) * 2),
         0x00020000);
     d.rb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(B_TR ? B + n0 : B + static_cast<int64_t>(n0) * ldb),
-        static_cast<short>(0),
+        const_cast<uint16_t*>(b0), static_cast<short>(0),
         static_cast<int>(B_TR ? ((K - 1) * ldb + rows_b) * 2 : ((rows_b - 1) * ldb + K) * 2),
         0x00020000);
     d.step_a = A_TR ? static_cast<int>(BK * lda * 2) : BK * 2;
@@ -732,12 +599,14 @@ __global__ __launch_bounds__(kDirectThreads) void gemm_nt_direct_kernel(
     direct_offsets<B_TR>(d.ob, wave, lane, rows_b, ldb);
 
     if (!halves)
-        direct_tile<OUT_F32, A_TR, B_TR, 4>(d, st0, st1, C, ldc, M, N, K, m0, n0, 0, wm, wn, lane,
-                                            wave, rowscale, colbias, accumulate);
+        direct_tile<OUT_F32, A_TR, B_TR, 4, TAIL>(d, st0, st1, a0, lda, rows_a, b0, ldb, rows_b,
+                                                  C, ldc, M, N, K, m0, n0, 0, wm, wn, lane, wave,
+                                                  rowscale, colbias, accumulate);
     else
-        direct_tile<OUT_F32, A_TR, B_TR, 2>(d, st0, st1, C, ldc, M, N, K, m0, n0,
-                                            ((L - full_tiles) & 1) * (BN / 2), wm, wn, lane,
-                                            wave, rowscale, colbias, accumulate);
+        direct_tile<OUT_F32, A_TR, B_TR, 2, TAIL>(d, st0, st1, a0, lda, rows_a, b0, ldb, rows_b,
+                                                  C, ldc, M, N, K, m0, n0,
+                                                  ((L - full_tiles) & 1) * (BN / 2), wm, wn,
+                                                  lane, wave, rowscale, colbias, accumulate);
 }
 
 // C for an empty reduction (K == 0): zeros, or the bf16 column bias in every
@@ -909,17 +778,67 @@ inline int tuned_group_m(int tiles_m, int tiles_n, int nk, bool a_tr, bool b_tr)
     return kGroupM;
 }
 
-// Whether a call takes the direct-to-LDS kernel.  A k-scale keeps the call on
-// the register-staged kernel: the direct kernel's loads go from memory to LDS
-// without passing registers, so the scale would have to be applied to every A
-// fragment after its LDS read (unpack, multiply, round, repack: about 20 VALU
-// operations per fragment).  Measured on MI355X for y (8192 x 11008 x 4096,
-// A k-contiguous, the scale staged in LDS), that variant was bit-identical to
-// the staged kernel's but ran 759-819 us against 551 us without the scale,
-// while all it saves the RMSNorm + linear layer is writing and reading h
-// (about 15 us).
-inline bool direct_eligible(int64_t K, const float* kscale) {
-    return kscale == nullptr && K % BK == 0;
+template <bool A_TR, bool B_TR>
+int launch_direct(bool f32, const GemmCall& c) {
+    const int tiles_m = (c.M + BM - 1) / BM, tiles_n = (c.N + BN - 1) / BN;
+    const int gm = tuned_group_m(tiles_m, tiles_n, c.K / BK, A_TR, B_TR);
+    const int tiles = tiles_m * tiles_n;
+    const int full = direct_full_tiles(tiles, device_cus());
+    const dim3 grid(full + 2 * (tiles - full)), block(kDirectThreads);
+#define AGK_DIRECT(F32, TAIL)                                                                  \
+    hipLaunchKernelGGL((gemm_nt_direct_kernel<F32, A_TR, B_TR, TAIL>), grid, block, 0, c.st,   \
+                       c.A, c.lda, c.B, c.ldb, c.C, c.ldc, c.M, c.N, c.K, c.rowscale,          \
+                       c.colbias, c.accumulate, tiles_m, tiles_n, gm, full)
+    const bool tail = c.K % BK != 0;
+    if (f32) {
+        if (tail) AGK_DIRECT(true, true);
+        else AGK_DIRECT(true, false);
+    } else {
+        if (tail) AGK_DIRECT(false, true);
+        else AGK_DIRECT(false, false);
+    }
+#undef AGK_DIRECT
+    return hipGetLastError() == hipSuccess ? AGK_OK : AGK_EHIP;
+}
+
+// The kernel and tile a product runs on: 0 the direct kernel's 256 x 256
+// tiles, otherwise a ring shape.  The cost of a shape is its rounds of tiles
+// over the CUs times a k-step's time, which depends on how full the round is
+// (the loads of a full chip queue behind each other; the MFMAs of a full chip
+// lower the clock): light for a round of few workgroups, full for a full one,
+// light + (full - light) * fill^2 between.  The two times per shape were
+// measured on MI355X (random bf16, k-contiguous operands, K = 4096: 512 and
+// 8192 rows by 4096 columns); with them the rule came within 10 % of the best
+// shape's time at every product of the sweep:
+//   rows x columns x K (us)   256x256  ring shape taken   other shapes
+//   512 x 4096 x 4096              58      22 (128x64)    22-42
+//   1032 x 4096 x 4096             65      39 (192x128)   39-73
+//   2048 x 4096 x 4096             84      57 (128x256)   59-137
+//   4096 x 4096 x 1032             36      -              38-77
+//   8192 x 4096 x 4096            204      -              225-489
+// Each round also costs about four steps (first loads, epilogue).
+inline int pick_shape(int M, int N, int K, int cus) {
+    if (K < BK) return kRingSmallK;
+    int best = 0;
+    double best_cost = 0.0;
+    for (const RingCost& s : kRingCosts) {
+        const double tiles = static_cast<double>((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        const double slots = static_cast<double>(cus) * s.per_cu;
+        const double rounds = static_cast<double>(static_cast<int64_t>(tiles / slots));
+        const double fill = tiles / slots - rounds;
+        const double step = rounds * s.full + (fill > 0 ? s.light + (s.full - s.light) * fill * fill : 0.0);
+        const double cost = step * (static_cast<double>(K) / BK + 4.0);
+        if (s.id == 0 || cost < best_cost) {
+            best = s.id;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <bool A_TR, bool B_TR>
+int launch_tiled(int shape, bool f32, const GemmCall& c) {
+    return shape == 0 ? launch_direct<A_TR, B_TR>(f32, c) : launch_ring<A_TR, B_TR>(shape, f32, c);
 }
 
 // No layout needs a workspace: the direct kernel stages either layout of each
@@ -986,34 +905,19 @@ int gemm_impl(const void* A, int64_t lda, int a_trans, const void* B, int64_t ld
         return (tr ? (K - 1) * ld + BM : (BM - 1) * ld + K) * 2 <= 0x7fffffffLL;
     };
     const bool a_tr = a_trans != 0, b_tr = b_trans == 0;
-    if (direct_eligible(K, kscale) && fits(lda, a_tr) && fits(ldb, b_tr)) {
-        const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
-        const int gm = tuned_group_m(tiles_m, tiles_n, k / BK, a_tr, b_tr);
-        const int tiles = tiles_m * tiles_n;
-        const int full = direct_full_tiles(tiles, device_cus());
-        const dim3 grid(full + 2 * (tiles - full)), block(kDirectThreads);
+    if (kscale == nullptr && fits(lda, a_tr) && fits(ldb, b_tr)) {
         const uint16_t* a16 = static_cast<const uint16_t*>(A);
         const uint16_t* b16 = static_cast<const uint16_t*>(B);
-#define AGK_DIRECT(F32, ATR, BTR)                                                              \
-    hipLaunchKernelGGL((gemm_nt_direct_kernel<F32, ATR, BTR>), grid, block, 0, st, a16, lda, b16, \
-                       ldb, C, ldc, m, n, k, rowscale, colbias, acc, tiles_m, tiles_n, gm, full)
+        const int shape = pick_shape(m, n, k, device_cus());
+        const GemmCall call{a16, lda, b16, ldb, C, ldc, m, n, k, rowscale, colbias, acc, st};
         const bool f32 = c_dtype == AGK_F32;
-        if (f32) {
-            if (a_tr && b_tr) AGK_DIRECT(true, true, true);
-            else if (a_tr) AGK_DIRECT(true, true, false);
-            else if (b_tr) AGK_DIRECT(true, false, true);
-            else AGK_DIRECT(true, false, false);
-        } else {
-            if (a_tr && b_tr) AGK_DIRECT(false, true, true);
-            else if (a_tr) AGK_DIRECT(false, true, false);
-            else if (b_tr) AGK_DIRECT(false, false, true);
-            else AGK_DIRECT(false, false, false);
-        }
-#undef AGK_DIRECT
-        return hipGetLastError() == hipSuccess ? AGK_OK : AGK_EHIP;
+        if (a_tr) return b_tr ? launch_tiled<true, true>(shape, f32, call)
+                              : launch_tiled<true, false>(shape, f32, call);
+        return b_tr ? launch_tiled<false, true>(shape, f32, call)
+                    : launch_tiled<false, false>(shape, f32, call);
     }
-    // Leading dimensions too large for the direct kernel's offsets, K not a
-    // multiple of 64, or a k-scale: the register-staged kernel.
+    // Leading dimensions too large for the direct kernels' offsets, or a
+    // k-scale: the register-staged kernel.
     const bool ak = !a_trans, bk = b_trans != 0, ks = kscale != nullptr;
     const uint16_t* cb = colbias;
     if (ak && bk) return dispatch_ks<true, true>(ks, c_dtype, A, lda, B, ldb, C, ldc, m, n, k, kscale, rowscale, cb, acc, st);

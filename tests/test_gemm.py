@@ -1,9 +1,8 @@
 """bf16 GEMM on MFMA (agk_gemm_bf16) and the bf16 transpose, through the C ABI.
 
-GPU: every operand layout (the direct-to-LDS kernel reads k-contiguous operands
-with 16-byte LDS reads and k-strided ones with transposing reads; K not a
-multiple of 64 and the k-scale take the register-staged kernel), the k- and
-row-scales, fp32 and bf16 output, accumulation and ragged sizes, each against a
+GPU: every operand layout (the direct-to-LDS kernels read k-contiguous operands
+with 16-byte LDS reads and k-strided ones with transposing reads; the k-scale
+takes the register-staged kernel), every tile shape, the k- and row-scales, fp32 and bf16 output, accumulation and ragged sizes, each against a
 plain PyTorch fp32 product of the same bf16 operands; transposes bit-exact;
 repeated calls bit-identical; the four layouts of one product bit-identical.
 CPU: argument validation and the workspace rule.
@@ -59,8 +58,8 @@ def _ref(a, b, ta, tb, ks, rs):
     return C
 
 
-# K / 64 = 1, 2, 3, 5, 7, 16 on the direct-to-LDS kernel (K a multiple of 64):
-# odd and even tile counts of its peeled two-stage loop, with ragged M and N tiles.
+# K / 64 = 1, 2, 3, 5, 7, 16 and K with a tail: odd and even tile counts of the peeled
+# k loops, with ragged M and N tiles.
 CASES = [(256, 256, 64), (264, 520, 72), (8, 8, 8), (1000, 1032, 520), (512, 768, 1024),
          (136, 264, 192), (264, 520, 128), (520, 264, 320), (200, 136, 448)]
 
@@ -94,6 +93,31 @@ def test_gemm_against_torch(cuda, M, N, K, ta, tb, ws):
     r = _ref(a, b, ta, tb, None, None) + base
     assert ((c - r).abs().max() / r.abs().max()).item() <= 1e-5
     assert torch.equal(c, c2)
+
+
+# One size per tile shape the dispatch picks (256 x 256 last), with ragged last tiles;
+# K: only a tail (40), one and two whole k-tiles with and without a tail, and more
+# k-tiles than the ring has stages.
+SHAPE_CASES = [(456, 5376), (688, 5392), (336, 5624), (1168, 4864), (5416, 664), (5808, 1032),
+               (392, 4840), (72, 136), (3392, 2320)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", SHAPE_CASES)
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 1), (1, 0)])
+def test_gemm_tile_shapes(cuda, M, N, ta, tb):
+    """Every tile shape, layout and kind of K: fp32 output against a float64 product.  The bar
+    is that of fp32 sums of exact products, K 2^-24 |a| |b| per element (K <= 456)."""
+    import torch
+    torch.manual_seed(M * 5 + N + 2 * ta + tb)
+    for K in (40, 64, 72, 128, 200, 456):
+        a = torch.randn((K, M) if ta else (M, K), device=cuda).bfloat16()
+        b = torch.randn((N, K) if tb else (K, N), device=cuda).bfloat16()
+        A, B = (a.t() if ta else a).double(), (b.t() if tb else b).double()
+        c = agk.gemm_bf16(a, b, trans_a=bool(ta), trans_b=bool(tb), out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        bound = K * 2.0 ** -24 * (A.abs() @ B.abs())
+        assert ((c.double() - A @ B).abs() <= bound).all().item(), (M, N, K, ta, tb)
 
 
 @pytest.mark.gpu
