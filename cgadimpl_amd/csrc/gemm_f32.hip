@@ -7,35 +7,42 @@
 //
 //   C[M][ldc] (+)= op(A) op(B)
 //
-// Shape.  A workgroup of 256 lanes (4 waves, 2 x 2) computes a TILE x TILE
-// tile of C; each wave owns (TILE / 2)^2 of it as 32 x 32 MFMA accumulators
-// (TILE 128: 2 x 2 of them, 64 AGPRs).  Products with fewer 128-tiles than
-// the GPU has CUs take TILE 64 (four times the workgroups).
-// K is walked in steps of 16 through two LDS stages (40 KiB per workgroup, so
-// four workgroups share a CU and hide each other's load latency): the next
-// step's 8 + 8 values per lane are loaded into registers while the current
-// step is multiplied, then written to the other stage (one barrier per step).
+// Tiled kernel.  A workgroup of 256 lanes (4 waves, 2 x 2) computes a BM x BN
+// tile of C; each wave owns a quarter of it as 32 x 32 MFMA accumulators.  K
+// is walked in steps of 32 through two LDS stages: the loads of step t + 2 are
+// issued while step t is multiplied and step t + 1's values, loaded a step
+// earlier, are written to the other stage (one barrier per step).  An fp32
+// MFMA takes 64 cycles, so a step's MFMAs (0.4 us per wave and 32 x 32 block)
+// outlast everything else once a step's loads have two steps to arrive; with
+// one step of 16 k to arrive in, as before, the wait for them set the pace.
 //
 // Operands.  Each operand is staged as a logical [rows][K] matrix (A: M rows,
-// B: N rows) into LDS laid out [k][row], whatever its memory layout:
-//  - k contiguous in memory (A as [M][K], B given as B^T [N][K]): lane t loads
-//    k (t % 4) * 4 .. + 3 of rows t / 4 + 64 i as one 16-byte access when the
-//    rows are 16-byte aligned, else k = t % 16 of rows t / 16 + 16 i (16
-//    neighbouring lanes read 64 contiguous bytes either way);
-//  - rows contiguous (A given as A^T [K][M], B as [K][N]): lane t loads row
-//    t % 128 of k = t / 128 + 2 i, 128 neighbouring lanes 512 bytes.
-// Elements outside the matrix are staged as zeros, so edge tiles need no
-// other special case.  LDS k-rows are kStride = 160 floats apart: k and k + 1
-// start 32 banks apart, so an MFMA operand read (lanes 0-31 at k, 32-63 at
-// k + 1, 32 consecutive rows each) touches every bank once.
+// B: N rows) into LDS rows of 32 k (128 bytes, 16-byte chunks XOR-swizzled by
+// the row), whatever its memory layout:
+//  - k contiguous in memory (A as [M][K], B given as B^T [N][K]): 8 lanes load a
+//    row's 128 bytes and store them as they are;
+//  - rows contiguous (A given as A^T [K][M], B as [K][N]): a lane loads four
+//    rows at each of BM / 32 consecutive k and stores BM / 32 k of each row.
+// Every load is four consecutive floats, which needs only 4-byte alignment.
+// Rows past the matrix repeat valid ones (their products are not stored); k
+// past K are staged as zeros.
+// An MFMA multiplies two k; which two is free as long as A and B agree, so a
+// lane takes four consecutive k of its row as one 16-byte LDS read (lanes 0-31
+// k 8 s .. + 3 of substep s, lanes 32-63 k 8 s + 4 .. + 7) and spends them on
+// four MFMAs.
+//
+// Split kernel.  A product with too few tiles for the CUs runs one 32 x 32
+// tile per workgroup, its four waves taking the 32-deep steps of K in turn
+// (no LDS staging: operands go from memory to the MFMA's registers), their
+// sums added in wave order through LDS.
 //
 // MFMA lane layout (the 32 x 32 block instructions' layout, as in gemm.hip):
 // A operand lane l holds row l % 32, k = l / 32; B operand lane l holds
 // column l % 32, the same k; accumulator element e of lane l is
 // C[8 * (e / 4) + 4 * (l / 32) + e % 4][l % 32].
 //
-// Determinism: every output element is summed in the same k order in every
-// call (no split-K, no atomics), so results are bit-identical run to run.
+// Determinism: every output element is summed in an order fixed by the sizes
+// (no atomics), so results are bit-identical run to run.
 // Rounding: fp32 products and sums in the matrix core; the bound is that of
 // fp32 summation, |C - exact| <= (K + 1) 2^-24 (|A| |B|).
 
@@ -44,158 +51,400 @@
 #include <stdint.h>
 
 #include "agk_rmsnorm.h"
+#include "gemm_common.hpp"
 #include "rowcommon.hpp"
 
 namespace agk_sgemm {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));  // in memory, at any float
 
-constexpr int BK = 16;
-constexpr int kThreads = 256;
-constexpr int kStride = 160;              // floats per LDS k-row (at most 128 used)
-constexpr int kStage = BK * kStride;      // floats per operand per stage
+constexpr int BK = 32;
 
-// One operand's values for one k-step: element (row r0 + row, k0 + k) of the
-// logical [rows][K] matrix, at p[row * ld + k] (KC) or p[k * ld + row] (!KC);
-// TILE * BK / 256 values per lane.
-// KC with VEC (16-byte aligned rows, ld a multiple of 4): lane t loads the
-// four k (t % 4) * 4 .. + 3 of rows t / 4 + 64 i as one 16-byte access (a
-// group of four k past K element by element).
-template <int TILE, bool KC, bool VEC>
-__device__ __forceinline__ void load_step(float (&v)[TILE * BK / kThreads],
-                                          const float* __restrict__ p, int64_t ld, int r0,
-                                          int rows, int k0, int K) {
-    const int t = threadIdx.x;
-    if constexpr (KC && VEC) {
-        typedef float f32x4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-        for (int i = 0; i < TILE * BK / kThreads / 4; ++i) {
-            const int row = t / 4 + (kThreads / 4) * i;
-            const int gr = r0 + row, gk = k0 + (t % 4) * 4;
-            f32x4 q = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (gr < rows) {
-                const float* a = p + static_cast<int64_t>(gr) * ld + gk;
-                if (gk + 3 < K) {
-                    q = *reinterpret_cast<const f32x4*>(a);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) q[e] = gk + e < K ? a[e] : 0.0f;
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * i + e] = q[e];
-        }
-        return;
+// Float offset of 16-byte chunk c (0..7) of LDS row `row`: two rows share 256
+// bytes (all 64 banks), whose 16 chunks are XOR-swizzled by the row pair.  The
+// 16 lanes a 16-byte access serves at a time (rows 0-7 and 24-31 of one chunk,
+// or 8 row quads of two chunks) then touch every bank once.
+__device__ __forceinline__ int chunk_off(int row, int c) {
+    return (row >> 1) * (2 * BK) + (((((row & 1) << 3) | c) ^ ((row >> 1) & 15)) << 2);
+}
+
+// One operand's 32-deep step of ROWS rows, as a lane holds it between its
+// loads and its LDS writes: ROWS / 32 quads.
+template <int ROWS>
+struct Step {
+    f32x4 v[ROWS / 32];
+};
+
+// What lane t of 256 loads of the operand whose rows r0 .. start at p, fixed for
+// all steps.  KC: quad i holds k (t % 8) * 4 .. + 3 of row t / 8 + 32 i.
+// Otherwise quad i holds four rows at k + i; 8 lanes cover 32 rows (128 bytes).
+template <bool KC, int ROWS>
+struct Place {
+    const float* p;    // the quad's address at k = 0, quad 0
+    int64_t ld;
+    int rows;          // valid rows of the tile
+    int r, k;          // first row and first k of the lane's quads, as staged
+    int from;          // !KC: the first row loaded (below r by `shift` at the matrix's edge)
+    int shift;
+    bool edge;         // !KC: some lane of the workgroup has a shift
+};
+
+template <bool KC, int ROWS>
+__device__ __forceinline__ Place<KC, ROWS> place(const float* __restrict__ src, int64_t ld, int r0,
+                                                 int rows_total, int t) {
+    Place<KC, ROWS> q;
+    q.ld = ld;
+    q.rows = rows_total - r0 < ROWS ? rows_total - r0 : ROWS;
+    q.shift = 0;
+    q.edge = false;
+    if constexpr (KC) {
+        q.r = q.from = t >> 3;
+        q.k = (t & 7) * 4;
+        q.p = src + static_cast<int64_t>(r0) * ld;
+    } else {
+        constexpr int kKb = 32 / (ROWS / 32);  // k groups of a step
+        q.r = ((t & 7) + 8 * ((t >> 3) / kKb)) * 4;
+        q.k = ((t >> 3) % kKb) * (ROWS / 32);
+        q.p = src + r0;
+        // rows_total >= 4: the quad stays inside the matrix (perhaps in the
+        // tile before this one)
+        q.from = q.r <= q.rows - 4 ? q.r : q.rows - 4;
+        q.shift = q.r - q.from < 4 ? q.r - q.from : 0;
+        q.edge = (q.rows & 3) != 0;
     }
+    return q;
+}
+
+// Loads the whole step at k0 (k0 + 32 <= K).
+template <bool KC, int ROWS>
+__device__ __forceinline__ void load_step(Step<ROWS>& s, const Place<KC, ROWS>& q, int k0) {
 #pragma unroll
-    for (int i = 0; i < TILE * BK / kThreads; ++i) {
-        const int row = KC ? t / BK + (kThreads / BK) * i : t % TILE;
-        const int k = KC ? t % BK : t / TILE + (kThreads / TILE) * i;
-        const int gr = r0 + row, gk = k0 + k;
-        v[i] = (gr < rows && gk < K)
-                   ? (KC ? p[static_cast<int64_t>(gr) * ld + gk] : p[static_cast<int64_t>(gk) * ld + gr])
-                   : 0.0f;
+    for (int i = 0; i < ROWS / 32; ++i) {
+        if constexpr (KC) {
+            const int row = q.r + 32 * i < q.rows ? q.r + 32 * i : q.rows - 1;
+            s.v[i] = *reinterpret_cast<const f32x4_a4*>(q.p + static_cast<int64_t>(row) * q.ld + k0 +
+                                                        q.k);
+        } else {
+            s.v[i] = *reinterpret_cast<const f32x4_a4*>(
+                q.p + static_cast<int64_t>(k0 + q.k + i) * q.ld + q.from);
+        }
     }
 }
 
-template <int TILE, bool KC, bool VEC>
-__device__ __forceinline__ void store_step(const float (&v)[TILE * BK / kThreads], float* lds) {
-    const int t = threadIdx.x;
-    if constexpr (KC && VEC) {
+// The last K % 32 k, at k0: element by element, zeros past K.
+template <bool KC, int ROWS>
+__device__ __forceinline__ void load_tail(Step<ROWS>& s, const Place<KC, ROWS>& q, int k0, int K) {
 #pragma unroll
-        for (int i = 0; i < TILE * BK / kThreads / 4; ++i)
+    for (int i = 0; i < ROWS / 32; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                lds[((t % 4) * 4 + e) * kStride + t / 4 + (kThreads / 4) * i] = v[4 * i + e];
-        return;
+        for (int e = 0; e < 4; ++e) {
+            const int k = k0 + q.k + (KC ? e : i);
+            int row = KC ? q.r + 32 * i : q.from + e;
+            row = row < q.rows ? row : q.rows - 1;
+            s.v[i][e] = k >= K ? 0.0f
+                               : KC ? q.p[static_cast<int64_t>(row) * q.ld + k]
+                                    : q.p[static_cast<int64_t>(k) * q.ld + row];
+        }
+}
+
+template <bool KC, int ROWS>
+__device__ __forceinline__ void store_step(const Step<ROWS>& s, const Place<KC, ROWS>& q,
+                                           float* lds) {
+    if constexpr (KC) {
+#pragma unroll
+        for (int i = 0; i < ROWS / 32; ++i)
+            *reinterpret_cast<f32x4*>(lds + chunk_off(q.r + 32 * i, q.k >> 2)) = s.v[i];
+    } else {
+        Step<ROWS> w = s;
+        if (q.edge) {  // a quad moved down by `shift` rows holds row r + e at e + shift
+#pragma unroll
+            for (int i = 0; i < ROWS / 32; ++i)
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    float x = s.v[i][e];
+                    x = q.shift == 1 ? s.v[i][e + 1] : x;
+                    x = q.shift == 2 ? s.v[i][e + 2 < 4 ? e + 2 : 3] : x;
+                    x = q.shift == 3 ? s.v[i][3] : x;
+                    w.v[i][e] = x;
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float* at = lds + chunk_off(q.r + e, q.k >> 2) + (q.k & 3);
+            if constexpr (ROWS == 64)
+                *reinterpret_cast<f32x2*>(at) = f32x2{w.v[0][e], w.v[1][e]};
+            else
+                *reinterpret_cast<f32x4*>(at) =
+                    f32x4{w.v[0][e], w.v[1][e], w.v[2][e], w.v[3][e]};
+        }
     }
+}
+
+template <int NT>
+struct Quads {
+    f32x4 v[NT];
+};
+
+// The quads of substep s for NT blocks of 32 rows from row0.
+template <int NT>
+__device__ __forceinline__ void read_quads(Quads<NT>& f, const float* lds, int row0, int s,
+                                           int lane) {
 #pragma unroll
-    for (int i = 0; i < TILE * BK / kThreads; ++i) {
-        const int row = KC ? t / BK + (kThreads / BK) * i : t % TILE;
-        const int k = KC ? t % BK : t / TILE + (kThreads / TILE) * i;
-        lds[k * kStride + row] = v[i];
-    }
+    for (int i = 0; i < NT; ++i)
+        f.v[i] = *reinterpret_cast<const f32x4*>(
+            lds + chunk_off(row0 + i * 32 + (lane & 31), 2 * s + (lane >> 5)));
+}
+
+template <int TM, int TN>
+__device__ __forceinline__ void mfma_quads(const Quads<TM>& a, const Quads<TN>& b,
+                                           f32x16 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.v[i][e], b.v[j][e], acc[i][j],
+                                                                 0, 0, 0);
 }
 
 // A_KC: A is [M][lda] (k contiguous), else A^T [K][lda]; B_KC: B is given as
 // B^T [N][ldb] (k contiguous), else B [K][ldb].
-template <int TILE, bool A_KC, bool B_KC, bool VEC>
-__global__ __launch_bounds__(kThreads) void gemm_f32_kernel(
+template <int BM, int BN, bool A_KC, bool B_KC>
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
-    float* __restrict__ C, int64_t ldc, int M, int N, int K, int accumulate, int tiles_n) {
-    __shared__ float lds[2][2 * kStage];  // [stage][A k-rows, then B k-rows]
+    float* __restrict__ C, int64_t ldc, int M, int N, int K, int accumulate, int tiles_m,
+    int tiles_n) {
+    constexpr int kStage = (BM + BN) * BK;
+    __shared__ __attribute__((aligned(16))) float l0[kStage];
+    __shared__ __attribute__((aligned(16))) float l1[kStage];
 
-    constexpr int NT = TILE / 64;  // 32 x 32 MFMA blocks per wave along each dimension
-    constexpr int WT = TILE / 2;   // the wave's block of C is WT x WT
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    constexpr int TM = BM / 64, TN = BN / 64;  // 32 x 32 MFMA blocks per wave
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = (static_cast<int>(blockIdx.x) / tiles_n) * TILE;
-    const int n0 = (static_cast<int>(blockIdx.x) % tiles_n) * TILE;
+    int tm, tn;
+    agk_gemm::tile_of(blockIdx.x, tiles_m, tiles_n, agk_gemm::kGroupM, tm, tn);
+    const int m0 = tm * BM;
+    const int n0 = tn * BN;
 
-    f32x16 acc[NT][NT];
+    f32x16 acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    float va[TILE * BK / kThreads], vb[TILE * BK / kThreads];
-    const int nk = (K + BK - 1) / BK;
-    load_step<TILE, A_KC, VEC>(va, A, lda, m0, M, 0, K);
-    load_step<TILE, B_KC, VEC>(vb, B, ldb, n0, N, 0, K);
-    store_step<TILE, A_KC, VEC>(va, lds[0]);
-    store_step<TILE, B_KC, VEC>(vb, lds[0] + kStage);
-    __syncthreads();
-
-    const int fr = lane & 31;  // operand row / column within a 32-block
-    const int fk = lane >> 5;  // operand k within a 2-deep MFMA step
-    for (int kt = 0; kt < nk; ++kt) {
-        const float* as = lds[kt & 1];
-        const float* bs = as + kStage;
-        const bool more = kt + 1 < nk;
-        if (more) {
-            load_step<TILE, A_KC, VEC>(va, A, lda, m0, M, (kt + 1) * BK, K);
-            load_step<TILE, B_KC, VEC>(vb, B, ldb, n0, N, (kt + 1) * BK, K);
-        }
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 2) {
-            float a[NT], b[NT];
-#pragma unroll
-            for (int i = 0; i < NT; ++i) a[i] = as[(kk + fk) * kStride + wm * WT + i * 32 + fr];
-#pragma unroll
-            for (int j = 0; j < NT; ++j) b[j] = bs[(kk + fk) * kStride + wn * WT + j * 32 + fr];
-#pragma unroll
-            for (int i = 0; i < NT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            float* nxt = lds[(kt + 1) & 1];
-            store_step<TILE, A_KC, VEC>(va, nxt);
-            store_step<TILE, B_KC, VEC>(vb, nxt + kStage);
-        }
+    const Place<A_KC, BM> pa = place<A_KC, BM>(A, lda, m0, M, tid);
+    const Place<B_KC, BN> pb = place<B_KC, BN>(B, ldb, n0, N, tid);
+    const int nk = K / BK;  // whole steps
+    Quads<TM> fa[2];
+    Quads<TN> fb[2];
+    auto read = [&](int f, const float* stage, int s) {
+        read_quads(fa[f], stage, wm * (BM / 2), s, lane);
+        read_quads(fb[f], stage + BM * BK, wn * (BN / 2), s, lane);
+    };
+    if (K % BK) {  // the ragged end of K first
+        Step<BM> ta;
+        Step<BN> tb;
+        load_tail(ta, pa, nk * BK, K);
+        load_tail(tb, pb, nk * BK, K);
+        store_step(ta, pa, l1);
+        store_step(tb, pb, l1 + BM * BK);
         __syncthreads();
+        for (int s = 0; s * 8 < K % BK; ++s) {
+            read(0, l1, s);
+            mfma_quads(fa[0], fb[0], acc);
+        }
+    }
+    if (nk > 0) {
+        Step<BM> a0, a1;
+        Step<BN> b0, b1;
+        // step u, or the last one again: the loop below loads and stores
+        // without conditions, so that the compiler can count the loads in
+        // flight (behind a condition it waited for all of them each step)
+        auto load = [&](Step<BM>& a, Step<BN>& b, int u) {
+            const int k0 = (u < nk ? u : nk - 1) * BK;
+            load_step(a, pa, k0);
+            load_step(b, pb, k0);
+        };
+        auto store = [&](const Step<BM>& a, const Step<BN>& b, float* stage) {
+            store_step(a, pa, stage);
+            store_step(b, pb, stage + BM * BK);
+        };
+        load(a0, b0, 0);
+        load(a1, b1, 1);
+        store(a0, b0, l0);
+        __syncthreads();
+        // Step t out of `cur`.  (na, nb) are free and take step t + 2; (wa, wb)
+        // hold step t + 1, for `nxt`.  The fragments run one substep ahead of
+        // the MFMAs, across the barrier.
+#define AGK_F32_STEP(FIRST, t, cur, nxt, na, nb, wa, wb) \
+    load(na, nb, (t) + 2);                               \
+    read(0, cur, 0);                                     \
+    if (!FIRST) mfma_quads(fa[1], fb[1], acc);           \
+    read(1, cur, 1);                                     \
+    mfma_quads(fa[0], fb[0], acc);                       \
+    read(0, cur, 2);                                     \
+    mfma_quads(fa[1], fb[1], acc);                       \
+    read(1, cur, 3);                                     \
+    store(wa, wb, nxt);                                  \
+    mfma_quads(fa[0], fb[0], acc);                       \
+    __syncthreads();
+        AGK_F32_STEP(true, 0, l0, l1, a0, b0, a1, b1)
+        int t = 1;
+        for (; t + 1 < nk; t += 2) {
+            AGK_F32_STEP(false, t, l1, l0, a1, b1, a0, b0)
+            AGK_F32_STEP(false, t + 1, l0, l1, a0, b0, a1, b1)
+        }
+        if (t < nk) {
+            AGK_F32_STEP(false, t, l1, l0, a1, b1, a0, b0)
+        }
+#undef AGK_F32_STEP
+        mfma_quads(fa[1], fb[1], acc);  // the last step's substep 3
     }
 
     const int col_l = lane & 31;
     const int row_l = 4 * (lane >> 5);
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const int row = m0 + wm * WT + i * 32 + 8 * (e >> 2) + row_l + (e & 3);
+            const int row = m0 + wm * (BM / 2) + i * 32 + 8 * (e >> 2) + row_l + (e & 3);
             if (row >= M) continue;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const int col = n0 + wn * WT + j * 32 + col_l;
+            for (int j = 0; j < TN; ++j) {
+                const int col = n0 + wn * (BN / 2) + j * 32 + col_l;
                 if (col >= N) continue;
                 float* p = C + static_cast<int64_t>(row) * ldc + col;
                 const float v = acc[i][j][e];
                 *p = accumulate ? agk::acc_add(*p, v) : v;
             }
+        }
+    }
+}
+
+// ---- split kernel --------------------------------------------------------------------
+constexpr int kSplitWaves = 4;
+
+// An operand's values for a 32-deep step, in MFMA order: v[s][e] is k
+// 8 s + 4 (lane / 32) + e of the lane's row.
+struct DirectStep {
+    f32x4 v[4];
+};
+
+// p: the lane's row at k = 4 (lane / 32) of the step's first k.
+template <bool KC>
+__device__ __forceinline__ void direct_step(DirectStep& d, const float* __restrict__ p,
+                                            int64_t ld) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if constexpr (KC) {
+            d.v[s] = *reinterpret_cast<const f32x4_a4*>(p + 8 * s);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d.v[s][e] = p[(8 * s + e) * ld];
+        }
+    }
+}
+
+// The ragged last step: `left` k remain from the lane's first; zeros past them.
+template <bool KC>
+__device__ __forceinline__ void direct_tail(DirectStep& d, const float* __restrict__ p, int64_t ld,
+                                            int left) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            d.v[s][e] = 8 * s + e >= left ? 0.0f : KC ? p[8 * s + e] : p[(8 * s + e) * ld];
+}
+
+__device__ __forceinline__ void direct_mfma(const DirectStep& a, const DirectStep& b,
+                                            f32x16& acc) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.v[s][e], b.v[s][e], acc, 0, 0, 0);
+}
+
+template <bool A_KC, bool B_KC>
+__global__ __launch_bounds__(kSplitWaves * 64, 2) void gemm_f32_split_kernel(
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
+    float* __restrict__ C, int64_t ldc, int M, int N, int K, int accumulate, int tiles_n) {
+    __shared__ float part[kSplitWaves][16][64];  // [wave][accumulator element][lane]
+
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int half = lane >> 5;
+    const int m0 = (static_cast<int>(blockIdx.x) / tiles_n) * 32;
+    const int n0 = (static_cast<int>(blockIdx.x) % tiles_n) * 32;
+    const int64_t ra = m0 + (lane & 31) < M ? m0 + (lane & 31) : M - 1;
+    const int64_t rb = n0 + (lane & 31) < N ? n0 + (lane & 31) : N - 1;
+    // the lane's row at k = 32 wave + 4 half, and what 32 kSplitWaves k further on are
+    const int64_t k1 = 32 * wave + 4 * half;
+    const float* pa = A_KC ? A + ra * lda + k1 : A + k1 * lda + ra;
+    const float* pb = B_KC ? B + rb * ldb + k1 : B + k1 * ldb + rb;
+    const int64_t da = 32 * kSplitWaves * (A_KC ? 1 : lda), db = 32 * kSplitWaves * (B_KC ? 1 : ldb);
+
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    // this wave's steps: wave, wave + kSplitWaves, ...; the next one's loads are in
+    // flight while one is multiplied
+    const int whole = K / BK;
+    DirectStep a0, b0, a1, b1;
+    int t = wave;
+    if (t < whole) {
+        direct_step<A_KC>(a0, pa, lda);
+        direct_step<B_KC>(b0, pb, ldb);
+    }
+    for (; t + kSplitWaves < whole; t += 2 * kSplitWaves) {
+        pa += da;
+        pb += db;
+        direct_step<A_KC>(a1, pa, lda);
+        direct_step<B_KC>(b1, pb, ldb);
+        direct_mfma(a0, b0, acc);
+        pa += da;
+        pb += db;
+        if (t + 2 * kSplitWaves < whole) {
+            direct_step<A_KC>(a0, pa, lda);
+            direct_step<B_KC>(b0, pb, ldb);
+        }
+        direct_mfma(a1, b1, acc);
+    }
+    if (t < whole) {
+        direct_mfma(a0, b0, acc);
+        t += kSplitWaves;
+        pa += da;
+        pb += db;
+    }
+    if (t * BK < K) {  // the ragged step falls to the wave whose turn it is
+        const int left = K - t * BK - 4 * half;
+        direct_tail<A_KC>(a0, pa, lda, left);
+        direct_tail<B_KC>(b0, pb, ldb, left);
+        direct_mfma(a0, b0, acc);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) part[wave][e][lane] = acc[e];
+    __syncthreads();
+    // wave w adds and stores elements 16 w / kSplitWaves ..
+#pragma unroll
+    for (int i = 0; i < 16 / kSplitWaves; ++i) {
+        const int e = wave * (16 / kSplitWaves) + i;
+        float v = part[0][e][lane];
+#pragma unroll
+        for (int w = 1; w < kSplitWaves; ++w) v += part[w][e][lane];
+        const int row = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
+        const int col = n0 + (lane & 31);
+        if (row < M && col < N) {
+            float* p = C + static_cast<int64_t>(row) * ldc + col;
+            *p = accumulate ? agk::acc_add(*p, v) : v;
         }
     }
 }
@@ -206,6 +455,30 @@ __global__ __launch_bounds__(256) void zero_rows_kernel(float* __restrict__ C, i
                                                         int N) {
     float* r = C + static_cast<int64_t>(blockIdx.x) * ldc;
     for (int c = threadIdx.x; c < N; c += 256) r[c] = 0.0f;
+}
+
+// 2: 128 x 128 tiles, 1: 64 x 64 tiles, 0: 32 x 32 tiles with K split over the
+// waves.  The cheapest by the microseconds a CU spends per 32-deep step: its
+// share of the tiles times a tile's time, measured on MI355X.  A tile's MFMAs
+// take 1.7 / 0.43 / 0.11 us; what it costs beyond them is staging and, alone
+// on its CU, waiting:
+//               alone   with others   measured (us; K-contiguous operands)
+//   128 x 128    2.1       1.95       4096^3: 1000 (64 x 64: 1022, split: 1803)
+//   64 x 64      0.6       0.53       1024^3: 24 (128 x 128: 71, split: 34)
+//   split        0.25      0.25       300 x 500 x 4095: 33 (64 x 64: 77)
+// The kernel this replaced: 1024^3 42 us, 300 x 500 x 4095 143 us,
+// 4096^3 1138-1333 us (by layout; now 1000-1049).
+inline int pick_f32(int64_t M, int64_t N) {
+    constexpr int64_t kCus = 256;
+    auto per_cu = [&](int64_t t) {
+        return static_cast<double>((((M + t - 1) / t) * ((N + t - 1) / t) + kCus - 1) / kCus);
+    };
+    const double c32 = per_cu(32), c64 = per_cu(64), c128 = per_cu(128);
+    const double split = 0.25 * c32;
+    const double small = c64 > 1 ? 0.53 * c64 : 0.6;
+    const double large = c128 > 1 ? 1.95 * c128 : 2.1;
+    if (split < small && split < large) return 0;
+    return small < large ? 1 : 2;
 }
 
 }  // namespace agk_sgemm
@@ -231,45 +504,36 @@ extern "C" int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const floa
                            ldc, n);
         return agk::check_launch();
     }
-    // 128 x 128 tiles, or 64 x 64 when the 128-tiles would not fill the CUs
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        cus = 256;
-    const bool small = ((M + 127) / 128) * ((N + 127) / 128) < cus;
-    const int tile = small ? 64 : 128;
-    const int64_t tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
-    if (tiles_m * tiles_n > kMax) return AGK_EINVAL;
-    const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n)), block(kThreads);
-    const int acc = accumulate != 0;
-    const int tn = static_cast<int>(tiles_n);
     // A k-contiguous unless given transposed; B k-contiguous only when given as B^T
     const bool a_kc = a_trans == 0, b_kc = b_trans != 0;
-    // 16-byte loads of the k-contiguous operands when their rows allow it
-    auto vec_ok = [](const float* p, int64_t ld) {
-        return (reinterpret_cast<uintptr_t>(p) & 15u) == 0 && ld % 4 == 0;
-    };
-    const bool vec = (!a_kc || vec_ok(A, lda)) && (!b_kc || vec_ok(B, ldb));
-#define AGK_F32(T, AK, BKC)                                                                   \
-    do {                                                                                      \
-        if (vec)                                                                              \
-            hipLaunchKernelGGL((gemm_f32_kernel<T, AK, BKC, true>), grid, block, 0, st, A, lda, \
-                               B, ldb, C, ldc, m, n, k, acc, tn);                             \
-        else                                                                                  \
-            hipLaunchKernelGGL((gemm_f32_kernel<T, AK, BKC, false>), grid, block, 0, st, A,     \
-                               lda, B, ldb, C, ldc, m, n, k, acc, tn);                        \
-    } while (0)
-#define AGK_F32_LAYOUTS(T)                  \
-    if (a_kc && b_kc) AGK_F32(T, true, true);   \
-    else if (a_kc) AGK_F32(T, true, false);     \
-    else if (b_kc) AGK_F32(T, false, true);     \
-    else AGK_F32(T, false, false);
-    if (small) {
-        AGK_F32_LAYOUTS(64)
-    } else {
-        AGK_F32_LAYOUTS(128)
+    int shape = pick_f32(M, N);
+    // the tiled kernel loads four rows at a time of an operand whose rows are
+    // contiguous: it needs four of them
+    if ((!a_kc && M < 4) || (!b_kc && N < 4)) shape = 0;
+    const int tile = shape == 2 ? 128 : shape == 1 ? 64 : 32;
+    const int64_t tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
+    if (tiles_m * tiles_n > kMax) return AGK_EINVAL;
+    const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
+    const int acc = accumulate != 0;
+    const int tm = static_cast<int>(tiles_m), tn = static_cast<int>(tiles_n);
+#define AGK_F32(AK, BKC)                                                                      \
+    switch (shape) {                                                                          \
+        case 2:                                                                               \
+            hipLaunchKernelGGL((gemm_f32_kernel<128, 128, AK, BKC>), grid, dim3(256), 0, st,  \
+                               A, lda, B, ldb, C, ldc, m, n, k, acc, tm, tn);                 \
+            break;                                                                            \
+        case 1:                                                                               \
+            hipLaunchKernelGGL((gemm_f32_kernel<64, 64, AK, BKC>), grid, dim3(256), 0, st, A, \
+                               lda, B, ldb, C, ldc, m, n, k, acc, tm, tn);                    \
+            break;                                                                            \
+        default:                                                                              \
+            hipLaunchKernelGGL((gemm_f32_split_kernel<AK, BKC>), grid, dim3(kSplitWaves * 64), \
+                               0, st, A, lda, B, ldb, C, ldc, m, n, k, acc, tn);              \
     }
-#undef AGK_F32_LAYOUTS
+    if (a_kc && b_kc) AGK_F32(true, true)
+    else if (a_kc) AGK_F32(true, false)
+    else if (b_kc) AGK_F32(false, true)
+    else AGK_F32(false, false)
 #undef AGK_F32
     return agk::check_launch();
 }

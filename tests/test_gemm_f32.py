@@ -20,14 +20,41 @@ from gpu_util import to_dev, to_host
 pytestmark = pytest.mark.gpu
 
 OK, EINVAL = 0, 1  # agk_status
-# below the CU count in 128-tiles: the 64 x 64 tile; from (2048, 2048, 40) on
-# (256 and 289 128-tiles): the 128 x 128 tile, the second with edge tiles
+# the split kernel (32 x 32 tiles) for few tiles, 64 x 64 tiles from (1000, 520, 64)'s
+# neighbours up, 128 x 128 tiles at (2048, 2048, 40)
 SHAPES = [(1, 1, 1), (7, 5, 3), (64, 48, 33), (129, 257, 95), (300, 17, 1000), (1000, 520, 64),
           (256, 384, 513), (2048, 1024, 160), (2048, 2048, 40), (2100, 2060, 33)]
 
 
 def _bound(a, b, K):
     return (K + 1) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 1e-30
+
+
+# Split kernel: K of 0-2 steps per wave, a ragged step in each wave's turn, one row or
+# column.  Tiled kernels: one, two, three and more 32-deep steps, with and without a
+# ragged end, odd edge tiles (1 to 3 rows in the last one).
+EDGE_SHAPES = [(33, 31, 31), (65, 34, 129), (40, 50, 161), (31, 33, 290), (3, 200, 257),
+               (200, 2, 63), (1, 1000, 130), (1027, 1021, 32), (1025, 1023, 64), (1026, 1022, 97),
+               (1027, 1021, 170), (2039, 2037, 67), (2041, 2045, 128), (2046, 2047, 31)]
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("M,N,K", EDGE_SHAPES, ids=lambda v: str(v))
+def test_tile_edges_match_fp64(cuda, M, N, K, trans_a, trans_b):
+    """The bar of test_product_matches_fp64, computed on the GPU in float64; operands start one
+    float off a 16-byte boundary."""
+    import torch
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(M * 7 + N * 3 + K)
+    a = torch.randn(M * K + 1, generator=gen, device=cuda)[1:].view((K, M) if trans_a else (M, K))
+    b = torch.randn(K * N + 1, generator=gen, device=cuda)[1:].view((N, K) if trans_b else (K, N))
+    print(f"gemm_f32 {M}x{N}x{K} ta={trans_a} tb={trans_b}", flush=True)
+    c = agk.gemm_f32(a, b, trans_a=trans_a, trans_b=trans_b)
+    A, B = (a.t() if trans_a else a).double(), (b.t() if trans_b else b).double()
+    bound = (K + 1) * 2.0 ** -24 * (A.abs() @ B.abs()) + 1e-30
+    torch.cuda.synchronize()
+    assert ((c.double() - A @ B).abs() <= bound).all().item()
 
 
 @pytest.mark.parametrize("trans_b", [False, True])
