@@ -61,7 +61,8 @@ namespace agk {
 // but [51, 13824] fp32 4.19-4.21 -> 4.38-4.39 us (a long row's gamma loads
 // compete with its x loads before the sum) and many rows lose ~3 % (live
 // registers).  Same arithmetic either way.
-template <class S, int TPR, int NV, int G, bool MUL = false, bool EARLY_G = false>
+template <class S, int TPR, int NV, int G, bool MUL = false, bool EARLY_G = false,
+          bool RAG = false>
 __global__ __launch_bounds__(TPR * G) void rms_fwd_resident(
     const typename S::T* __restrict__ x, const typename S::T* __restrict__ gamma,
     typename S::T* __restrict__ y, float* __restrict__ inv_rms, int64_t rows, int cols,
@@ -81,21 +82,27 @@ __global__ __launch_bounds__(TPR * G) void rms_fwd_resident(
     for (int e = 0; e < W; ++e) part[e] = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int col = (t + k * TPR) * W;
-        xv[k] = (active && col < cols) ? load16_stream<S>(xr + col) : u32x4{0u, 0u, 0u, 0u};
+        const int col = slot_col<RAG, W>(t + k * TPR, cols);
+        xv[k] = (active && col < cols)
+                    ? (RAG ? load16_any_stream<S>(xr + col) : load16_stream<S>(xr + col))
+                    : u32x4{0u, 0u, 0u, 0u};
     }
     [[maybe_unused]] u32x4 gv[EARLY_G ? NV : 1];
     if constexpr (EARLY_G) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int col = (t + k * TPR) * W;
-            gv[k] = (active && col < cols) ? load16<S>(gamma + col) : u32x4{0u, 0u, 0u, 0u};
+            const int col = slot_col<RAG, W>(t + k * TPR, cols);
+            gv[k] = (active && col < cols)
+                        ? (RAG ? load16_any<S>(gamma + col) : load16<S>(gamma + col))
+                        : u32x4{0u, 0u, 0u, 0u};
         }
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         float f[W];
         S::unpack(xv[k], f);
+        if constexpr (RAG)
+            drop_dup(f, (t + k * TPR) * W - slot_col<RAG, W>(t + k * TPR, cols));
 #pragma unroll
         for (int e = 0; e < W; ++e) part[e] += f[e] * f[e];
     }
@@ -117,13 +124,13 @@ __global__ __launch_bounds__(TPR * G) void rms_fwd_resident(
     T* yr = y + row * static_cast<int64_t>(cols);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int col = (t + k * TPR) * W;
+        const int col = slot_col<RAG, W>(t + k * TPR, cols);
         if (col < cols) {
             float f[W];
             S::unpack(xv[k], f);
             if (MUL) {
                 float gm[W];
-                S::unpack(load16<S>(gamma + col), gm);
+                S::unpack(RAG ? load16_any<S>(gamma + col) : load16<S>(gamma + col), gm);
 #pragma unroll
                 for (int e = 0; e < W; ++e) f[e] = f[e] * gm[e];
             } else if (EARLY_G) {
@@ -133,14 +140,15 @@ __global__ __launch_bounds__(TPR * G) void rms_fwd_resident(
                 for (int e = 0; e < W; ++e) f[e] = (f[e] * r) * gm[e];
             } else if (gamma) {
                 float gm[W];
-                S::unpack(load16<S>(gamma + col), gm);
+                S::unpack(RAG ? load16_any<S>(gamma + col) : load16<S>(gamma + col), gm);
 #pragma unroll
                 for (int e = 0; e < W; ++e) f[e] = (f[e] * r) * gm[e];
             } else {
 #pragma unroll
                 for (int e = 0; e < W; ++e) f[e] = f[e] * r;
             }
-            store16_stream<S>(yr + col, S::pack(f));
+            if constexpr (RAG) store16_any_stream<S>(yr + col, S::pack(f));
+            else store16_stream<S>(yr + col, S::pack(f));
         }
     }
 }
@@ -193,7 +201,7 @@ struct BwdSet {
 //               layer): partials += dy, no row reduction, nothing stored.
 enum : int { kBwdRms = 0, kBwdMul = 1, kBwdRmsMul = 2, kBwdColSum = 3 };
 
-template <class S, int TPR, int NV, int G, bool ACC, int KIND>
+template <class S, int TPR, int NV, int G, bool ACC, int KIND, bool RAG = false>
 struct BwdCtx {
     using T = typename S::T;
     static constexpr int W = S::kVec;
@@ -209,6 +217,7 @@ struct BwdCtx {
     uint32_t row_bytes, x_bytes, old_bytes, dx_bytes, dr_bytes, roff;
     uint32_t off[NV];
     float inv_cols;
+    int klast, dup;  // RAG: the index of the row's last slot, and what it overlaps in this lane
 
     // First row of the wave's rows at `step` (clamped into range) and how many exist.
     __device__ __forceinline__ void wave_rows(int64_t step, int64_t& r0, uint32_t& n) const {
@@ -257,8 +266,8 @@ __device__ __forceinline__ void stored_product(float (&f)[S::kVec], const float 
     for (int e = 0; e < W; ++e) asm("" : "+v"(f[e]));
 }
 
-template <class S, int TPR, int NV, int G, bool ACC, int KIND>
-__device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIND>& c,
+template <class S, int TPR, int NV, int G, bool ACC, int KIND, bool RAG = false>
+__device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIND, RAG>& c,
                                             BwdSet<S, NV, ACC>& b,
                                             int64_t step, int parity, const u32x4 (&gv)[NV],
                                             bool has_gamma, float (&dg)[NV][S::kVec],
@@ -303,6 +312,12 @@ __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIN
                 S::unpack(gv[k], gm);
 #pragma unroll
                 for (int e = 0; e < W; ++e) fd[e] = fd[e] * gm[e];
+            }
+            if constexpr (RAG) {
+                if (k == c.klast) {  // uniform; both factors, so that 0 * inf adds nothing
+                    drop_dup(fx, c.dup);
+                    drop_dup(fd, c.dup);
+                }
             }
 #pragma unroll
             for (int e = 0; e < W; ++e) part[e] += fd[e] * fx[e];
@@ -363,7 +378,17 @@ __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIN
 #pragma unroll
             for (int e = 0; e < W; ++e) o[e] = acc_add(old[e], o[e]);
         }
-        bstore16_stream(rdx, c.off[k], S::pack(o));
+        if constexpr (RAG && ACC) {
+            if (k == c.klast && c.dup > 0) {
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+                    if (e >= c.dup) bstore_elem<S>(rdx, c.off[k] + e * sizeof(typename S::T), o[e]);
+            } else {
+                bstore16_stream(rdx, c.off[k], S::pack(o));
+            }
+        } else {
+            bstore16_stream(rdx, c.off[k], S::pack(o));
+        }
         if constexpr (MUL) {
 #pragma unroll
             for (int e = 0; e < W; ++e) dg[k][e] += fd[e] * fx[e];
@@ -383,8 +408,8 @@ __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIN
 
 // Runs steps 0 .. steps-1 of c's row sequence with NSET (1, 2 or 3) register
 // sets, adding each lane's dgamma terms into dg.
-template <class S, int TPR, int NV, int G, int NSET, bool ACC, int KIND>
-__device__ __forceinline__ void bwd_segment(const BwdCtx<S, TPR, NV, G, ACC, KIND>& c, int64_t steps,
+template <class S, int TPR, int NV, int G, int NSET, bool ACC, int KIND, bool RAG = false>
+__device__ __forceinline__ void bwd_segment(const BwdCtx<S, TPR, NV, G, ACC, KIND, RAG>& c, int64_t steps,
                                             const u32x4 (&gv)[NV], bool has_gamma,
                                             float (&dg)[NV][S::kVec],
                                             float (*red)[TPR > 64 ? G * (TPR / 64) : 1]) {
@@ -437,7 +462,7 @@ __device__ __forceinline__ void bwd_segment(const BwdCtx<S, TPR, NV, G, ACC, KIN
 // Writes one partial row of dgamma: the G groups' sums (each group's in its
 // own LDS row) added in group order, column by column.  Ends with a barrier
 // so the LDS rows can be written again.
-template <class S, int TPR, int NV, int G>
+template <class S, int TPR, int NV, int G, bool RAG = false>
 __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int cols, int t,
                                                   int grp, const float (&dg)[NV][S::kVec],
                                                   float* lds_part) {
@@ -445,7 +470,7 @@ __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int 
     if constexpr (G == 1) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int col = (t + k * TPR) * W;
+            const int col = slot_col<RAG, W>(t + k * TPR, cols);
             if (col < cols) {
 #pragma unroll
                 for (int e = 0; e < W; ++e) prow[col + e] = dg[k][e];
@@ -454,7 +479,7 @@ __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int 
     } else {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int col = (t + k * TPR) * W;
+            const int col = slot_col<RAG, W>(t + k * TPR, cols);
             if (col < cols) {
 #pragma unroll
                 for (int e = 0; e < W; ++e) lds_part[grp * cols + col + e] = dg[k][e];
@@ -473,8 +498,8 @@ __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int 
 // The skeleton's per-lane context for workgroup blk of a grid of nblk row
 // workgroups (group q of workgroup blk takes rows blk*G + q + k*nblk*G), and
 // the lane's slots of gamma.
-template <class S, int TPR, int NV, int G, bool ACC, int KIND>
-__device__ __forceinline__ void bwd_setup(BwdCtx<S, TPR, NV, G, ACC, KIND>& c, u32x4 (&gv)[NV],
+template <class S, int TPR, int NV, int G, bool ACC, int KIND, bool RAG = false>
+__device__ __forceinline__ void bwd_setup(BwdCtx<S, TPR, NV, G, ACC, KIND, RAG>& c, u32x4 (&gv)[NV],
                                           const typename S::T* x, const typename S::T* gamma,
                                           const float* inv_rms, const typename S::T* dy,
                                           typename S::T* dx, typename S::T* dr, int64_t rows,
@@ -504,23 +529,28 @@ __device__ __forceinline__ void bwd_setup(BwdCtx<S, TPR, NV, G, ACC, KIND>& c, u
     c.dr_bytes = dr ? c.row_bytes : 0u;
     c.roff = static_cast<uint32_t>(sub) * 4u;
     c.inv_cols = 1.0f / static_cast<float>(cols);
+    if constexpr (RAG) {
+        const int last = (cols + W - 1) / W - 1;  // the row's last slot
+        c.klast = last / TPR;
+        c.dup = t == last % TPR ? (last + 1) * W - cols : 0;
+    }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int col = (t + k * TPR) * W;
+        const int col = slot_col<RAG, W>(t + k * TPR, cols);
         c.off[k] = col < cols ? (static_cast<uint32_t>(sub) * static_cast<uint32_t>(cols) +
                                  static_cast<uint32_t>(col)) * static_cast<uint32_t>(sizeof(T))
                               : kOffOut;
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int col = (t + k * TPR) * W;
-        gv[k] = (gamma != nullptr && col < cols) ? load16<S>(gamma + col) : u32x4{0u, 0u, 0u, 0u};
+        const int col = slot_col<RAG, W>(t + k * TPR, cols);
+        gv[k] = (gamma != nullptr && col < cols) ? (RAG ? load16_any<S>(gamma + col) : load16<S>(gamma + col)) : u32x4{0u, 0u, 0u, 0u};
     }
 }
 
 // Rows are dealt round-robin to the gridDim.x workgroups; workgroup b writes
 // partial row b.
-template <class S, int TPR, int NV, int G, int NSET, bool ACC, int KIND>
+template <class S, int TPR, int NV, int G, int NSET, bool ACC, int KIND, bool RAG = false>
 __device__ __forceinline__ void bwd_resident_body(
     const typename S::T* __restrict__ x, const typename S::T* __restrict__ gamma,
     const float* __restrict__ inv_rms, const typename S::T* __restrict__ dy,
@@ -530,7 +560,7 @@ __device__ __forceinline__ void bwd_resident_body(
     const int t = threadIdx.x % TPR;
     const int grp = threadIdx.x / TPR;
 
-    BwdCtx<S, TPR, NV, G, ACC, KIND> c;
+    BwdCtx<S, TPR, NV, G, ACC, KIND, RAG> c;
     u32x4 gv[NV];
     bwd_setup(c, gv, x, gamma, inv_rms, dy, dx, dr, rows, cols, blockIdx.x, gridDim.x);
     const bool has_gamma = gamma != nullptr;
@@ -541,27 +571,27 @@ __device__ __forceinline__ void bwd_resident_body(
         for (int e = 0; e < W; ++e) dg[k][e] = 0.0f;
 
     const int64_t steps = c.first < rows ? (rows - c.first + c.stride - 1) / c.stride : 0;
-    bwd_segment<S, TPR, NV, G, NSET, ACC, KIND>(c, steps, gv, has_gamma, dg, red);
+    bwd_segment<S, TPR, NV, G, NSET, ACC, KIND, RAG>(c, steps, gv, has_gamma, dg, red);
     if (partials)
-        bwd_write_partial<S, TPR, NV, G>(partials + static_cast<int64_t>(blockIdx.x) * cols, cols,
+        bwd_write_partial<S, TPR, NV, G, RAG>(partials + static_cast<int64_t>(blockIdx.x) * cols, cols,
                                          t, grp, dg, lds_part);
 }
 
 // RMSNorm backward: dx (+)= r*(dy*gamma - x*r*r*dot/cols), dgamma partials.
-template <class S, int TPR, int NV, int G, int NSET, bool ACC>
+template <class S, int TPR, int NV, int G, int NSET, bool ACC, bool RAG = false>
 __global__ __launch_bounds__(TPR * G) void rms_bwd_resident(
     const typename S::T* __restrict__ x, const typename S::T* __restrict__ gamma,
     const float* __restrict__ inv_rms, const typename S::T* __restrict__ dy,
     typename S::T* __restrict__ dx, float* __restrict__ partials, int64_t rows, int cols) {
     __shared__ float red[2][TPR > 64 ? G * (TPR / 64) : 1];
     extern __shared__ float lds_part[];  // [G][cols] when G > 1 and partials
-    bwd_resident_body<S, TPR, NV, G, NSET, ACC, kBwdRms>(x, gamma, inv_rms, dy, dx, nullptr,
+    bwd_resident_body<S, TPR, NV, G, NSET, ACC, kBwdRms, RAG>(x, gamma, inv_rms, dy, dx, nullptr,
                                                          partials, rows, cols, red, lds_part);
 }
 
 // The composition y = rms(x) * gamma (kBwdRmsMul): dr = gy*gamma, dx (+)=
 // the RMSNorm VJP of dr, dgamma partials of gy*rms(x).  gamma is required.
-template <class S, int TPR, int NV, int G, int NSET, bool ACC>
+template <class S, int TPR, int NV, int G, int NSET, bool ACC, bool RAG = false>
 __global__ __launch_bounds__(TPR * G) void rms_mul_bwd_resident(
     const typename S::T* __restrict__ x, const typename S::T* __restrict__ gamma,
     const float* __restrict__ inv_rms, const typename S::T* __restrict__ gy,
@@ -569,31 +599,31 @@ __global__ __launch_bounds__(TPR * G) void rms_mul_bwd_resident(
     int64_t rows, int cols) {
     __shared__ float red[2][TPR > 64 ? G * (TPR / 64) : 1];
     extern __shared__ float lds_part[];  // [G][cols] when G > 1 and partials
-    bwd_resident_body<S, TPR, NV, G, NSET, ACC, kBwdRmsMul>(x, gamma, inv_rms, gy, dx, dr,
+    bwd_resident_body<S, TPR, NV, G, NSET, ACC, kBwdRmsMul, RAG>(x, gamma, inv_rms, gy, dx, dr,
                                                             partials, rows, cols, red, lds_part);
 }
 
 // Broadcast multiply backward (vjp_Mul with reduce_for_broadcast): da (+)=
 // gy*b, db partials of gy*a.  a, b, da may be null when not needed.
-template <class S, int TPR, int NV, int G, int NSET, bool ACC>
+template <class S, int TPR, int NV, int G, int NSET, bool ACC, bool RAG = false>
 __global__ __launch_bounds__(TPR * G) void mul_rowbcast_bwd_resident(
     const typename S::T* __restrict__ a, const typename S::T* __restrict__ b,
     const typename S::T* __restrict__ gy, typename S::T* __restrict__ da,
     float* __restrict__ partials, int64_t rows, int cols) {
     __shared__ float red[2][TPR > 64 ? G * (TPR / 64) : 1];
     extern __shared__ float lds_part[];  // [G][cols] when G > 1 and partials
-    bwd_resident_body<S, TPR, NV, G, NSET, ACC, kBwdMul>(a, b, nullptr, gy, da, nullptr, partials,
+    bwd_resident_body<S, TPR, NV, G, NSET, ACC, kBwdMul, RAG>(a, b, nullptr, gy, da, nullptr, partials,
                                                          rows, cols, red, lds_part);
 }
 
 // Column sums (kBwdColSum): partial rows of sum_rows x, as the backward's dgamma.
-template <class S, int TPR, int NV, int G, int NSET>
+template <class S, int TPR, int NV, int G, int NSET, bool RAG = false>
 __global__ __launch_bounds__(TPR * G) void sum_rows_resident(const typename S::T* __restrict__ x,
                                                              float* __restrict__ partials,
                                                              int64_t rows, int cols) {
     __shared__ float red[2][TPR > 64 ? G * (TPR / 64) : 1];
     extern __shared__ float lds_part[];  // [G][cols] when G > 1
-    bwd_resident_body<S, TPR, NV, G, NSET, false, kBwdColSum>(nullptr, nullptr, nullptr, x,
+    bwd_resident_body<S, TPR, NV, G, NSET, false, kBwdColSum, RAG>(nullptr, nullptr, nullptr, x,
                                                               nullptr, nullptr, partials, rows,
                                                               cols, red, lds_part);
 }
@@ -724,6 +754,8 @@ __global__ __launch_bounds__(TPR * G) void bwd_fewrows(
 }
 
 // ---- looped kernels (any alignment, any width) --------------------------------
+// For rows shorter than one 16-byte slot or too wide for the resident shapes, and
+// for outputs that overlap an input.
 // One workgroup per row (forward) or per row block (backward); element-wise
 // accesses; the row is read twice (second read normally hits L2).  In the
 // backward, lane c % kBlock exclusively owns column c of this block's partial
@@ -1095,6 +1127,14 @@ inline Plan bwd_plan(int64_t nslot) {
     return p;
 }
 
+// p (the shape for row_slots(cols, w) slots) in its ragged form; none for rows
+// of less than one slot.
+inline Plan ragged(Plan p, int64_t cols, int w) {
+    if (p.tpr == 0 || cols < w) return Plan{};
+    p.rag = true;
+    return p;
+}
+
 // Row blocking of the resident backward: min(kBwdBlocks, rows) workgroups,
 // about one per CU, so the whole grid runs in one generation and finishes
 // together; workgroup b takes rows b*G + q + k*nblk*G (round-robin, so the
@@ -1146,19 +1186,20 @@ int launch_fwd_plan(const Plan& p, const void* x, const void* gamma, void* y, fl
     // one generation of workgroups over short rows, with gamma: gamma loaded beside x
     const bool early_g = gp != nullptr && grid <= kFwdEarlyGammaGrid &&
                          static_cast<int64_t>(p.tpr) * p.nv <= kFwdEarlyGammaSlots;
-#define AGK_X(a, b, c)                                                                       \
-    if (p.tpr == a && p.nv == b && p.g == c) {                                               \
-        if (early_g)                                                                          \
-            hipLaunchKernelGGL((rms_fwd_resident<S, a, b, c, false, true>),                  \
-                               dim3(static_cast<unsigned>(grid)), dim3(a * c), 0, st, xp, gp, \
-                               yp, inv_rms, rows, cols, eps);                                \
-        else                                                                                  \
-            hipLaunchKernelGGL((rms_fwd_resident<S, a, b, c>), dim3(static_cast<unsigned>(grid)), \
-                               dim3(a * c), 0, st, xp, gp, yp, inv_rms, rows, cols, eps);    \
-        return check_launch();                                                               \
+#define AGK_FWD(EARLY, RAG, a, b, c)                                                          \
+    hipLaunchKernelGGL((rms_fwd_resident<S, a, b, c, false, EARLY, RAG>),                     \
+                       dim3(static_cast<unsigned>(grid)), dim3(a * c), 0, st, xp, gp, yp,     \
+                       inv_rms, rows, cols, eps)
+#define AGK_X(a, b, c)                                       \
+    if (p.tpr == a && p.nv == b && p.g == c) {               \
+        if (p.rag) AGK_FWD(false, true, a, b, c);            \
+        else if (early_g) AGK_FWD(true, false, a, b, c);     \
+        else AGK_FWD(false, false, a, b, c);                 \
+        return check_launch();                               \
     }
     AGK_FWD_SHAPES(AGK_X)
 #undef AGK_X
+#undef AGK_FWD
     return AGK_EINVAL;
 }
 
@@ -1178,6 +1219,9 @@ int launch_fwd(const void* x, const void* gamma, void* y, float* inv_rms, int64_
             return launch_wide_team_fwd<S>(x, gamma, y, inv_rms, ws, rows, cols, eps, st);
         return launch_wide_fwd<S>(x, gamma, y, inv_rms, rows, cols, eps, st);
     }
+    // Rows off the 16-byte grid: the same shape in its ragged form.  In place
+    // (y = x) too: a row's loads end in its sum, which comes before its stores.
+    if (!vec) p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), cols, S::kVec);
     return launch_fwd_plan<S>(p, x, gamma, y, inv_rms, rows, cols, eps, st);
 }
 
@@ -1193,6 +1237,11 @@ int launch_mul_fwd(const void* a, const void* b, void* y, int64_t rows, int cols
     const bool vec = (cols % S::kVec) == 0 && aligned16(a) && aligned16(b) && aligned16(y);
     Plan p;
     if (vec) p = fwd_plan(cols / S::kVec, rows);
+    // Ragged rows, unless y overwrites an operand: a slot's stores may then
+    // come before the loads of the slot that overlaps it.
+    const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(T));
+    if (!vec && disjoint(a, y, bytes) && disjoint(b, y, bytes))
+        p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), cols, S::kVec);
     if (p.tpr == 0) {
         if (rows > 0x7fffffffLL) return AGK_EINVAL;
         const int64_t chunk = mul_chunk(rows, cols, vec ? S::kVec : 1);
@@ -1206,9 +1255,14 @@ int launch_mul_fwd(const void* a, const void* b, void* y, int64_t rows, int cols
     if (grid > 0x7fffffffLL) return AGK_EINVAL;
 #define AGK_X(a_, b_, c_)                                                                 \
     if (p.tpr == a_ && p.nv == b_ && p.g == c_) {                                         \
-        hipLaunchKernelGGL((rms_fwd_resident<S, a_, b_, c_, true>),                       \
-                           dim3(static_cast<unsigned>(grid)), dim3(a_ * c_), 0, st, ap, bp, \
-                           yp, nullptr, rows, cols, 0.0f);                                \
+        if (p.rag)                                                                        \
+            hipLaunchKernelGGL((rms_fwd_resident<S, a_, b_, c_, true, false, true>),      \
+                               dim3(static_cast<unsigned>(grid)), dim3(a_ * c_), 0, st, ap, \
+                               bp, yp, nullptr, rows, cols, 0.0f);                        \
+        else                                                                              \
+            hipLaunchKernelGGL((rms_fwd_resident<S, a_, b_, c_, true>),                   \
+                               dim3(static_cast<unsigned>(grid)), dim3(a_ * c_), 0, st, ap, \
+                               bp, yp, nullptr, rows, cols, 0.0f);                        \
         return check_launch();                                                            \
     }
     AGK_FWD_SHAPES(AGK_X)
@@ -1229,9 +1283,15 @@ int launch_bwd_resident(const Plan& p, int64_t nblk, const void* x, const void* 
 #define AGK_X(a, b, c, d)                                                                  \
     if constexpr (bwd_shape_enabled<S>(a, b)) {                                            \
         if (p.tpr == a && p.nv == b && p.g == c) {                                         \
-            hipLaunchKernelGGL((rms_bwd_resident<S, a, b, c, bwd_sets<S>(b, d), ACC>),     \
-                               dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, xp, \
-                               gp, inv_rms, dyp, dxp, partials, rows, cols);                \
+            if (p.rag)                                                                     \
+                hipLaunchKernelGGL((rms_bwd_resident<S, a, b, c, bwd_sets<S>(b, d), ACC,   \
+                                                     true>),                               \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, \
+                                   xp, gp, inv_rms, dyp, dxp, partials, rows, cols);       \
+            else                                                                           \
+                hipLaunchKernelGGL((rms_bwd_resident<S, a, b, c, bwd_sets<S>(b, d), ACC>), \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, \
+                                   xp, gp, inv_rms, dyp, dxp, partials, rows, cols);       \
             return check_launch();                                                         \
         }                                                                                  \
     }
@@ -1253,10 +1313,17 @@ int launch_mul_bwd_resident(const Plan& p, int64_t nblk, const void* a, const vo
 #define AGK_X(a_, b_, c_, d_)                                                              \
     if constexpr (bwd_shape_enabled<S>(a_, b_)) {                                          \
         if (p.tpr == a_ && p.nv == b_ && p.g == c_) {                                      \
-            hipLaunchKernelGGL((mul_rowbcast_bwd_resident<S, a_, b_, c_,                   \
-                                                          bwd_sets<S>(b_, d_), ACC>),      \
-                               dim3(static_cast<unsigned>(nblk)), dim3(a_ * c_), lds, st,   \
-                               ap, bp, gp, dap, partials, rows, cols);                     \
+            if (p.rag)                                                                     \
+                hipLaunchKernelGGL((mul_rowbcast_bwd_resident<S, a_, b_, c_,               \
+                                                              bwd_sets<S>(b_, d_), ACC,    \
+                                                              true>),                      \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a_ * c_), lds,  \
+                                   st, ap, bp, gp, dap, partials, rows, cols);             \
+            else                                                                           \
+                hipLaunchKernelGGL((mul_rowbcast_bwd_resident<S, a_, b_, c_,               \
+                                                              bwd_sets<S>(b_, d_), ACC>),  \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a_ * c_), lds,  \
+                                   st, ap, bp, gp, dap, partials, rows, cols);             \
             return check_launch();                                                         \
         }                                                                                  \
     }
@@ -1274,9 +1341,15 @@ int launch_sum_rows_resident(const Plan& p, int64_t nblk, const void* x, float* 
 #define AGK_X(a_, b_, c_, d_)                                                              \
     if constexpr (bwd_shape_enabled<S>(a_, b_)) {                                          \
         if (p.tpr == a_ && p.nv == b_ && p.g == c_) {                                      \
-            hipLaunchKernelGGL((sum_rows_resident<S, a_, b_, c_, bwd_sets<S>(b_, d_)>),    \
-                               dim3(static_cast<unsigned>(nblk)), dim3(a_ * c_), lds, st,   \
-                               xp, partials, rows, cols);                                  \
+            if (p.rag)                                                                     \
+                hipLaunchKernelGGL((sum_rows_resident<S, a_, b_, c_, bwd_sets<S>(b_, d_),  \
+                                                      true>),                              \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a_ * c_), lds,  \
+                                   st, xp, partials, rows, cols);                          \
+            else                                                                           \
+                hipLaunchKernelGGL((sum_rows_resident<S, a_, b_, c_, bwd_sets<S>(b_, d_)>), \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a_ * c_), lds,  \
+                                   st, xp, partials, rows, cols);                          \
             return check_launch();                                                         \
         }                                                                                  \
     }
@@ -1306,6 +1379,24 @@ inline Plan bwd_plan_for(const void* x, const void* gamma, const void* dy, const
     return p;
 }
 
+// The ragged form of the resident backward for rows that bwd_plan_for keeps off
+// the resident kernels because of their alignment; none where an output
+// overlaps an input (a row's column terms are then read after it is stored).
+// Its blocking is the resident one: nblk never exceeds the looped kernel's
+// (bwd_num_blocks), which sizes the workspace.  Measured on MI355X at f32
+// [4099, 1030] against the looped kernels: forward 8.6 us from 11.8, backward
+// 12.9 from 40.1, its finalize 3.5 from 4.6 (a quarter of the partial rows).
+template <class S>
+inline Plan ragged_bwd_plan(const void* x, const void* dy, const void* dx, const void* dr,
+                            int64_t rows, int cols) {
+    const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(typename S::T));
+    for (const void* o : {dx, dr})
+        if (!disjoint(o, x, bytes) || !disjoint(o, dy, bytes)) return Plan{};
+    const Plan p = ragged(bwd_plan<S>(row_slots(cols, S::kVec)), cols, S::kVec);
+    if (p.tpr != 0 && p.g > 1 && static_cast<int64_t>(p.g) * cols * 4 > 64 * 1024) return Plan{};
+    return p;
+}
+
 template <class S, bool ACC>
 int launch_rms_mul_bwd_resident(const Plan& p, int64_t nblk, const void* x, const void* gamma,
                                 const float* inv_rms, const void* gy, void* dx, void* dr,
@@ -1320,10 +1411,16 @@ int launch_rms_mul_bwd_resident(const Plan& p, int64_t nblk, const void* x, cons
 #define AGK_X(a, b, c, d)                                                                  \
     if constexpr (bwd_shape_enabled<S>(a, b)) {                                            \
         if (p.tpr == a && p.nv == b && p.g == c) {                                         \
-            hipLaunchKernelGGL((rms_mul_bwd_resident<S, a, b, c, rms_mul_sets<S>(b, d),    \
-                                                     ACC>),                                \
-                               dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, xp, \
-                               gp, inv_rms, gyp, dxp, drp, partials, rows, cols);           \
+            if (p.rag)                                                                     \
+                hipLaunchKernelGGL((rms_mul_bwd_resident<S, a, b, c, rms_mul_sets<S>(b, d), \
+                                                         ACC, true>),                      \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, \
+                                   xp, gp, inv_rms, gyp, dxp, drp, partials, rows, cols);  \
+            else                                                                           \
+                hipLaunchKernelGGL((rms_mul_bwd_resident<S, a, b, c, rms_mul_sets<S>(b, d), \
+                                                         ACC>),                            \
+                                   dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, \
+                                   xp, gp, inv_rms, gyp, dxp, drp, partials, rows, cols);  \
             return check_launch();                                                         \
         }                                                                                  \
     }
@@ -1395,7 +1492,11 @@ int launch_bwd(const void* x, const void* gamma, const float* inv_rms, const voi
         rpb = bwd_rows_per_block(rows);
         nblk = bwd_num_blocks(rows);
     }
-    if (p.tpr != 0 && rows <= kFewRowsMax) {
+    if (p.tpr == 0) {
+        p = ragged_bwd_plan<S>(x, dy, dx, dr, rows, cols);
+        if (p.tpr != 0) nblk = bwd_resident_blocks(rows);
+    }
+    if (p.tpr != 0 && !p.rag && rows <= kFewRowsMax) {
         nblk = 0;
         return dr ? launch_fewrows<S, kBwdRmsMul>(p, x, gamma, inv_rms, dy, dx, dr, dgamma, rows,
                                                   cols, accumulate, acc_dg, st)
@@ -1866,10 +1967,15 @@ int agk_mul_rowbcast_bwd(const void* gy, const void* a, const void* b, void* da,
     }
     const int c = static_cast<int>(cols);
     int64_t nblk = 0, rpb = 0;
-    const Plan p = dtype == AGK_F32 ? bwd_plan_for<F32>(a, b, gy, da, rows, c, nblk, rpb)
-                                    : bwd_plan_for<BF16>(a, b, gy, da, rows, c, nblk, rpb);
+    Plan p = dtype == AGK_F32 ? bwd_plan_for<F32>(a, b, gy, da, rows, c, nblk, rpb)
+                              : bwd_plan_for<BF16>(a, b, gy, da, rows, c, nblk, rpb);
+    if (p.tpr == 0) {
+        p = dtype == AGK_F32 ? ragged_bwd_plan<F32>(a, gy, da, nullptr, rows, c)
+                             : ragged_bwd_plan<BF16>(a, gy, da, nullptr, rows, c);
+        if (p.tpr != 0) nblk = bwd_resident_blocks(rows);
+    }
     if (nblk > 0x7fffffffLL) return AGK_EINVAL;
-    if (p.tpr != 0 && rows <= kFewRowsMax)  // few rows: db written directly
+    if (p.tpr != 0 && !p.rag && rows <= kFewRowsMax)  // few rows: db written directly
         return dtype == AGK_F32
                    ? launch_fewrows<F32, kBwdMul>(p, a, b, nullptr, gy, da, nullptr, db, rows, c,
                                                   acc_da, acc_db, st)
@@ -1931,11 +2037,15 @@ int agk_sum_rows(const void* x, float* out, void* workspace, size_t workspace_by
     float* partials = static_cast<float*>(workspace);
     const int c = static_cast<int>(cols);
     int64_t nblk = 0, rpb = 0;
-    const Plan p = dtype == AGK_F32 ? bwd_plan_for<F32>(x, nullptr, x, nullptr, rows, c, nblk, rpb)
-                                    : bwd_plan_for<BF16>(x, nullptr, x, nullptr, rows, c, nblk,
-                                                         rpb);
+    Plan p = dtype == AGK_F32 ? bwd_plan_for<F32>(x, nullptr, x, nullptr, rows, c, nblk, rpb)
+                              : bwd_plan_for<BF16>(x, nullptr, x, nullptr, rows, c, nblk, rpb);
+    if (p.tpr == 0) {
+        p = dtype == AGK_F32 ? ragged_bwd_plan<F32>(x, x, nullptr, nullptr, rows, c)
+                             : ragged_bwd_plan<BF16>(x, x, nullptr, nullptr, rows, c);
+        if (p.tpr != 0) nblk = bwd_resident_blocks(rows);
+    }
     if (nblk > 0x7fffffffLL) return AGK_EINVAL;
-    if (p.tpr != 0 && rows <= kFewRowsMax)  // few rows: out written directly
+    if (p.tpr != 0 && !p.rag && rows <= kFewRowsMax)  // few rows: out written directly
         return dtype == AGK_F32
                    ? launch_fewrows<F32, kBwdColSum>(p, nullptr, nullptr, nullptr, x, nullptr,
                                                      nullptr, out, rows, c, 0, accumulate, st)

@@ -124,6 +124,58 @@ __device__ __forceinline__ void store16_stream(typename S::T* p, u32x4 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
+// ---- ragged rows ------------------------------------------------------------------
+// Rows that are not whole 16-byte slots, or that start off a 16-byte boundary,
+// run on the same resident kernels in a ragged form (template argument RAG):
+// 16-byte accesses at element alignment, and the row's last slot moved back to
+// end with the row, so that it overlaps the slot before it by `dup` elements.
+// An overlapped element has the same value in both slots: row sums leave it out
+// of the last one, plain stores write it twice with the same bits, and
+// accumulating stores skip it in the last one.  Rows of at least one slot only.
+// Measured on MI355X (copy of 512 MiB, 16 bytes per lane): 6.4 TB/s aligned,
+// 5.9-6.1 at 4-byte alignment, 5.8-5.9 at 2-byte alignment.
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+
+template <class S>
+__device__ __forceinline__ u32x4 load16_any(const typename S::T* p) {
+    if constexpr (sizeof(typename S::T) == 4) return *reinterpret_cast<const u32x4_a4*>(p);
+    else return *reinterpret_cast<const u32x4_a2*>(p);
+}
+template <class S>
+__device__ __forceinline__ u32x4 load16_any_stream(const typename S::T* p) {
+    if constexpr (sizeof(typename S::T) == 4)
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a4*>(p));
+    else
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a2*>(p));
+}
+template <class S>
+__device__ __forceinline__ void store16_any_stream(typename S::T* p, u32x4 v) {
+    if constexpr (sizeof(typename S::T) == 4)
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a4*>(p));
+    else
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a2*>(p));
+}
+
+// First column of slot `slot` (columns slot * W .., or moved back to end with
+// the row); at least cols for a slot past the row.
+template <bool RAG, int W>
+__device__ __forceinline__ int slot_col(int slot, int cols) {
+    const int c = slot * W;
+    if constexpr (RAG) return c < cols && c + W > cols ? cols - W : c;
+    else return c;
+}
+
+// Zeroes the first `dup` elements (those the slot before holds too).
+template <int W>
+__device__ __forceinline__ void drop_dup(float (&f)[W], int dup) {
+#pragma unroll
+    for (int e = 0; e < W; ++e) f[e] = e < dup ? 0.0f : f[e];
+}
+
+// Slots of a row, the last one perhaps partly filled.
+inline int64_t row_slots(int64_t cols, int w) { return (cols + w - 1) / w; }
+
 // ---- buffer resources ---------------------------------------------------------
 // A raw buffer resource (stride 0, no swizzle) over `bytes` bytes at `base`.
 // The hardware range-checks every access against `bytes`: a load at or past
@@ -146,6 +198,15 @@ __device__ __forceinline__ u32x4 bload16_stream(rsrc_t r, uint32_t off) {
 }
 __device__ __forceinline__ void bstore16_stream(rsrc_t r, uint32_t off, u32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, kCachePolicyNT);
+}
+// One element, rounded to storage.
+template <class S>
+__device__ __forceinline__ void bstore_elem(rsrc_t r, uint32_t off, float v) {
+    if constexpr (sizeof(typename S::T) == 4)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(f32_to_bf16_bits(v)), r, off,
+                                              0, 0);
 }
 __device__ __forceinline__ float bload_f32(rsrc_t r, uint32_t off) {
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
@@ -212,6 +273,7 @@ struct Plan {
     int tpr = 0;  // 0 = looped kernel
     int nv = 0;
     int g = 0;
+    bool rag = false;  // the ragged form
 };
 
 // Instantiated shapes.  Each compiles without register spills for both
@@ -282,12 +344,18 @@ inline Plan pick_plan(const Shape3 (&shapes)[N], int64_t nslot, int nv0, int sma
     }
     if (has_shape(shapes, p)) return p;
     for (const Shape3& s : shapes)  // same (TPR, NV), another G
-        if (s.tpr == p.tpr && s.nv == p.nv) return Plan{s.tpr, s.nv, s.g};
+        if (s.tpr == p.tpr && s.nv == p.nv) return Plan{s.tpr, s.nv, s.g, false};
     return Plan{};
 }
 
 inline Plan fwd_plan(int64_t nslot, int64_t rows) {
     return pick_plan(kFwdShapes, nslot, rows > kLargeRows ? 2 : 4, 512, 8);
+}
+
+// Whether two tensors of `bytes` bytes share no byte (NULL: no tensor).
+inline bool disjoint(const void* a, const void* b, int64_t bytes) {
+    const char *p = static_cast<const char*>(a), *q = static_cast<const char*>(b);
+    return !p || !q || p + bytes <= q || q + bytes <= p;
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
