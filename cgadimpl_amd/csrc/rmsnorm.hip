@@ -1128,9 +1128,9 @@ inline Plan bwd_plan(int64_t nslot) {
 }
 
 // p (the shape for row_slots(cols, w) slots) in its ragged form; none for rows
-// of less than one slot.
-inline Plan ragged(Plan p, int64_t cols, int w) {
-    if (p.tpr == 0 || cols < w) return Plan{};
+// of less than one slot, or few short ones.
+inline Plan ragged(Plan p, int64_t rows, int64_t cols, int w) {
+    if (p.tpr == 0 || cols < w || few_short_rows(rows, cols)) return Plan{};
     p.rag = true;
     return p;
 }
@@ -1221,7 +1221,7 @@ int launch_fwd(const void* x, const void* gamma, void* y, float* inv_rms, int64_
     }
     // Rows off the 16-byte grid: the same shape in its ragged form.  In place
     // (y = x) too: a row's loads end in its sum, which comes before its stores.
-    if (!vec) p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), cols, S::kVec);
+    if (!vec) p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), rows, cols, S::kVec);
     return launch_fwd_plan<S>(p, x, gamma, y, inv_rms, rows, cols, eps, st);
 }
 
@@ -1237,11 +1237,16 @@ int launch_mul_fwd(const void* a, const void* b, void* y, int64_t rows, int cols
     const bool vec = (cols % S::kVec) == 0 && aligned16(a) && aligned16(b) && aligned16(y);
     Plan p;
     if (vec) p = fwd_plan(cols / S::kVec, rows);
-    // Ragged rows, unless y overwrites an operand: a slot's stores may then
-    // come before the loads of the slot that overlaps it.
+    // Ragged rows in many rows or large tensors: a product reads each row once
+    // either way, so the element-wise kernel keeps the others (measured on
+    // MI355X, us, element-wise / ragged: f32 2500 x 4099 15.1 / 16.2, bf16 8192 x
+    // 8193 46 / 56; f32 65536 x 1001 123 / 91, 8192 x 8193 118 / 90, bf16 65536 x 129
+    // 25.7 / 10.7).  Not where y overwrites an operand: a slot's stores may come
+    // before the loads of the slot that overlaps it.
     const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(T));
-    if (!vec && disjoint(a, y, bytes) && disjoint(b, y, bytes))
-        p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), cols, S::kVec);
+    if (!vec && (rows >= kLargeRows || bytes >= (1LL << 28)) && disjoint(a, y, bytes) &&
+        disjoint(b, y, bytes))
+        p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), rows, cols, S::kVec);
     if (p.tpr == 0) {
         if (rows > 0x7fffffffLL) return AGK_EINVAL;
         const int64_t chunk = mul_chunk(rows, cols, vec ? S::kVec : 1);
@@ -1392,7 +1397,7 @@ inline Plan ragged_bwd_plan(const void* x, const void* dy, const void* dx, const
     const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(typename S::T));
     for (const void* o : {dx, dr})
         if (!disjoint(o, x, bytes) || !disjoint(o, dy, bytes)) return Plan{};
-    const Plan p = ragged(bwd_plan<S>(row_slots(cols, S::kVec)), cols, S::kVec);
+    const Plan p = ragged(bwd_plan<S>(row_slots(cols, S::kVec)), rows, cols, S::kVec);
     if (p.tpr != 0 && p.g > 1 && static_cast<int64_t>(p.g) * cols * 4 > 64 * 1024) return Plan{};
     return p;
 }

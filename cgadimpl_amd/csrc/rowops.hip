@@ -169,7 +169,9 @@ __device__ __forceinline__ void row_reduce(float (&v)[N],
 //   put_f32(p, v), put_val(p, v)     p[row] = v (fp32 / storage type)
 // a and b are the elements of in0 and in1 (b = 0 for one-input ops).
 
-template <class S, int TPR, int NV, int G, int NIN>
+// RAG: ragged rows (rowcommon.hpp); the reductions leave out the elements that
+// the last slot repeats.
+template <class S, int TPR, int NV, int G, int NIN, bool RAG = false>
 struct Resident {
     using T = typename S::T;
     static constexpr int W = S::kVec;
@@ -203,12 +205,46 @@ struct Resident {
         const T* y = NIN == 2 ? static_cast<const T*>(p.in1) + off : nullptr;
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int col = (t + k * TPR) * W;
+            const int col = slot_col<RAG, W>(t + k * TPR, cols);
             const bool ok = active && col < cols;
-            a[k] = ok ? load16_stream<S>(x + col) : u32x4{0u, 0u, 0u, 0u};
-            if constexpr (NIN == 2)
-                b[k] = ok ? load16_stream<S>(y + col) : u32x4{0u, 0u, 0u, 0u};
+            a[k] = ok ? load_row(x + col) : u32x4{0u, 0u, 0u, 0u};
+            if constexpr (NIN == 2) b[k] = ok ? load_row(y + col) : u32x4{0u, 0u, 0u, 0u};
         }
+    }
+
+    __device__ static __forceinline__ u32x4 load_row(const T* p) {
+        if constexpr (RAG) return load16_any_stream<S>(p);
+        else return load16_stream<S>(p);
+    }
+    __device__ static __forceinline__ u32x4 load_col(const T* p) {
+        if constexpr (RAG) return load16_any<S>(p);
+        else return load16<S>(p);
+    }
+    // Elements of slot t + k * TPR that the slot before it holds too.
+    __device__ __forceinline__ int dup(int k) const {
+        if constexpr (RAG) return (t + k * TPR) * W - slot_col<RAG, W>(t + k * TPR, cols);
+        else return 0;
+    }
+
+    // out[col ..] (+)= r for slot k.
+    __device__ __forceinline__ void put(T* o, int k, int acc, float (&r)[W]) const {
+        const int col = slot_col<RAG, W>(t + k * TPR, cols);
+        if constexpr (RAG) {
+            if (acc && dup(k) > 0) {  // a repeated element is the other slot's to add to
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+                    if (e >= dup(k)) S::put(o + col + e, acc_add(S::get(o + col + e), r[e]));
+                return;
+            }
+        }
+        if (acc) {
+            float old[W];
+            S::unpack(load_row(o + col), old);
+#pragma unroll
+            for (int e = 0; e < W; ++e) r[e] = acc_add(old[e], r[e]);
+        }
+        if constexpr (RAG) store16_any_stream<S>(o + col, S::pack(r));
+        else store16_stream<S>(o + col, S::pack(r));
     }
 
     template <class R, int N, class F>
@@ -229,7 +265,10 @@ struct Resident {
                     float o[N];
                     f(fa[e], NIN == 2 ? fb[e] : 0.0f, o);
 #pragma unroll
-                    for (int i = 0; i < N; ++i) part[i][e] = R::op(part[i][e], o[i]);
+                    for (int i = 0; i < N; ++i) {
+                        if (RAG) part[i][e] = e < dup(k) ? part[i][e] : R::op(part[i][e], o[i]);
+                        else part[i][e] = R::op(part[i][e], o[i]);
+                    }
                 }
             }
         }
@@ -312,7 +351,8 @@ struct Resident {
 #pragma unroll
                 for (int e = 0; e < W; ++e) {
                     kept[k][e] = f(fa[e], NIN == 2 ? fb[e] : 0.0f);
-                    part[e] += kept[k][e];
+                    if (RAG) part[e] += e < dup(k) ? 0.0f : kept[k][e];
+                    else part[e] += kept[k][e];
                 }
             }
         }
@@ -330,8 +370,7 @@ struct Resident {
         T* o = static_cast<T*>(out) + row * static_cast<int64_t>(cols);
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int col = (t + k * TPR) * W;
-            if (col < cols) {
+            if ((t + k * TPR) * W < cols) {
                 float r[W];
                 if constexpr (kBig) {  // recomputed: the same function of the same value
                     float fa[W], fb[W];
@@ -343,13 +382,7 @@ struct Resident {
 #pragma unroll
                     for (int e = 0; e < W; ++e) r[e] = g(kept[k][e]);
                 }
-                if (acc) {
-                    float old[W];
-                    S::unpack(load16_stream<S>(o + col), old);
-#pragma unroll
-                    for (int e = 0; e < W; ++e) r[e] = acc_add(old[e], r[e]);
-                }
-                store16_stream<S>(o + col, S::pack(r));
+                put(o, k, acc, r);
             }
         }
     }
@@ -361,32 +394,26 @@ struct Resident {
         T* o = static_cast<T*>(out) + row * static_cast<int64_t>(cols);
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int col = (t + k * TPR) * W;
+            const int col = slot_col<RAG, W>(t + k * TPR, cols);
             if (col < cols) {
                 float fa[W], fb[W], fu[W], fv[W], r[W];
                 S::unpack(a[k], fa);
                 if constexpr (NIN == 2) S::unpack(b[k], fb);
                 if (c0) {
-                    S::unpack(load16<S>(static_cast<const T*>(c0) + col), fu);
+                    S::unpack(load_col(static_cast<const T*>(c0) + col), fu);
                 } else {
 #pragma unroll
                     for (int e = 0; e < W; ++e) fu[e] = d0;
                 }
                 if (c1) {
-                    S::unpack(load16<S>(static_cast<const T*>(c1) + col), fv);
+                    S::unpack(load_col(static_cast<const T*>(c1) + col), fv);
                 } else {
 #pragma unroll
                     for (int e = 0; e < W; ++e) fv[e] = d1;
                 }
 #pragma unroll
                 for (int e = 0; e < W; ++e) r[e] = f(fa[e], NIN == 2 ? fb[e] : 0.0f, fu[e], fv[e]);
-                if (acc) {
-                    float old[W];
-                    S::unpack(load16_stream<S>(o + col), old);
-#pragma unroll
-                    for (int e = 0; e < W; ++e) r[e] = acc_add(old[e], r[e]);
-                }
-                store16_stream<S>(o + col, S::pack(r));
+                put(o, k, acc, r);
             }
         }
     }
@@ -953,9 +980,9 @@ struct LseJvp {
 
 // ---- kernels and launch ------------------------------------------------------------
 
-template <class S, int TPR, int NV, int G, class Op>
+template <class S, int TPR, int NV, int G, class Op, bool RAG = false>
 __global__ __launch_bounds__(TPR * G) void row_resident(const RowArgs p, int64_t rows, int cols) {
-    using Ctx = Resident<S, TPR, NV, G, Op::kIn>;
+    using Ctx = Resident<S, TPR, NV, G, Op::kIn, RAG>;
     __shared__ float red[2][Ctx::kSlots];
     Ctx c(p, rows, cols, red);
     Op::run(c, p);
@@ -1084,6 +1111,30 @@ int maybe_team(const RowArgs& p, void* ws, size_t ws_bytes, int64_t rows, int co
 
 int team_wait_limit() { return agk::team_wait_polls(); }
 
+// Rows short enough for 32-bit buffer offsets.
+template <class S>
+inline bool fits_buffer(int cols) {
+    return static_cast<uint64_t>(cols) * sizeof(typename S::T) < 0x80000000ull;
+}
+
+// Rows off the 16-byte grid take the resident kernels' ragged form (shapes of
+// up to four slots per lane), except wide rows that the 16-byte looped kernel's
+// head / body / tail form serves better: from kVecMinCols columns, rows of one
+// input, and rows of two past 2048 bf16 slots.  Measured on MI355X (graph
+// replays, us, before against ragged):
+//   f32 4099 x 1001: layernorm 11.4 / 12.0 -> 7.4 / 8.5, softmax 11.1 / 11.5 ->
+//     6.9 / 9.5; f32 20000 x 4099: 256 / 266 -> 126 / 164, 276 / 265 -> 111 / 161;
+//     bf16 20000 x 4099: 196 / 198 -> 82 / 113, 208 / 186 -> 77 / 98 (element-wise
+//     looped kernel before);
+//   f32 4000 x 16383 (looped 16-byte kernel before): backward 163 -> 139, softmax
+//     forward 85 -> 93, log-sum-exp forward 39 -> 42; bf16 4000 x 30001: backward
+//     143 -> 168, softmax forward 75 -> 101, log-sum-exp forward 37 -> 57.
+template <class Op, class S>
+inline bool prefers_looped_vec(const RowArgs& p, int cols) {
+    if (cols < kVecMinCols || !fits_buffer<S>(cols) || !same_offset<typename S::T>(p)) return false;
+    return Op::kIn == 1 || (std::is_same<S, BF16>::value && row_slots(cols, S::kVec) > 2048);
+}
+
 template <class Op, class S>
 int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
     const bool vec = (cols % S::kVec) == 0 && aligned16(p.in0) && aligned_or_null(p.in1) &&
@@ -1093,8 +1144,14 @@ int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
     if (vec) pl = fwd_plan(cols / S::kVec, rows);
     if (stream_wide_bf16<Op>() && std::is_same<S, BF16>::value && pl.nv == 8) pl = Plan{};
     if (four_slots_bf16<Op>() && std::is_same<S, BF16>::value && pl.nv == 2 && pl.tpr >= 128) {
-        const Plan q{pl.tpr / 2, 4, pl.tpr >= 512 ? 1 : 512 / pl.tpr};
+        const Plan q{pl.tpr / 2, 4, pl.tpr >= 512 ? 1 : 512 / pl.tpr, false};
         if (has_shape(kFwdShapes, q)) pl = q;
+    }
+    if (!vec && cols >= S::kVec && !few_short_rows(rows, cols) &&
+        !prefers_looped_vec<Op, S>(p, cols)) {
+        pl = fwd_plan(row_slots(cols, S::kVec), rows);
+        pl.rag = true;
+        if (pl.nv > 4) pl = Plan{};
     }
     if constexpr (Resident16<Op>::value) {
         const int64_t nslot = cols / S::kVec;
@@ -1110,7 +1167,7 @@ int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
         // rows short enough for 32-bit buffer offsets: whole 16-byte slots and
         // aligned pointers, or (from kVecMinCols columns) every row tensor at
         // the same offset from a 16-byte boundary
-        const bool fits = static_cast<uint64_t>(cols) * sizeof(typename S::T) < 0x80000000ull;
+        const bool fits = fits_buffer<S>(cols);
         if (vec && fits)
             hipLaunchKernelGGL((row_looped_vec<S, Op, true>), dim3(static_cast<unsigned>(rows)),
                                dim3(kVecLanes), 0, st, p, rows, cols);
@@ -1126,6 +1183,14 @@ int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
     if (grid > 0x7fffffffLL) return AGK_EINVAL;
 #define AGK_X(a, b, c)                                                                          \
     if (pl.tpr == a && pl.nv == b && pl.g == c) {                                               \
+        if constexpr (b <= 4) {                                                                 \
+            if (pl.rag) {                                                                       \
+                hipLaunchKernelGGL((row_resident<S, a, b, c, Op, true>),                        \
+                                   dim3(static_cast<unsigned>(grid)), dim3(a * c), 0, st, p,    \
+                                   rows, cols);                                                 \
+                return check_launch();                                                          \
+            }                                                                                   \
+        }                                                                                       \
         hipLaunchKernelGGL((row_resident<S, a, b, c, Op>), dim3(static_cast<unsigned>(grid)),    \
                            dim3(a * c), 0, st, p, rows, cols);                                  \
         return check_launch();                                                                  \

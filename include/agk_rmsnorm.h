@@ -369,7 +369,10 @@ int agk_set_team_forward(int enabled);
  * backward plan[3] = rows per tile, plan[4] = dgamma partial rows, 0 when
  * the tiles write dgamma directly), else the looped kernel (rows that are
  * not a whole number of 16-byte slots, or too wide for registers and not
- * split).  A resident backward of at most 255 rows reports 0 partial rows:
+ * split).  Rows that are not whole slots may run the ragged form of a
+ * resident shape instead, with at most min(256, rows) dgamma partial rows;
+ * the plan reports the looped kernel's blocking, which the workspace is
+ * sized for, either way.  A resident backward of at most 255 rows reports 0 partial rows:
  * it runs row and column workgroups in one launch and writes dgamma
  * directly.  Used by the tests to run every reachable shape.                 */
 int agk_rmsnorm_launch_plan(int64_t rows, int64_t cols, int dtype, int backward,

@@ -21,8 +21,10 @@
  *
  * Any alignment and any cols are accepted: 16-byte aligned tensors with cols
  * a multiple of the vector width (4 fp32 / 8 bf16) take the register-resident
- * kernels (one HBM read per input element, one write per output element);
- * anything else takes a looped kernel that re-reads the row from cache.
+ * kernels (one HBM read per input element, one write per output element), and
+ * other rows of at least one vector their ragged form; rows too wide for
+ * registers, and few short ragged rows, take a looped kernel that re-reads the
+ * row from cache.
  */
 #ifndef AGK_ROWOPS_H
 #define AGK_ROWOPS_H

@@ -47,7 +47,7 @@ def _check(x, g, dy, y, inv, dx, dg, label):
 
 
 @pytest.mark.parametrize("dtype,cols", CASES, ids=str)
-@pytest.mark.parametrize("rows", [1, 37, 300])
+@pytest.mark.parametrize("rows", [1, 37, 600])
 def test_layer_matches_fp64(cuda, dtype, cols, rows):
     import torch
     print(f"{dtype} {rows}x{cols}", flush=True)
@@ -84,7 +84,7 @@ def test_composition_equals_its_two_calls(cuda, dtype, cols, accumulate):
     """agk_rms_mul_bwd against the multiply's VJP then the RMSNorm VJP of dr, bit for bit, and
     the column sums of a linear layer's bias."""
     import torch
-    rows = 300
+    rows = 600
     x, g, gy = device_inputs((rows, cols), dtype, cols, cuda)
     r, inv = agk.rmsnorm_fwd(x, None, EPS)
     y = agk.mul_rowbcast_fwd(r, g)
@@ -111,6 +111,20 @@ def test_composition_equals_its_two_calls(cuda, dtype, cols, accumulate):
     assert ((s.double() - gy.double().sum(0)).abs() <= 1e-5 * gy.double().abs().sum(0)).all().item()
 
 
+@pytest.mark.parametrize("dtype,cols", [("f32", 5), ("bf16", 9), ("f32", 129), ("bf16", 1001)],
+                         ids=str)
+def test_many_row_multiply(cuda, dtype, cols):
+    """The row-vector multiply over enough rows for its ragged form: torch's product, bit for
+    bit, also in place."""
+    import torch
+    a, b, _ = device_inputs((16411, cols), dtype, cols, cuda)
+    want = a * b
+    y = agk.mul_rowbcast_fwd(a, b)
+    agk.mul_rowbcast_fwd(a, b, y=a)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want) and torch.equal(a, want)
+
+
 @pytest.mark.parametrize("dtype,cols", [("f32", 1024), ("bf16", 2048), ("f32", 100),
                                         ("bf16", 8192)], ids=str)
 @pytest.mark.parametrize("shift", [1, 3])
@@ -119,7 +133,7 @@ def test_rows_off_a_boundary_match_aligned_rows(cuda, dtype, cols, shift):
     own offset): y, inv_rms and dx are the aligned call's bits (the same lanes add the same
     slots); dgamma's partial rows too."""
     import torch
-    rows = 300
+    rows = 600
     x, g, dy = device_inputs((rows, cols), dtype, cols + shift, cuda)
 
     def off(t, n):
@@ -141,7 +155,7 @@ def test_infinities_and_nans_stay_where_they_belong(cuda, dtype, cols):
     """An infinite or NaN dy or x in the overlapped columns (which two slots hold): the same
     NaN / infinity pattern as the formula in fp32, other rows and columns untouched."""
     import torch
-    x, g, dy = device_inputs((300, cols), dtype, cols, cuda)
+    x, g, dy = device_inputs((600, cols), dtype, cols, cuda)
     _, _, clean_dx, clean_dg, _ = _ref(x, g, dy)
     dy[3, cols - 3] = float("inf")
     dy[5, cols - 1] = float("nan")
@@ -155,7 +169,7 @@ def test_infinities_and_nans_stay_where_they_belong(cuda, dtype, cols):
     want = r * (gy - xf * s)
     assert torch.equal(torch.isnan(dx), torch.isnan(want))
     assert torch.equal(torch.isinf(dx), torch.isinf(want))
-    rows = [i for i in range(300) if i not in (3, 5, 7)]
+    rows = [i for i in range(600) if i not in (3, 5, 7)]
     bar = (1e-5 + (2.0 ** -8 if dtype == "bf16" else 0.0)) * clean_dx.abs().amax()
     assert ((dx[rows].double() - clean_dx[rows]).abs() <= bar).all().item()
     bad = [cols - 9, cols - 3, cols - 1]
@@ -163,3 +177,81 @@ def test_infinities_and_nans_stay_where_they_belong(cuda, dtype, cols):
     good = torch.ones(cols, dtype=torch.bool, device=cuda)
     good[bad] = False
     assert torch.isfinite(dg[good]).all().item()
+
+
+ROWOP_COLS = {"f32": [4, 5, 9, 61, 253, 515, 1001, 4099, 8195, 16383],
+              "bf16": [8, 9, 121, 1001, 4099, 8195, 16391, 32767]}
+
+
+@pytest.mark.parametrize("dtype,cols", [(d, c) for d in ROWOP_COLS for c in ROWOP_COLS[d]], ids=str)
+@pytest.mark.parametrize("rows", [1, 541])
+def test_row_ops_match_fp64(cuda, dtype, cols, rows):
+    """LayerNorm, softmax and log-sum-exp, the RMSNorm JVP, with masked logits in the overlapped
+    columns.  Bars: 1e-5 of the row's scale (fp32 sums and the hardware exponential's
+    |z - max| 2^-24 ln 2), one storage rounding for bf16."""
+    import torch
+    print(f"{dtype} {rows}x{cols}", flush=True)
+    x, g, dy = device_inputs((rows, cols), dtype, rows * 13 + cols, cuda)
+    one = 2.0 ** -8 if dtype == "bf16" else 0.0
+    bar = 1e-5 + one
+
+    def close(got, want, scale, what):
+        assert ((got.double() - want).abs() <= bar * scale + 1e-30).all().item(), what
+
+    def accumulates(call, fresh, what):
+        pre = torch.full_like(x, 0.25)
+        got = call(pre.clone())
+        torch.cuda.synchronize()
+        if dtype == "f32":
+            assert torch.equal(got, pre + fresh), what
+        else:  # the accumulated term is not rounded to bf16 first
+            f = fresh.float()
+            assert ((got.float() - (0.25 + f)).abs() <= 2.0 ** -8 * (0.25 + f.abs())).all().item()
+
+    x64, d64, g64 = x.double(), dy.double(), g.double()
+    y, mean, rstd = agk.layernorm_fwd(x, 1e-5)
+    dx = agk.layernorm_bwd(x, mean, rstd, dy)
+    m = x64.mean(-1, keepdim=True)
+    r = ((x64 - m).square().mean(-1, keepdim=True) + 1e-5).rsqrt()
+    xh = (x64 - m) * r
+    close(y, xh, xh.abs().amax(-1, keepdim=True), "layernorm")
+    want = r * (d64 - d64.mean(-1, keepdim=True) - xh * (d64 * xh).mean(-1, keepdim=True))
+    # |dx| <= r (2 + max|xh|) max|dy| (mean |xh| <= 1): the scale its rounding is relative to
+    close(dx, want, r * (2 + xh.abs().amax(-1, keepdim=True)) * d64.abs().amax(-1, keepdim=True),
+          "layernorm dx")
+    accumulates(lambda o: agk.layernorm_bwd(x, mean, rstd, dy, dx=o, accumulate=True), dx, "ln acc")
+
+    _, inv = agk.rmsnorm_fwd(x, g, EPS)
+    ty = agk.rmsnorm_jvp(x, g, inv, dy, tgamma=g)
+    ri = inv.double().view(-1, 1)
+    want = g64 * ri * (d64 - x64 * ri.square() * (d64 * x64).mean(-1, keepdim=True)) + g64 * x64 * ri
+    # the same bound for each of the rule's two terms
+    xr = (x64 * ri).abs().amax(-1, keepdim=True)
+    close(ty, want, 1.5 * (ri * (1 + xr) * d64.abs().amax(-1, keepdim=True) + 1.5 * xr), "jvp")
+
+    z = (x * 3).contiguous()
+    z[:, -2:] = float("-inf")   # columns that two slots hold
+    z64 = z.double()
+    for ws in (False, None):
+        s = agk.softmax_fwd(z, workspace=ws)
+        dz = agk.softmax_bwd(s, dy, workspace=ws)
+        p = torch.softmax(z64, -1)
+        close(s, p, p.amax(-1, keepdim=True), "softmax")
+        s64 = s.double()
+        want = s64 * (d64 - (s64 * d64).sum(-1, keepdim=True))
+        close(dz, want, (s64 * d64.abs().amax(-1, keepdim=True)).amax(-1, keepdim=True) * 2, "softmax dz")
+        dl = dy[:, :1].contiguous()
+        lb = agk.logsumexp_bwd(z, dl, workspace=ws)
+        close(lb, dl.double() * p, dl.double().abs() * p.amax(-1, keepdim=True), "lse dz")
+    accumulates(lambda o: agk.softmax_bwd(s, dy, dz=o, accumulate=True), dz, "softmax acc")
+    lse, keep = agk.logsumexp_fwd_keep(z)
+    want = torch.logsumexp(z64, -1, keepdim=True)
+    assert ((keep.double() - want).abs() <= 1e-5 * (1 + want.abs())).all().item()
+    assert ((lse.double() - want).abs() <= bar * (1 + want.abs())).all().item()
+    jv = agk.logsumexp_jvp(z, dy)
+    want = (p * d64).sum(-1, keepdim=True)
+    assert ((jv.double() - want).abs() <= bar * (p * d64.abs()).sum(-1, keepdim=True)).all().item()
+    in_place = z.clone()
+    agk.softmax_fwd(in_place, y=in_place)
+    torch.cuda.synchronize()
+    assert torch.equal(in_place, agk.softmax_fwd(z))
