@@ -15,6 +15,8 @@
 // The host merges adjacent axes that both operands walk contiguously (and
 // drops extent-1 output axes), so a launch sees at most 8 axes, usually 2-3.
 //
+// Otherwise:
+//
 // Forward / full-shape gradient (y (+)= a * b): one workgroup row per run of
 // the innermost output axis; its base offsets into a and b are decomposed once
 // per run, the lanes walk the run, 16 bytes at a time when the innermost axis
@@ -32,6 +34,14 @@
 //    (short sums) or one 256-lane workgroup (long sums) per output element;
 //    lane l takes positions l, l + lanes, ... of the reduced index space in
 //    row-major order, and the lanes' partials meet in a fixed tree in LDS.
+
+//
+// The broadcasts that training code writes most -- a full operand times a vector
+// per group of rows ([B, T, D] * [B, 1, D], [B, T, D] * [T, D]) or a scalar per row
+// ([B, T, D] * [B, T, 1]) -- have kernels of their own over a rows x cols view of
+// the full operand (RowsView): 16-byte accesses at any element alignment
+// (rowcommon.hpp, ragged rows), and a backward that reads gy and the full operand
+// once for both gradients.
 
 #include <hip/hip_runtime.h>
 
@@ -278,6 +288,242 @@ __global__ __launch_bounds__(kBcastBlock) void bcast_reduce_cols_kernel(
     }
 }
 
+// ---- rows x cols views -----------------------------------------------------------
+// The full operand as rows of cols contiguous elements; the other is a vector of
+// cols elements per group of `group` consecutive rows (row r uses vector
+// r / group), or with SCALAR one element per row.  cols holds at least one slot.
+
+// First column of slot `slot`: the last slot is moved back to end with the row.
+template <int W>
+__device__ __forceinline__ int64_t view_col(int64_t slot, int64_t cols) {
+    const int64_t c = slot * W;
+    return c + W > cols ? cols - W : c;
+}
+
+// y (+)= r for one slot, leaving out the first `dup` elements when adding.
+template <class S>
+__device__ __forceinline__ void view_store(typename S::T* y, float (&r)[S::kVec], int dup,
+                                           int accumulate) {
+    constexpr int W = S::kVec;
+    if (accumulate) {
+        if (dup > 0) {
+#pragma unroll
+            for (int e = 0; e < W; ++e)
+                if (e >= dup) S::put(y + e, acc_add(S::get(y + e), S::stored(r[e])));
+            return;
+        }
+        float old[W];
+        S::unpack(load16_any_stream<S>(y), old);
+#pragma unroll
+        for (int e = 0; e < W; ++e) r[e] = acc_add(old[e], S::stored(r[e]));
+    }
+    store16_any_stream<S>(y, S::pack(r));
+}
+
+// y (+)= full * other.  TPR lanes per row and chunk of 4 TPR slots, so that a
+// workgroup streams 16 KiB: HBM-bound (reads full, writes y; `other` comes from
+// the caches).
+// Measured on MI355X (us, before / now, the element-wise and run-per-workgroup
+// kernels before): bf16 32 x 2048 x 4096 by 32 x 1 x 4096 209 / 174 (6.2 TB/s), by 65536 x
+// 1 184 / 167; bf16 2 x 2048 x 4001 by 2 x 1 x 4001 78 / 16; f32 355 / 352.  With the
+// backward kernels below, both gradients: bf16 411 / 257, 587 / 274, 129 / 64; f32
+// 742 / 545, 794 / 573, 130 / 71.
+constexpr int kViewSlots = 4;
+
+template <class S, int TPR, bool SCALAR>
+__global__ __launch_bounds__(kBcastBlock) void bcast_rows_mul_kernel(
+    const typename S::T* __restrict__ full, const typename S::T* __restrict__ other,
+    typename S::T* __restrict__ y, int64_t rows, int64_t cols, int64_t group, int accumulate) {
+    constexpr int W = S::kVec, NV = kViewSlots, RPB = kBcastBlock / TPR;
+    const int t = threadIdx.x % TPR;
+    const int64_t nslot = (cols + W - 1) / W;
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + threadIdx.x / TPR; row < rows;
+         row += static_cast<int64_t>(gridDim.x) * RPB) {
+        const typename S::T* fr = full + row * cols;
+        typename S::T* yr = y + row * cols;
+        const typename S::T* orow = SCALAR ? other + row : other + row / group * cols;
+        const float os = SCALAR ? S::get(orow) : 0.0f;
+        for (int64_t s0 = static_cast<int64_t>(blockIdx.y) * (TPR * NV) + t; s0 < nslot;
+             s0 += static_cast<int64_t>(gridDim.y) * (TPR * NV)) {
+            u32x4 fv[NV], ov[SCALAR ? 1 : NV];
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int64_t s = s0 + k * TPR < nslot ? s0 + k * TPR : nslot - 1;
+                fv[k] = load16_any_stream<S>(fr + view_col<W>(s, cols));
+                if constexpr (!SCALAR) ov[k] = load16_any<S>(orow + view_col<W>(s, cols));
+            }
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                if (s0 + k * TPR >= nslot) break;
+                const int64_t col = view_col<W>(s0 + k * TPR, cols);
+                float f[W], o[W];
+                S::unpack(fv[k], f);
+                if constexpr (SCALAR) {
+#pragma unroll
+                    for (int e = 0; e < W; ++e) o[e] = os;
+                } else {
+                    S::unpack(ov[k], o);
+                }
+#pragma unroll
+                for (int e = 0; e < W; ++e) f[e] = f[e] * o[e];
+                view_store<S>(yr + col, f, static_cast<int>((s0 + k * TPR) * W - col), accumulate);
+            }
+        }
+    }
+}
+
+// Both gradients of full * (a vector per group of rows) in one pass over gy and
+// full: dfull (+)= gy * other (nullptr: not wanted), dother[group][col] (+)= the
+// group's sum of gy * full, exact products in fp64.  A workgroup takes TW slots of
+// columns of one group; its LANES / TW row lanes take the group's rows in turn,
+// BATCH of them in flight (loads past the group's end repeat its last row), and
+// their sums are added in lane order: an order fixed by the sizes.  HBM-bound at gy
+// + full + dfull; narrow tiles of 1024 lanes where wide ones would leave CUs idle.
+template <class S, int TW, int LANES, int BATCH>
+__global__ __launch_bounds__(LANES) void bcast_group_grad_kernel(
+    const typename S::T* __restrict__ gy, const typename S::T* __restrict__ full,
+    const typename S::T* __restrict__ other, typename S::T* __restrict__ dfull,
+    float* __restrict__ dother, int64_t groups, int64_t group, int64_t cols, int acc_full,
+    int acc_other) {
+    constexpr int W = S::kVec, RG = LANES / TW;
+    __shared__ double part[RG > 1 ? RG : 1][RG > 1 ? TW * W : 1];
+    const int t = threadIdx.x % TW;
+    const int g = threadIdx.x / TW;
+    const int64_t nslot = (cols + W - 1) / W;
+    const int64_t slot0 = static_cast<int64_t>(blockIdx.x) * TW;
+    const bool active = slot0 + t < nslot;
+    const int64_t slot = active ? slot0 + t : nslot - 1;
+    const int64_t col = view_col<W>(slot, cols);
+    const int dup = static_cast<int>(slot * W - col);
+    for (int64_t o = blockIdx.y; o < groups; o += gridDim.y) {
+        const int64_t base = o * group * cols + col;
+        float ov[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) ov[e] = 0.0f;
+        if (dfull) S::unpack(load16_any<S>(other + o * cols + col), ov);
+        double acc[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) acc[e] = 0.0;
+        u32x4 gv[BATCH], fv[BATCH];
+        auto load = [&](int u, int64_t r) {
+            gv[u] = load16_any_stream<S>(gy + base + r * cols);
+            fv[u] = load16_any_stream<S>(full + base + r * cols);
+        };
+        auto use = [&](int u, int64_t r) {
+            float a[W], b[W];
+            S::unpack(gv[u], a);
+            S::unpack(fv[u], b);
+#pragma unroll
+            for (int e = 0; e < W; ++e)
+                acc[e] += static_cast<double>(a[e]) * static_cast<double>(b[e]);
+            if (dfull && active) {
+#pragma unroll
+                for (int e = 0; e < W; ++e) a[e] = a[e] * ov[e];
+                view_store<S>(dfull + base + r * cols, a, dup, acc_full);
+            }
+        };
+        int64_t r = g;
+        if constexpr (LANES <= 256) {  // whole batches (1024 lanes have no registers for both)
+            for (; r + (BATCH - 1) * RG < group; r += BATCH * RG) {
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u) load(u, r + u * RG);
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u) use(u, r + u * RG);
+            }
+        }
+        for (; r < group; r += BATCH * RG) {  // partial batches: loads stay in the group
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+                load(u, r + u * RG < group ? r + u * RG : group - 1);
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+                if (r + u * RG < group) use(u, r + u * RG);
+        }
+        auto put = [&](int64_t at, double sum) {  // column `at` of this group
+            float* d = dother + o * cols + at;
+            *d = static_cast<float>((acc_other ? static_cast<double>(*d) : 0.0) + sum);
+        };
+        if constexpr (RG == 1) {
+#pragma unroll
+            for (int e = 0; e < W; ++e)
+                if (active && e >= dup) put(col + e, acc[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < W; ++e) part[g][t * W + e] = acc[e];
+            __syncthreads();
+            for (int c = threadIdx.x; c < TW * W; c += LANES) {
+                const int64_t sl = slot0 + c / W;
+                if (sl >= nslot) break;
+                const int64_t c0 = view_col<W>(sl, cols);
+                double sum = part[0][c];
+#pragma unroll 8
+                for (int q = 1; q < RG; ++q) sum += part[q][c];
+                if (c % W >= sl * W - c0) put(c0 + c % W, sum);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Both gradients of full * (a scalar per row): dfull (+)= gy * other[row]
+// (nullptr: not wanted), dother[row] (+)= the row's sum of gy * full, exact products
+// in fp64.  TPR lanes (one wave at most) per row; lane sums meet in a fixed
+// butterfly.  HBM-bound at gy + full + dfull.
+template <class S, int TPR>
+__global__ __launch_bounds__(kBcastBlock) void bcast_row_grad_kernel(
+    const typename S::T* __restrict__ gy, const typename S::T* __restrict__ full,
+    const typename S::T* __restrict__ other, typename S::T* __restrict__ dfull,
+    float* __restrict__ dother, int64_t rows, int64_t cols, int acc_full, int acc_other) {
+    constexpr int W = S::kVec, NV = kViewSlots, RPB = kBcastBlock / TPR;
+    const int t = threadIdx.x % TPR;
+    const int64_t nslot = (cols + W - 1) / W;
+    for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * RPB; r0 < rows;
+         r0 += static_cast<int64_t>(gridDim.x) * RPB) {
+        const bool active = r0 + threadIdx.x / TPR < rows;
+        const int64_t row = active ? r0 + threadIdx.x / TPR : rows - 1;
+        const float ov = dfull ? S::get(other + row) : 0.0f;
+        double acc[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) acc[e] = 0.0;
+        for (int64_t s0 = t; s0 < nslot; s0 += TPR * NV) {
+            u32x4 gv[NV], fv[NV];
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int64_t s = s0 + k * TPR < nslot ? s0 + k * TPR : nslot - 1;
+                gv[k] = load16_any_stream<S>(gy + row * cols + view_col<W>(s, cols));
+                fv[k] = load16_any_stream<S>(full + row * cols + view_col<W>(s, cols));
+            }
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                if (s0 + k * TPR >= nslot) break;
+                const int64_t col = view_col<W>(s0 + k * TPR, cols);
+                const int dup = static_cast<int>((s0 + k * TPR) * W - col);
+                float a[W], b[W];
+                S::unpack(gv[k], a);
+                S::unpack(fv[k], b);
+#pragma unroll
+                for (int e = 0; e < W; ++e) {
+                    const double p = static_cast<double>(a[e]) * static_cast<double>(b[e]);
+                    acc[e] = e < dup ? acc[e] : acc[e] + p;
+                }
+                if (dfull && active) {
+#pragma unroll
+                    for (int e = 0; e < W; ++e) a[e] = a[e] * ov;
+                    view_store<S>(dfull + row * cols + col, a, dup, acc_full);
+                }
+            }
+        }
+        double s = acc[0];
+#pragma unroll
+        for (int e = 1; e < W; ++e) s += acc[e];
+#pragma unroll
+        for (int m = TPR / 2; m > 0; m /= 2) s += __shfl_xor(s, m, 64);
+        if (active && t == 0)
+            dother[row] =
+                static_cast<float>((acc_other ? static_cast<double>(dother[row]) : 0.0) + s);
+    }
+}
+
 // Zeros n 16-bit words (a kernel rather than a memset node, so that the call
 // can be captured into a graph).
 __global__ __launch_bounds__(kBcastBlock) void bcast_zero_kernel(uint16_t* __restrict__ p,
@@ -358,6 +604,118 @@ inline BcastGeom make_geom(int nd, const int64_t* osize, const Aligned& a, const
         g.sa[0] = g.sb[0] = 0;
     }
     return g;
+}
+
+// The rows x cols view of a product of a full operand and a broadcast one; kind
+// 0: none applies.
+struct RowsView {
+    enum Kind { kNone = 0, kGroup = 1, kScalar = 2 };
+    int kind = kNone;
+    int64_t rows = 0, cols = 0, group = 1;
+};
+
+// g: make_geom's axes with the full operand first (its strides are the output's).
+inline RowsView rows_view(const BcastGeom& g, int w) {
+    RowsView v;
+    const int last = g.nd - 1;
+    if (g.nd == 2 && g.sb[0] == 0 && g.sb[1] == 1)
+        v = {RowsView::kGroup, g.size[0], g.size[1], g.size[0]};
+    else if (g.nd == 3 && g.sb[0] == g.size[2] && g.sb[1] == 0 && g.sb[2] == 1)
+        v = {RowsView::kGroup, g.size[0] * g.size[1], g.size[2], g.size[1]};
+    else if (g.nd == 2 && g.sb[0] == 1 && g.sb[1] == 0)
+        v = {RowsView::kScalar, g.size[0], g.size[1], 1};
+    else if (g.nd == 1 && g.sb[0] == 0)
+        v = {RowsView::kScalar, 1, g.size[0], 1};
+    if (v.cols < w || g.sa[last] != 1) v.kind = RowsView::kNone;
+    return v;
+}
+
+inline int64_t view_elems(const RowsView& v) { return v.rows * v.cols; }
+
+// Whether the one-pass gradient kernels take the view: long single rows spread
+// better over bcast_reduce_kernel's workgroups.
+inline bool grad_view_fits(const RowsView& v) {
+    if (v.kind == RowsView::kScalar) return v.cols <= 16384 || v.rows >= 1024;
+    return v.kind == RowsView::kGroup;
+}
+
+template <class S>
+int launch_rows_mul(const void* full, const void* other, void* y, const RowsView& v,
+                    int accumulate, hipStream_t st) {
+    using T = typename S::T;
+    const int64_t nslot = row_slots(v.cols, S::kVec);
+    const int64_t need = (nslot + kViewSlots - 1) / kViewSlots;
+    const int tpr = need <= 16 ? 16 : need <= 64 ? 64 : need <= 128 ? 128 : 256;
+    const int64_t bx = (v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr);
+    const int64_t by = (nslot + tpr * kViewSlots - 1) / (tpr * kViewSlots);
+    const dim3 grid(static_cast<unsigned>(bx < 0x7fffffffLL ? bx : 0x7fffffffLL),
+                    static_cast<unsigned>(by < 65535 ? by : 65535));
+#define AGK_ROWS_MUL(TPR)                                                                         \
+    do {                                                                                          \
+        if (v.kind == RowsView::kScalar)                                                          \
+            hipLaunchKernelGGL((bcast_rows_mul_kernel<S, TPR, true>), grid, dim3(kBcastBlock), 0, \
+                               st, static_cast<const T*>(full), static_cast<const T*>(other),     \
+                               static_cast<T*>(y), v.rows, v.cols, v.group, accumulate);          \
+        else                                                                                      \
+            hipLaunchKernelGGL((bcast_rows_mul_kernel<S, TPR, false>), grid, dim3(kBcastBlock),   \
+                               0, st, static_cast<const T*>(full), static_cast<const T*>(other),  \
+                               static_cast<T*>(y), v.rows, v.cols, v.group, accumulate);          \
+    } while (0)
+    if (tpr == 16) AGK_ROWS_MUL(16);
+    else if (tpr == 64) AGK_ROWS_MUL(64);
+    else if (tpr == 128) AGK_ROWS_MUL(128);
+    else AGK_ROWS_MUL(256);
+#undef AGK_ROWS_MUL
+    return check_launch();
+}
+
+// The gradient of the broadcast operand, with dfull (nullptr: not wanted) in the
+// same pass.
+template <class S>
+int launch_rows_grad(const void* gy, const void* full, const void* other, void* dfull,
+                     float* dother, const RowsView& v, int acc_full, int acc_other,
+                     hipStream_t st) {
+    using T = typename S::T;
+    const T *g = static_cast<const T*>(gy), *f = static_cast<const T*>(full),
+            *o = static_cast<const T*>(other);
+    T* df = static_cast<T*>(dfull);
+    const int64_t nslot = row_slots(v.cols, S::kVec);
+    if (v.kind == RowsView::kScalar) {
+        const int tpr = nslot <= 32 ? 16 : 64;
+        const int64_t bx = (v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr);
+        const dim3 grid(static_cast<unsigned>(bx < 0x7fffffffLL ? bx : 0x7fffffffLL));
+        if (tpr == 16)
+            hipLaunchKernelGGL((bcast_row_grad_kernel<S, 16>), grid, dim3(kBcastBlock), 0, st, g, f,
+                               o, df, dother, v.rows, v.cols, acc_full, acc_other);
+        else
+            hipLaunchKernelGGL((bcast_row_grad_kernel<S, 64>), grid, dim3(kBcastBlock), 0, st, g, f,
+                               o, df, dother, v.rows, v.cols, acc_full, acc_other);
+        return check_launch();
+    }
+    const int64_t groups = v.rows / v.group;
+    // One row lane for short groups; else whole kilobytes per row (four row
+    // lanes), or narrower tiles of 64 or 256 row lanes where those would leave CUs
+    // without a workgroup and the group has the rows.  Measured on MI355X, both
+    // gradients (us, 4- / 16- / 64-slot tiles): f32 8 x 2048 x 1024 86 / 50 / -, bf16
+    // 42 / 51 / -; f32 2 x 2048 x 4001 126 / 71 / -; bf16 20 groups' rows of 117520
+    // - / 32 / 16; f32 2 x 2048 x 64 15 / 28 / - (the two passes this replaces: 76,
+    // 73, 130, 15, 32).
+    auto tiles = [&](int64_t tw) { return (nslot + tw - 1) / tw; };
+    int tw = v.group <= 8 ? 256 : 64;
+    if (v.group >= 128 && tiles(64) * groups < 256)
+        tw = v.group >= 512 && tiles(16) * groups < 100 ? 4 : 16;
+    if (tiles(tw) > 0x7fffffffLL) return AGK_EINVAL;
+    const dim3 grid(static_cast<unsigned>(tiles(tw)),
+                    static_cast<unsigned>(groups < 65535 ? groups : 65535));
+#define AGK_GROUP_GRAD(TW, LANES, BATCH)                                                         \
+    hipLaunchKernelGGL((bcast_group_grad_kernel<S, TW, LANES, BATCH>), grid, dim3(LANES), 0, st, \
+                       g, f, o, df, dother, groups, v.group, v.cols, acc_full, acc_other)
+    if (tw == 256) AGK_GROUP_GRAD(256, 256, 8);
+    else if (tw == 64) AGK_GROUP_GRAD(64, 256, 8);
+    else if (tw == 16) AGK_GROUP_GRAD(16, 1024, 4);
+    else AGK_GROUP_GRAD(4, 1024, 4);
+#undef AGK_GROUP_GRAD
+    return check_launch();
 }
 
 template <class S>
@@ -452,12 +810,34 @@ inline bool is_full(int nd, const int64_t* osize, const Aligned& t) {
     return true;
 }
 
+// The rows x cols view of a * b written to y (or of a gradient gy * other): which
+// operand is full and which broadcast; none when y overlaps one of them (a slot
+// moved back to the row's end may be stored before its neighbour is loaded).
+inline RowsView product_view(int nd, const int64_t* osize, const Aligned& al, const Aligned& bl,
+                             const void* a, const void* b, const void* y, int dtype,
+                             const void** full, const void** other) {
+    const bool af = is_full(nd, osize, al), bf = is_full(nd, osize, bl);
+    if (af == bf) return RowsView{};
+    const int w = dtype == AGK_F32 ? F32::kVec : BF16::kVec;
+    const RowsView v = rows_view(af ? make_geom(nd, osize, al, bl) : make_geom(nd, osize, bl, al), w);
+    *full = af ? a : b;
+    *other = af ? b : a;
+    const int64_t bytes = view_elems(v) * (16 / w);
+    if (v.kind != RowsView::kNone && (!disjoint(y, *full, bytes) || !disjoint(y, *other, bytes)))
+        return RowsView{};
+    return v;
+}
+
 template <class S>
 int bcast_bwd_one(const void* gy, const void* other, const Aligned& t, const Aligned& o,
                   const Aligned& gyal, int nd, const int64_t* osize, void* d, int accumulate,
                   hipStream_t st) {
     if (is_full(nd, osize, t)) {
-        // d (+)= gy * other: the forward kernel with gy as the full operand
+        // d (+)= gy * other: the forward kernels with gy as the full operand
+        const void *full = nullptr, *bc = nullptr;
+        const int dtype = S::kVec == 4 ? AGK_F32 : AGK_BF16;
+        const RowsView v = product_view(nd, osize, gyal, o, gy, other, d, dtype, &full, &bc);
+        if (v.kind != RowsView::kNone) return launch_rows_mul<S>(full, bc, d, v, accumulate, st);
         const BcastGeom g = make_geom(nd, osize, gyal, o);
         return launch_bcast_mul<S>(gy, other, d, g, accumulate, st);
     }
@@ -530,9 +910,14 @@ extern "C" int agk_mul_bcast_fwd(const void* a, const int64_t* a_shape, int a_nd
     if (numel == 0) return AGK_OK;
     if (!a || !b || !y) return AGK_EINVAL;
     clear_pending_error();
-    const BcastGeom g = make_geom(nd, osize, al, bl);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const int acc = accumulate != 0;
+    const void *full = nullptr, *other = nullptr;
+    const RowsView v = product_view(nd, osize, al, bl, a, b, y, dtype, &full, &other);
+    if (v.kind != RowsView::kNone)
+        return dtype == AGK_F32 ? launch_rows_mul<F32>(full, other, y, v, acc, st)
+                                : launch_rows_mul<BF16>(full, other, y, v, acc, st);
+    const BcastGeom g = make_geom(nd, osize, al, bl);
     return dtype == AGK_F32 ? launch_bcast_mul<F32>(a, b, y, g, acc, st)
                             : launch_bcast_mul<BF16>(a, b, y, g, acc, st);
 }
@@ -579,6 +964,25 @@ extern "C" int agk_mul_bcast_bwd(const void* gy, const void* a, const int64_t* a
     Aligned gyal;  // gy in the output layout
     if (!align_operand(osize, nd, nd, gyal)) return AGK_EINVAL;
     int rc = AGK_OK;
+    // One operand full and the other a vector per group of rows or a scalar per
+    // row: the broadcast operand's gradient and the full one's in one pass.
+    {
+        const bool a_full = is_full(nd, osize, al);
+        void* dfull = a_full ? da : db;
+        void* dother = a_full ? db : da;
+        const int acc_full = (accumulate & (a_full ? AGK_ACCUM_DX : AGK_ACCUM_DGAMMA)) != 0;
+        const int acc_other = (accumulate & (a_full ? AGK_ACCUM_DGAMMA : AGK_ACCUM_DX)) != 0;
+        const void *full = nullptr, *other = nullptr;
+        const RowsView v = product_view(nd, osize, al, bl, a, b, dfull, dtype, &full, &other);
+        const int64_t bytes = view_elems(v) * (dtype == AGK_F32 ? 4 : 2);
+        if (dother && grad_view_fits(v) && disjoint(dfull, gy, bytes))
+            return dtype == AGK_F32
+                       ? launch_rows_grad<F32>(gy, full, other, dfull, static_cast<float*>(dother),
+                                               v, acc_full, acc_other, st)
+                       : launch_rows_grad<BF16>(gy, full, other, dfull,
+                                                static_cast<float*>(dother), v, acc_full,
+                                                acc_other, st);
+    }
     if (da) {
         const int acc = (accumulate & AGK_ACCUM_DX) != 0;
         rc = dtype == AGK_F32 ? bcast_bwd_one<F32>(gy, b, al, bl, gyal, nd, osize, da, acc, st)

@@ -184,3 +184,61 @@ def test_row_vector_cases_agree_with_the_row_kernels(cuda):
     g1, g2 = to_host(db1).astype(np.float64), to_host(db2).astype(np.float64)
     assert np.all(np.abs(g1 - r) <= REL * np.abs(r) + 1e-30)
     assert np.max(np.abs(g2 - r)) <= TOL_F32 * np.max(np.abs(r))
+
+
+# rows x cols views: a vector per group of rows (one, few and many rows; one batch, a
+# remainder, both), a scalar per row, and shapes just outside them
+VIEW_SHAPES = [((5, 37, 61), (5, 1, 61)), ((3, 9, 8), (3, 1, 8)), ((2, 300, 129), (300, 129)),
+               ((300, 17), (1, 17)), ((3, 1000, 1031), (3, 1, 1031)), ((2, 64, 4096), (2, 1, 4096)),
+               ((33, 2051), (1, 2051)), ((7, 33, 5), (7, 33, 1)), ((4100, 40), (4100, 1)),
+               ((2, 3, 20001), (2, 3, 1)), ((1500, 300), (1500, 1)), ((1030,), (1,)),
+               ((40, 3), (40, 1)), ((2, 3, 4, 32), (2, 1, 4, 32)), ((70000, 9), (70000, 1))]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shapes", VIEW_SHAPES, ids=str)
+@pytest.mark.parametrize("swap", [False, True])
+def test_row_views_match_torch(cuda, dtype, shapes, swap):
+    """Products and full gradients: torch's element-wise product, bit for bit; sums: fp64 sums of
+    exact products rounded once (2^-24 relative, plus fp64 rounding of the terms' magnitude);
+    one operand's gradient alone and accumulation."""
+    import torch
+    dt = torch.float32 if dtype == "f32" else torch.bfloat16
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(sum(shapes[0]))
+    a = torch.randn(*shapes[0], generator=gen, device=cuda).to(dt)
+    b = torch.randn(*shapes[1], generator=gen, device=cuda).to(dt)
+    if swap:
+        a, b = b, a
+    want = a * b
+    gy = torch.randn(want.shape, generator=gen, device=cuda).to(dt)
+    full, vec = (b, a) if swap else (a, b)
+    y = agk.mul_bcast_fwd(a, b)
+    assert torch.equal(y, want)
+    da, db = agk.mul_bcast_bwd(gy, a, b)
+    d_full, d_vec = (db, da) if swap else (da, db)
+    assert torch.equal(d_full, gy * vec)
+    axes = [i for i in range(want.dim())
+            if i < want.dim() - vec.dim() or vec.shape[i - want.dim() + vec.dim()] != want.shape[i]]
+    terms = gy.double() * full.double()
+    ref = terms.sum(axes, keepdim=True).reshape(vec.shape)
+    mag = terms.abs().sum(axes, keepdim=True).reshape(vec.shape)
+    assert ((d_vec.double() - ref).abs() <= 2.0 ** -24 * ref.abs() + 1e-13 * mag).all().item()
+    # each gradient alone, and added to what is there
+    only_a, _ = agk.mul_bcast_bwd(gy, a, b, want_db=False)
+    _, only_b = agk.mul_bcast_bwd(gy, a, b, want_da=False)
+    assert torch.equal(only_a, da) and torch.equal(only_b, db)
+    pre_a, pre_b = torch.full_like(da, 0.5), torch.full_like(db, 0.5)
+    acc_a, acc_b = agk.mul_bcast_bwd(gy, a, b, da=pre_a.clone(), db=pre_b.clone(),
+                                     accumulate=agk.AGK_ACCUM_ALL)
+    torch.cuda.synchronize()
+    acc_full, acc_vec = (acc_b, acc_a) if swap else (acc_a, acc_b)
+    assert torch.equal(acc_full, 0.5 + d_full)
+    assert ((acc_vec.double() - (0.5 + ref)).abs()
+            <= 2.0 ** -24 * (0.5 + ref).abs() + 1e-13 * mag).all().item()
+    # an output over an operand: the same product
+    in_place = full.clone()
+    args = (a, in_place) if swap else (in_place, b)
+    agk.mul_bcast_fwd(*args, y=in_place)
+    torch.cuda.synchronize()
+    assert torch.equal(in_place, want)
