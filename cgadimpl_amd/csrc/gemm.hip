@@ -470,13 +470,30 @@ __device__ __forceinline__ void direct_step(const DirectStage& d, const uint16_t
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Stores columns [64 H, 64 H + 64) of a wave's 128 x 128 block, whose first column
+// is col0 of C.  H is a template argument, not a loop's: a loop over the halves is
+// too large for the compiler to unroll, and acc, indexed by a variable, moves to
+// scratch memory.
+template <bool OUT_F32, Stores S, int H>
+__device__ __forceinline__ void store_half(const f32x16 (&acc)[TM][2 * TN], void* __restrict__ C,
+                                           int64_t ldc, int M, int N, int row0, int col0,
+                                           int lane, const float* __restrict__ rowscale,
+                                           const uint16_t* __restrict__ colbias, int accumulate) {
+    f32x16 part[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) part[i][j] = acc[i][H * TN + j];
+    store_block<OUT_F32, S>(part, C, ldc, M, N, row0, col0, lane, rowscale, colbias, accumulate);
+}
+
 // One tile's k loop and store.  NB = 4: the 256 x 256 tile at (m0, n0), wave
 // (wm, wn) owning its 128 x 128 block; NB = 2: the 256 x 128 half of that tile
 // starting at column n0 + half_off, wave (wm, wn) owning a 128 x 64 block.
 // Both stage the tile's full 256 B columns (the same loads).  TAIL: K is not a
 // multiple of 64; the last K % 64 k are multiplied first, staged through
 // registers into st1 (which tile 1's loads fill only after it).
-template <bool OUT_F32, bool A_TR, bool B_TR, int NB, bool TAIL>
+template <bool OUT_F32, bool A_TR, bool B_TR, int NB, bool TAIL, Stores S>
 __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0, uint16_t* st1,
                                             const uint16_t* __restrict__ a0, int64_t lda,
                                             int rows_a, const uint16_t* __restrict__ b0,
@@ -532,19 +549,13 @@ __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0,
 
     if constexpr (NB == 4) {
         // the wave's 128 x 128 block leaves as two 128 x 64 halves
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            f32x16 part[TM][TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) part[i][j] = acc[i][h * TN + j];
-            store_block<OUT_F32>(part, C, ldc, M, N, m0 + wm * WM, n0 + (2 * wn + h) * WN, lane,
-                                 rowscale, colbias, accumulate);
-        }
+        store_half<OUT_F32, S, 0>(acc, C, ldc, M, N, m0 + wm * WM, n0 + 2 * wn * WN, lane, rowscale,
+                               colbias, accumulate);
+        store_half<OUT_F32, S, 1>(acc, C, ldc, M, N, m0 + wm * WM, n0 + (2 * wn + 1) * WN, lane,
+                               rowscale, colbias, accumulate);
     } else {
-        store_block<OUT_F32>(acc, C, ldc, M, N, m0 + wm * WM, n0 + half_off + wn * WN, lane,
-                             rowscale, colbias, accumulate);
+        store_block<OUT_F32, S>(acc, C, ldc, M, N, m0 + wm * WM, n0 + half_off + wn * WN, lane,
+                                rowscale, colbias, accumulate);
     }
 }
 
@@ -555,7 +566,7 @@ __device__ __forceinline__ void direct_tile(const DirectStage& d, uint16_t* st0,
 // (workgroup full_tiles + 2 h + q: half q of tile full_tiles + h), so that a
 // last round of few tiles runs on twice as many CUs for half as long.  Every
 // output element is summed in the same k order either way (bit-identical).
-template <bool OUT_F32, bool A_TR, bool B_TR, bool TAIL>
+template <bool OUT_F32, bool A_TR, bool B_TR, bool TAIL, Stores S>
 __global__ __launch_bounds__(kDirectThreads) void gemm_nt_direct_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
     void* __restrict__ C, int64_t ldc, int M, int N, int K, const float* __restrict__ rowscale,
@@ -599,11 +610,11 @@ __global__ __launch_bounds__(kDirectThreads) void gemm_nt_direct_kernel(
     direct_offsets<B_TR>(d.ob, wave, lane, rows_b, ldb);
 
     if (!halves)
-        direct_tile<OUT_F32, A_TR, B_TR, 4, TAIL>(d, st0, st1, a0, lda, rows_a, b0, ldb, rows_b,
+        direct_tile<OUT_F32, A_TR, B_TR, 4, TAIL, S>(d, st0, st1, a0, lda, rows_a, b0, ldb, rows_b,
                                                   C, ldc, M, N, K, m0, n0, 0, wm, wn, lane, wave,
                                                   rowscale, colbias, accumulate);
     else
-        direct_tile<OUT_F32, A_TR, B_TR, 2, TAIL>(d, st0, st1, a0, lda, rows_a, b0, ldb, rows_b,
+        direct_tile<OUT_F32, A_TR, B_TR, 2, TAIL, S>(d, st0, st1, a0, lda, rows_a, b0, ldb, rows_b,
                                                   C, ldc, M, N, K, m0, n0,
                                                   ((L - full_tiles) & 1) * (BN / 2), wm, wn,
                                                   lane, wave, rowscale, colbias, accumulate);
@@ -785,17 +796,24 @@ int launch_direct(bool f32, const GemmCall& c) {
     const int tiles = tiles_m * tiles_n;
     const int full = direct_full_tiles(tiles, device_cus());
     const dim3 grid(full + 2 * (tiles - full)), block(kDirectThreads);
-#define AGK_DIRECT(F32, TAIL)                                                                  \
-    hipLaunchKernelGGL((gemm_nt_direct_kernel<F32, A_TR, B_TR, TAIL>), grid, block, 0, c.st,   \
-                       c.A, c.lda, c.B, c.ldb, c.C, c.ldc, c.M, c.N, c.K, c.rowscale,          \
+#define AGK_DIRECT(F32, TAIL, S)                                                               \
+    hipLaunchKernelGGL((gemm_nt_direct_kernel<F32, A_TR, B_TR, TAIL, Stores::S>), grid, block, \
+                       0, c.st, c.A, c.lda, c.B, c.ldb, c.C, c.ldc, c.M, c.N, c.K, c.rowscale, \
                        c.colbias, c.accumulate, tiles_m, tiles_n, gm, full)
     const bool tail = c.K % BK != 0;
+    if constexpr (!A_TR && !B_TR) {  // the layout of agk_linear_bf16
+        if (!f32 && c.colbias != nullptr && c.rowscale == nullptr && !c.accumulate) {
+            if (tail) AGK_DIRECT(false, true, kBiasOnly);
+            else AGK_DIRECT(false, false, kBiasOnly);
+            return hipGetLastError() == hipSuccess ? AGK_OK : AGK_EHIP;
+        }
+    }
     if (f32) {
-        if (tail) AGK_DIRECT(true, true);
-        else AGK_DIRECT(true, false);
+        if (tail) AGK_DIRECT(true, true, kNoBias);
+        else AGK_DIRECT(true, false, kNoBias);
     } else {
-        if (tail) AGK_DIRECT(false, true);
-        else AGK_DIRECT(false, false);
+        if (tail) AGK_DIRECT(false, true, kNoBias);
+        else AGK_DIRECT(false, false, kNoBias);
     }
 #undef AGK_DIRECT
     return hipGetLastError() == hipSuccess ? AGK_OK : AGK_EHIP;

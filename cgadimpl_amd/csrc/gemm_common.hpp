@@ -1,5 +1,4 @@
-// gemm_common.hpp -- what the bf16 product kernels (gemm.hip, gemm_ring.hpp,
-// gemm_skinny.hip) share: types and conversions, the LDS layouts of staged
+// gemm_common.hpp -- what the bf16 product kernels (gemm.hip, gemm_ring.hpp) share: types and conversions, the LDS layouts of staged
 // operands, the order of the tiles over the XCDs, the epilogue and the
 // description of one product.
 #pragma once
@@ -151,11 +150,18 @@ __device__ __forceinline__ float with_bias(float v, uint16_t b) {
     return v + __uint_as_float(static_cast<uint32_t>(b) << 16);
 }
 
-// GENERAL: rowscale, a column bias (bf16 output only) and accumulate
-// honoured; CHECK: rows past M and columns past N skipped.  store_block picks the
-// variant once per call (uniform values), so the common plain, interior store
-// has no per-element branches.
-template <bool OUT_F32, bool GENERAL, bool CHECK, int TMW, int TNW>
+// What a store applies to the product: nothing, a column bias (bf16 output
+// only), or any of rowscale, bias and accumulate, tested per element.
+enum class Epi { kPlain, kBias, kAny };
+
+// CHECK: rows past M and columns past N skipped.  store_block picks the variant
+// once per call (uniform values), so the plain and the biased interior stores
+// have no per-element branches.  kBias loads the lane's TNW bias values once; in
+// kAny each element waits for a load of its own, up to 256 in a row, which is
+// what bounded a biased product.  y = x w^T + b, kAny -> kBias: 1032 x 4096 x 4096
+// 62.7 -> 42.4 us, 3288 x 3568 x 136 75 -> 21.6, 2480 x 2064 x 1152 34.4 -> 25.3,
+// 3000 x 800 x 2624 32 -> 25.3; the same bits.
+template <bool OUT_F32, Epi EPI, bool CHECK, int TMW, int TNW>
 __device__ __forceinline__ void store_c_impl(const f32x16 (&acc)[TMW][TNW], void* __restrict__ C,
                                              int64_t ldc, int M, int N, int row0, int col0,
                                              int lane, const float* __restrict__ rowscale,
@@ -163,6 +169,14 @@ __device__ __forceinline__ void store_c_impl(const f32x16 (&acc)[TMW][TNW], void
                                              int accumulate) {
     const int col_l = lane & 31;
     const int row_l = 4 * (lane >> 5);
+    uint16_t bias[TNW] = {};
+    if constexpr (EPI == Epi::kBias) {
+#pragma unroll
+        for (int j = 0; j < TNW; ++j) {
+            const int col = col0 + j * 32 + col_l;
+            if (!CHECK || col < N) bias[j] = colbias[col];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < TMW; ++i) {
 #pragma unroll
@@ -170,20 +184,20 @@ __device__ __forceinline__ void store_c_impl(const f32x16 (&acc)[TMW][TNW], void
             const int row = row0 + i * 32 + 8 * (e >> 2) + row_l + (e & 3);
             if (CHECK && row >= M) continue;
             float rs = 1.0f;
-            if constexpr (GENERAL) rs = rowscale ? rowscale[row] : 1.0f;
+            if constexpr (EPI == Epi::kAny) rs = rowscale ? rowscale[row] : 1.0f;
 #pragma unroll
             for (int j = 0; j < TNW; ++j) {
                 const int col = col0 + j * 32 + col_l;
                 if (CHECK && col >= N) continue;
                 float v = acc[i][j][e];
-                if constexpr (GENERAL) {
+                if constexpr (EPI == Epi::kAny) {
                     v *= rs;
                     // accumulation rounds the product first (no fused multiply-add)
                     asm volatile("" : "+v"(v));
                 }
                 if constexpr (OUT_F32) {
                     float* p = static_cast<float*>(C) + static_cast<int64_t>(row) * ldc + col;
-                    if constexpr (GENERAL) {
+                    if constexpr (EPI == Epi::kAny) {
                         *p = accumulate ? *p + v : v;
                     } else {
                         // Plain fp32 stores are whole 128-byte lines per 32 lanes:
@@ -197,9 +211,11 @@ __device__ __forceinline__ void store_c_impl(const f32x16 (&acc)[TMW][TNW], void
                     }
                 } else {
                     uint16_t* p = static_cast<uint16_t*>(C) + static_cast<int64_t>(row) * ldc + col;
-                    if constexpr (GENERAL) {
+                    if constexpr (EPI == Epi::kAny) {
                         if (accumulate) v = __uint_as_float(static_cast<uint32_t>(*p) << 16) + v;
                         if (colbias) v = with_bias(v, colbias[col]);
+                    } else if constexpr (EPI == Epi::kBias) {
+                        v = with_bias(v, bias[j]);
                     }
                     *p = static_cast<uint16_t>(f32_to_bf16_bits(v));
                 }
@@ -208,23 +224,46 @@ __device__ __forceinline__ void store_c_impl(const f32x16 (&acc)[TMW][TNW], void
     }
 }
 
+// The stores a kernel holds.  kBiasOnly: a bias, nothing else.  kNoBias: the plain
+// ones, and kAny for the rest (a bias too).  kAll: kNoBias with the biased ones.
+// The 256 x 256 kernel, whose unrolled stores are four times the others', is built
+// as kNoBias and as kBiasOnly: holding all of them in one kernel costs its plain
+// product 0.7 % in a training pass, where each kernel's code is fetched afresh
+// (8192 x 11008 x 4096: 600 -> 604 us; equal when it repeats alone).
+enum class Stores { kAll, kNoBias, kBiasOnly };
+
 // Stores a wave's block of TMW x TNW accumulators whose first element is
 // C[row0][col0]; which variant runs is uniform over the wave.
-template <bool OUT_F32, int TMW, int TNW>
+template <bool OUT_F32, Stores S, int TMW, int TNW>
 __device__ __forceinline__ void store_block(const f32x16 (&acc)[TMW][TNW], void* __restrict__ C,
                                             int64_t ldc, int M, int N, int row0, int col0,
                                             int lane, const float* __restrict__ rowscale,
                                             const uint16_t* __restrict__ colbias,
                                             int accumulate) {
-    if (rowscale != nullptr || colbias != nullptr || accumulate) {
-        store_c_impl<OUT_F32, true, true>(acc, C, ldc, M, N, row0, col0, lane, rowscale, colbias,
-                                          accumulate);
-    } else if (row0 + TMW * 32 <= M && col0 + TNW * 32 <= N) {
-        store_c_impl<OUT_F32, false, false>(acc, C, ldc, M, N, row0, col0, lane, nullptr, nullptr,
-                                            0);
-    } else {
-        store_c_impl<OUT_F32, false, true>(acc, C, ldc, M, N, row0, col0, lane, nullptr, nullptr,
-                                           0);
+    const bool inner = row0 + TMW * 32 <= M && col0 + TNW * 32 <= N;
+    const bool scaled = rowscale != nullptr || accumulate;
+    if constexpr (!OUT_F32 && S != Stores::kNoBias) {
+        if (S == Stores::kBiasOnly || (!scaled && colbias != nullptr)) {
+            if (inner)
+                store_c_impl<OUT_F32, Epi::kBias, false>(acc, C, ldc, M, N, row0, col0, lane,
+                                                         nullptr, colbias, 0);
+            else
+                store_c_impl<OUT_F32, Epi::kBias, true>(acc, C, ldc, M, N, row0, col0, lane,
+                                                        nullptr, colbias, 0);
+            return;
+        }
+    }
+    if constexpr (S != Stores::kBiasOnly) {
+        if (scaled || colbias != nullptr) {
+            store_c_impl<OUT_F32, Epi::kAny, true>(acc, C, ldc, M, N, row0, col0, lane, rowscale,
+                                                   colbias, accumulate);
+        } else if (inner) {
+            store_c_impl<OUT_F32, Epi::kPlain, false>(acc, C, ldc, M, N, row0, col0, lane,
+                                                      nullptr, nullptr, 0);
+        } else {
+            store_c_impl<OUT_F32, Epi::kPlain, true>(acc, C, ldc, M, N, row0, col0, lane, nullptr,
+                                                     nullptr, 0);
+        }
     }
 }
 

@@ -355,9 +355,9 @@ __global__ __launch_bounds__(256, SH::kPerCu) void gemm_ring_kernel(
     }
     // the empty loads of the last steps still name this workgroup's LDS
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    store_block<OUT_F32, SH::kTm, SH::kTn>(acc, C, ldc, M, N, m0 + wm * SH::kTm * 32,
-                                           n0 + wn * SH::kTn * 32, lane, rowscale, colbias,
-                                           accumulate);
+    store_block<OUT_F32, Stores::kAll>(acc, C, ldc, M, N, m0 + wm * SH::kTm * 32,
+                                       n0 + wn * SH::kTn * 32, lane, rowscale, colbias,
+                                       accumulate);
 }
 
 template <bool A_TR, bool B_TR>

@@ -121,6 +121,25 @@ def test_gemm_tile_shapes(cuda, M, N, ta, tb):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N", SHAPE_CASES)
+def test_bias_store_per_tile_shape(cuda, M, N):
+    """The biased store of every tile shape, in whole tiles and in ragged last ones: the bits of
+    the plain product plus a bf16 add of the bias, nothing written past C."""
+    import torch
+    torch.manual_seed(M + N)
+    for K in (72, 200):
+        x = torch.randn(M, K, device=cuda).bfloat16()
+        w = torch.randn(N, K, device=cuda).bfloat16()
+        b = torch.randn(N, device=cuda).bfloat16()
+        room = torch.full((M + 1, N), 7.0, device=cuda, dtype=torch.bfloat16)
+        agk.linear_bf16(x, w, b, y=room[:M])
+        plain = agk.gemm_bf16(x, w, trans_b=True)
+        torch.cuda.synchronize()
+        assert torch.equal(room[:M], (plain.float() + b.float()).bfloat16()), (M, N, K)
+        assert (room[M] == 7.0).all().item(), (M, N, K)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols", [(8, 8), (128, 128), (136, 264), (4096, 11008), (1000, 8)])
 def test_transpose_bit_exact(cuda, rows, cols):
     import torch
