@@ -631,6 +631,9 @@ inline RowsView rows_view(const BcastGeom& g, int w) {
 }
 
 inline int64_t view_elems(const RowsView& v) { return v.rows * v.cols; }
+inline int64_t view_other_elems(const RowsView& v) {
+    return v.kind == RowsView::kScalar ? v.rows : v.rows / v.group * v.cols;
+}
 
 // Whether the one-pass gradient kernels take the view: long single rows spread
 // better over bcast_reduce_kernel's workgroups.
@@ -965,7 +968,10 @@ extern "C" int agk_mul_bcast_bwd(const void* gy, const void* a, const int64_t* a
     if (!align_operand(osize, nd, nd, gyal)) return AGK_EINVAL;
     int rc = AGK_OK;
     // One operand full and the other a vector per group of rows or a scalar per
-    // row: the broadcast operand's gradient and the full one's in one pass.
+    // row: the broadcast operand's gradient and the full one's in one pass.  Not
+    // where either gradient overlaps what the pass reads (or the other gradient): a
+    // workgroup may read an element that its neighbour has already overwritten.
+    // In two passes the first one has read everything before the second writes.
     {
         const bool a_full = is_full(nd, osize, al);
         void* dfull = a_full ? da : db;
@@ -975,7 +981,11 @@ extern "C" int agk_mul_bcast_bwd(const void* gy, const void* a, const int64_t* a
         const void *full = nullptr, *other = nullptr;
         const RowsView v = product_view(nd, osize, al, bl, a, b, dfull, dtype, &full, &other);
         const int64_t bytes = view_elems(v) * (dtype == AGK_F32 ? 4 : 2);
-        if (dother && grad_view_fits(v) && disjoint(dfull, gy, bytes))
+        const int64_t obytes = view_other_elems(v) * (dtype == AGK_F32 ? 4 : 2);
+        const int64_t dbytes = view_other_elems(v) * 4;  // a sum: fp32
+        if (dother && grad_view_fits(v) && disjoint(dfull, gy, bytes) &&
+            disjoint(dother, dbytes, gy, bytes) && disjoint(dother, dbytes, full, bytes) &&
+            disjoint(dother, dbytes, other, obytes) && disjoint(dother, dbytes, dfull, bytes))
             return dtype == AGK_F32
                        ? launch_rows_grad<F32>(gy, full, other, dfull, static_cast<float*>(dother),
                                                v, acc_full, acc_other, st)

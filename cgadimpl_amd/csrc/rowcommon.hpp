@@ -360,10 +360,13 @@ inline Plan fwd_plan(int64_t nslot, int64_t rows) {
     return pick_plan(kFwdShapes, nslot, rows > kLargeRows ? 2 : 4, 512, 8);
 }
 
-// Whether two tensors of `bytes` bytes share no byte (NULL: no tensor).
-inline bool disjoint(const void* a, const void* b, int64_t bytes) {
+// Whether two tensors share no byte (NULL: no tensor).
+inline bool disjoint(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
     const char *p = static_cast<const char*>(a), *q = static_cast<const char*>(b);
-    return !p || !q || p + bytes <= q || q + bytes <= p;
+    return !p || !q || p + a_bytes <= q || q + b_bytes <= p;
+}
+inline bool disjoint(const void* a, const void* b, int64_t bytes) {
+    return disjoint(a, bytes, b, bytes);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -242,3 +242,27 @@ def test_row_views_match_torch(cuda, dtype, shapes, swap):
     agk.mul_bcast_fwd(*args, y=in_place)
     torch.cuda.synchronize()
     assert torch.equal(in_place, want)
+
+
+@pytest.mark.parametrize("shape,vec", [((64, 1025), (1, 1025)), ((3, 40, 2051), (3, 1, 2051)),
+                                       ((700, 1025), (1, 1025)), ((5, 9, 130), (5, 9, 1))], ids=str)
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gradient_written_over_the_broadcast_operand(cuda, shape, vec, accumulate):
+    """db over b (fp32), at widths whose last 16-byte slot reaches back into the columns of the
+    slot before it: da is made of the b that the call was given, bit for bit, and db is the sum
+    (added to b where it accumulates), as two passes in order give them."""
+    import torch
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(shape[-1] + len(shape))
+    a, b, gy = (torch.randn(*s, generator=gen, device=cuda) for s in (shape, vec, shape))
+    over = b.clone()
+    da, db = agk.mul_bcast_bwd(gy, a, over, db=over, accumulate=agk.AGK_ACCUM_DGAMMA * accumulate)
+    torch.cuda.synchronize()
+    assert db.data_ptr() == over.data_ptr()
+    assert torch.equal(da, gy * b)
+    axes = [i for i in range(len(shape)) if vec[i] != shape[i]]
+    terms = gy.double() * a.double()
+    ref = terms.sum(axes, keepdim=True) + (b.double() if accumulate else 0.0)
+    # an fp64 sum of exact products, rounded once
+    mag = terms.abs().sum(axes, keepdim=True) + b.double().abs()
+    assert ((db.double() - ref).abs() <= 2.0 ** -24 * ref.abs() + 1e-13 * mag).all().item()
