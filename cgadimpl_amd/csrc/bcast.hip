@@ -825,8 +825,9 @@ inline RowsView product_view(int nd, const int64_t* osize, const Aligned& al, co
     const RowsView v = rows_view(af ? make_geom(nd, osize, al, bl) : make_geom(nd, osize, bl, al), w);
     *full = af ? a : b;
     *other = af ? b : a;
-    const int64_t bytes = view_elems(v) * (16 / w);
-    if (v.kind != RowsView::kNone && (!disjoint(y, *full, bytes) || !disjoint(y, *other, bytes)))
+    const int64_t es = 16 / w, bytes = view_elems(v) * es;
+    if (v.kind != RowsView::kNone && (!disjoint(y, *full, bytes) ||
+                                      !disjoint(y, bytes, *other, view_other_elems(v) * es)))
         return RowsView{};
     return v;
 }

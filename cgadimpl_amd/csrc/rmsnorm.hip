@@ -1245,7 +1245,7 @@ int launch_mul_fwd(const void* a, const void* b, void* y, int64_t rows, int cols
     // before the loads of the slot that overlaps it.
     const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(T));
     if (!vec && (rows >= kLargeRows || bytes >= (1LL << 28)) && disjoint(a, y, bytes) &&
-        disjoint(b, y, bytes))
+        disjoint(b, cols * static_cast<int64_t>(sizeof(T)), y, bytes))
         p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), rows, cols, S::kVec);
     if (p.tpr == 0) {
         if (rows > 0x7fffffffLL) return AGK_EINVAL;

@@ -266,3 +266,39 @@ def test_gradient_written_over_the_broadcast_operand(cuda, shape, vec, accumulat
     # an fp64 sum of exact products, rounded once
     mag = terms.abs().sum(axes, keepdim=True) + b.double().abs()
     assert ((db.double() - ref).abs() <= 2.0 ** -24 * ref.abs() + 1e-13 * mag).all().item()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shape,vec", [((4, 700, 96), (4, 1, 96)), ((300, 1025), (1, 1025)),
+                                       ((6, 50, 77), (6, 50, 1))], ids=str)
+def test_bits_do_not_depend_on_where_the_operands_lie(cuda, dtype, shape, vec):
+    """The broadcast operand right below y and da in one buffer, or far from them: the same
+    kernels, so the same bits in the product and both gradients."""
+    import math
+    import torch
+    dt = torch.float32 if dtype == "f32" else torch.bfloat16
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(shape[-1])
+    b = torch.randn(vec, generator=gen, device=cuda).to(dt)
+    # terms of many magnitudes that cancel along the summed axes: what is left of an fp64 sum is
+    # its rounding, which shows the order of the terms
+    a = torch.randn(shape, generator=gen, device=cuda)
+    a *= 2.0 ** torch.randint(-30, 31, shape, generator=gen, device=cuda)
+    axis = [i for i in range(len(shape)) if vec[i] != shape[i]][0]
+    a = (a - a.flip(axis)).to(dt)
+    gy = torch.ones_like(a)
+    n, m = math.prod(shape), math.prod(vec)
+    far = torch.empty(64 * n, device=cuda, dtype=dt)  # b, then 62 tensors of room, then y
+
+    def run(at):
+        bb, out = far[:m].view(vec), far[at:at + n].view(shape)
+        bb.copy_(b)
+        y = agk.mul_bcast_fwd(a, bb, y=out).clone()
+        da, db = agk.mul_bcast_bwd(gy, a, bb, da=out)
+        torch.cuda.synchronize()
+        return y, da.clone(), db.clone()
+
+    near, apart = run(m), run(62 * n)
+    for got, want in zip(near, apart):
+        assert torch.equal(got, want)
+    assert torch.equal(near[0], a * b) and torch.equal(near[1], gy * b)
