@@ -651,8 +651,7 @@ int launch_rows_mul(const void* full, const void* other, void* y, const RowsView
     const int tpr = need <= 16 ? 16 : need <= 64 ? 64 : need <= 128 ? 128 : 256;
     const int64_t bx = (v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr);
     const int64_t by = (nslot + tpr * kViewSlots - 1) / (tpr * kViewSlots);
-    const dim3 grid(static_cast<unsigned>(bx < 0x7fffffffLL ? bx : 0x7fffffffLL),
-                    static_cast<unsigned>(by < 65535 ? by : 65535));
+    const dim3 grid(capped_blocks(bx, kBcastBlock), static_cast<unsigned>(by < 65535 ? by : 65535));
 #define AGK_ROWS_MUL(TPR)                                                                         \
     do {                                                                                          \
         if (v.kind == RowsView::kScalar)                                                          \
@@ -686,7 +685,7 @@ int launch_rows_grad(const void* gy, const void* full, const void* other, void* 
     if (v.kind == RowsView::kScalar) {
         const int tpr = nslot <= 32 ? 16 : 64;
         const int64_t bx = (v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr);
-        const dim3 grid(static_cast<unsigned>(bx < 0x7fffffffLL ? bx : 0x7fffffffLL));
+        const dim3 grid(capped_blocks(bx, kBcastBlock));
         if (tpr == 16)
             hipLaunchKernelGGL((bcast_row_grad_kernel<S, 16>), grid, dim3(kBcastBlock), 0, st, g, f,
                                o, df, dother, v.rows, v.cols, acc_full, acc_other);

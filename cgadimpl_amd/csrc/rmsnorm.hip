@@ -1135,6 +1135,15 @@ inline Plan ragged(Plan p, int64_t rows, int64_t cols, int w) {
     return p;
 }
 
+// The ragged form of the forward's shape; none where its workgroups, one per g
+// rows, are more than a grid holds (wide rows by the million: the looped kernel's
+// 256 lanes per row still fit).
+inline Plan ragged_fwd_plan(int64_t rows, int64_t cols, int w) {
+    const Plan p = ragged(fwd_plan(row_slots(cols, w), rows), rows, cols, w);
+    if (p.tpr != 0 && !grid_fits((rows + p.g - 1) / p.g, p.tpr * p.g)) return Plan{};
+    return p;
+}
+
 // Row blocking of the resident backward: min(kBwdBlocks, rows) workgroups,
 // about one per CU, so the whole grid runs in one generation and finishes
 // together; workgroup b takes rows b*G + q + k*nblk*G (round-robin, so the
@@ -1221,7 +1230,7 @@ int launch_fwd(const void* x, const void* gamma, void* y, float* inv_rms, int64_
     }
     // Rows off the 16-byte grid: the same shape in its ragged form.  In place
     // (y = x) too: a row's loads end in its sum, which comes before its stores.
-    if (!vec) p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), rows, cols, S::kVec);
+    if (!vec) p = ragged_fwd_plan(rows, cols, S::kVec);
     return launch_fwd_plan<S>(p, x, gamma, y, inv_rms, rows, cols, eps, st);
 }
 
@@ -1246,7 +1255,7 @@ int launch_mul_fwd(const void* a, const void* b, void* y, int64_t rows, int cols
     const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(T));
     if (!vec && (rows >= kLargeRows || bytes >= (1LL << 28)) && disjoint(a, y, bytes) &&
         disjoint(b, cols * static_cast<int64_t>(sizeof(T)), y, bytes))
-        p = ragged(fwd_plan(row_slots(cols, S::kVec), rows), rows, cols, S::kVec);
+        p = ragged_fwd_plan(rows, cols, S::kVec);
     if (p.tpr == 0) {
         if (rows > 0x7fffffffLL) return AGK_EINVAL;
         const int64_t chunk = mul_chunk(rows, cols, vec ? S::kVec : 1);

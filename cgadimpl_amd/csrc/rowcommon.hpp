@@ -360,6 +360,16 @@ inline Plan fwd_plan(int64_t nslot, int64_t rows) {
     return pick_plan(kFwdShapes, nslot, rows > kLargeRows ? 2 : 4, 512, 8);
 }
 
+// HIP takes at most 2^32 - 1 lanes along a grid dimension: the workgroups of `lanes`
+// that fit, for kernels that loop over what the grid leaves, and whether `blocks`
+// of them do, for those that don't.
+constexpr int64_t kMaxGridLanes = 0xffffffffLL;
+inline unsigned capped_blocks(int64_t blocks, int lanes) {
+    const int64_t most = kMaxGridLanes / lanes;
+    return static_cast<unsigned>(blocks < most ? blocks : most);
+}
+inline bool grid_fits(int64_t blocks, int lanes) { return blocks <= kMaxGridLanes / lanes; }
+
 // Whether two tensors share no byte (NULL: no tensor).
 inline bool disjoint(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
     const char *p = static_cast<const char*>(a), *q = static_cast<const char*>(b);

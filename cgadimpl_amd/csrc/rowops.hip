@@ -1151,7 +1151,9 @@ int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
         !prefers_looped_vec<Op, S>(p, cols)) {
         pl = fwd_plan(row_slots(cols, S::kVec), rows);
         pl.rag = true;
-        if (pl.nv > 4) pl = Plan{};
+        // not where the looped kernel's 256 lanes per row fit a grid and these don't
+        if (pl.nv > 4 || (pl.tpr != 0 && !grid_fits((rows + pl.g - 1) / pl.g, pl.tpr * pl.g)))
+            pl = Plan{};
     }
     if constexpr (Resident16<Op>::value) {
         const int64_t nslot = cols / S::kVec;
