@@ -63,6 +63,8 @@ SIGNATURES = {
                                          ctypes.c_int, ctypes.c_int, _P]),
     "agk_gemm_f32": (ctypes.c_int, [_P, _I64, ctypes.c_int, _P, _I64, ctypes.c_int, _P, _I64,
                                     _I64, _I64, _I64, ctypes.c_int, _P]),
+    "agk_gemm_f32_launch_plan": (ctypes.c_int, [_I64, _I64, ctypes.c_int, ctypes.c_int,
+                                                ctypes.c_int, _P]),
     "agk_sum_rows_workspace_bytes": (ctypes.c_size_t, [_I64, _I64]),
     "agk_sum_rows": (ctypes.c_int, [_P, _P, _P, ctypes.c_size_t, _I64, _I64, ctypes.c_int,
                                     ctypes.c_int, _P]),
@@ -350,6 +352,16 @@ def gemm_bf16(a, b, c=None, trans_a: bool = False, trans_b: bool = False, out_dt
                              _stream(stream))
     _check(rc, "agk_gemm_bf16")
     return c
+
+
+def gemm_f32_launch_plan(M: int, N: int, trans_a: bool = False, trans_b: bool = False,
+                         cus: int = 0) -> dict:
+    """The kernel gemm_f32 takes for an M x N product (diagnostic; cus: compute units, 0 for the
+    current device's)."""
+    out = (ctypes.c_int64 * 5)()
+    _check(lib().agk_gemm_f32_launch_plan(M, N, int(trans_a), int(trans_b), cus, out),
+           "agk_gemm_f32_launch_plan")
+    return dict(zip(("shape", "tile_m", "tile_n", "blocks", "lanes"), out))
 
 
 def gemm_f32(a, b, c=None, trans_a: bool = False, trans_b: bool = False, accumulate=False,

@@ -47,8 +47,6 @@
 
 #include <stdint.h>
 
-#include <atomic>
-
 #include "agk_rmsnorm.h"
 #include "gemm_common.hpp"
 #include "gemm_ring.hpp"
@@ -696,22 +694,6 @@ inline int launch_transpose(const void* src, int64_t ld_src, void* dst, int64_t 
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-// Compute units of the current device (looked up once per device; 256 on
-// MI355X), for the direct kernel's last-round split.
-inline int device_cus() {
-    constexpr int kMaxDev = 64;
-    static std::atomic<int> cached[kMaxDev];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return 256;
-    int v = cached[dev].load(std::memory_order_relaxed);
-    if (v > 0) return v;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        v <= 0)
-        v = 256;
-    cached[dev].store(v, std::memory_order_relaxed);
-    return v;
-}
 
 // How many tiles the direct kernel computes whole: all of them, unless the
 // last round (tiles beyond a multiple of the CU count) would fill at most half

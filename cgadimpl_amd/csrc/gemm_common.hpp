@@ -7,6 +7,8 @@
 
 #include <stdint.h>
 
+#include <atomic>
+
 #include "agk_rmsnorm.h"
 
 namespace agk_gemm {
@@ -265,6 +267,22 @@ __device__ __forceinline__ void store_block(const f32x16 (&acc)[TMW][TNW], void*
                                                      nullptr, 0);
         }
     }
+}
+
+// Compute units of the current device (looked up once per device; 256 on
+// MI355X), for the choice of a tile shape and the direct kernel's last-round split.
+inline int device_cus() {
+    constexpr int kMaxDev = 64;
+    static std::atomic<int> cached[kMaxDev];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return 256;
+    int v = cached[dev].load(std::memory_order_relaxed);
+    if (v > 0) return v;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        v <= 0)
+        v = 256;
+    cached[dev].store(v, std::memory_order_relaxed);
+    return v;
 }
 
 // One product's arguments, for the direct and ring launches.

@@ -468,10 +468,9 @@ __global__ __launch_bounds__(256) void zero_rows_kernel(float* __restrict__ C, i
 //   split        0.25      0.25       300 x 500 x 4095: 33 (64 x 64: 77)
 // The kernel this replaced: 1024^3 42 us, 300 x 500 x 4095 143 us,
 // 4096^3 1138-1333 us (by layout; now 1000-1049).
-inline int pick_f32(int64_t M, int64_t N) {
-    constexpr int64_t kCus = 256;
+inline int pick_f32(int64_t M, int64_t N, int cus) {
     auto per_cu = [&](int64_t t) {
-        return static_cast<double>((((M + t - 1) / t) * ((N + t - 1) / t) + kCus - 1) / kCus);
+        return static_cast<double>((((M + t - 1) / t) * ((N + t - 1) / t) + cus - 1) / cus);
     };
     const double c32 = per_cu(32), c64 = per_cu(64), c128 = per_cu(128);
     const double split = 0.25 * c32;
@@ -481,7 +480,39 @@ inline int pick_f32(int64_t M, int64_t N) {
     return small < large ? 1 : 2;
 }
 
+struct F32Plan {
+    int shape, tile;  // pick_f32's, and its tile's rows and columns
+    int64_t tiles_m, tiles_n;
+};
+
+// a_kc: A k-contiguous (not given transposed); b_kc: B k-contiguous (given as B^T).
+inline F32Plan plan_f32(int64_t M, int64_t N, bool a_kc, bool b_kc, int cus) {
+    F32Plan p;
+    p.shape = pick_f32(M, N, cus);
+    // the tiled kernel loads four rows at a time of an operand whose rows are
+    // contiguous: it needs four of them
+    if ((!a_kc && M < 4) || (!b_kc && N < 4)) p.shape = 0;
+    p.tile = p.shape == 2 ? 128 : p.shape == 1 ? 64 : 32;
+    p.tiles_m = (M + p.tile - 1) / p.tile;
+    p.tiles_n = (N + p.tile - 1) / p.tile;
+    return p;
+}
+
 }  // namespace agk_sgemm
+
+extern "C" int agk_gemm_f32_launch_plan(int64_t M, int64_t N, int a_trans, int b_trans, int cus,
+                                        int64_t* plan) {
+    using namespace agk_sgemm;
+    constexpr int64_t kMax = 0x7fffffffLL;
+    if (!plan || M < 1 || N < 1 || M > kMax || N > kMax) return AGK_EINVAL;
+    const F32Plan p = plan_f32(M, N, a_trans == 0, b_trans != 0,
+                               cus > 0 ? cus : agk_gemm::device_cus());
+    plan[0] = p.shape;
+    plan[1] = plan[2] = p.tile;
+    plan[3] = p.tiles_m * p.tiles_n;
+    plan[4] = 256;
+    return AGK_OK;
+}
 
 extern "C" int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const float* B, int64_t ldb,
                             int b_trans, float* C, int64_t ldc, int64_t M, int64_t N, int64_t K,
@@ -504,20 +535,14 @@ extern "C" int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const floa
                            ldc, n);
         return agk::check_launch();
     }
-    // A k-contiguous unless given transposed; B k-contiguous only when given as B^T
     const bool a_kc = a_trans == 0, b_kc = b_trans != 0;
-    int shape = pick_f32(M, N);
-    // the tiled kernel loads four rows at a time of an operand whose rows are
-    // contiguous: it needs four of them
-    if ((!a_kc && M < 4) || (!b_kc && N < 4)) shape = 0;
-    const int tile = shape == 2 ? 128 : shape == 1 ? 64 : 32;
-    const int64_t tiles_m = (M + tile - 1) / tile, tiles_n = (N + tile - 1) / tile;
-    if (tiles_m * tiles_n > kMax) return AGK_EINVAL;
-    const dim3 grid(static_cast<unsigned>(tiles_m * tiles_n));
+    const F32Plan p = plan_f32(M, N, a_kc, b_kc, agk_gemm::device_cus());
+    if (p.tiles_m * p.tiles_n > kMax) return AGK_EINVAL;
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n));
     const int acc = accumulate != 0;
-    const int tm = static_cast<int>(tiles_m), tn = static_cast<int>(tiles_n);
+    const int tm = static_cast<int>(p.tiles_m), tn = static_cast<int>(p.tiles_n);
 #define AGK_F32(AK, BKC)                                                                      \
-    switch (shape) {                                                                          \
+    switch (p.shape) {                                                                        \
         case 2:                                                                               \
             hipLaunchKernelGGL((gemm_f32_kernel<128, 128, AK, BKC>), grid, dim3(256), 0, st,  \
                                A, lda, B, ldb, C, ldc, m, n, k, acc, tm, tn);                 \

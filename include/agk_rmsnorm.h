@@ -230,7 +230,8 @@ int agk_fill(void* dst, int64_t n, float value, int dtype, agk_stream_t stream);
  *   C[M][ldc] (+)= op(A) op(B), all fp32, row-major,
  *   A: a_trans == 0 -> [M][lda], else [K][lda];  B: b_trans == 0 -> [K][ldb],
  *   else [N][ldb].  Hand-written on the fp32 matrix instruction
- *   (v_mfma_f32_32x32x2_f32), 128 x 128 tiles, no split-K and no atomics:
+ *   (v_mfma_f32_32x32x2_f32): 128 x 128 or 64 x 64 tiles, or 32 x 32 tiles
+ *   whose waves share K where those would leave CUs idle; no atomics:
  *   bit-identical run to run.  Not on the RMSNorm layer's bf16 path.  M == 0
  *   or N == 0 is a no-op; K == 0 writes zeros (or leaves C when
  *   accumulating).  No alignment or multiple-of-8 requirements; a kernel
@@ -238,6 +239,13 @@ int agk_fill(void* dst, int64_t n, float value, int dtype, agk_stream_t stream);
 int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const float* B, int64_t ldb,
                  int b_trans, float* C, int64_t ldc, int64_t M, int64_t N, int64_t K,
                  int accumulate, agk_stream_t stream);
+
+/* The kernel agk_gemm_f32 takes for an M x N product on a device of `cus` compute
+ * units (0 or less: the current device): plan[5] = {0: K shared by a workgroup's
+ * waves, 1 or 2: tiles staged through LDS; rows and columns of a tile; workgroups;
+ * lanes per workgroup}.  Launches nothing; used by the tests.               */
+int agk_gemm_f32_launch_plan(int64_t M, int64_t N, int a_trans, int b_trans, int cus,
+                             int64_t* plan);
 
 /* Column sums out[j] (+)= sum_i x[i, j] of a rows x cols matrix, in fp32 and
  * in a fixed order (the same two-stage partial-row reduction as dgamma; no
