@@ -74,6 +74,7 @@ SIGNATURES = {
                                      ctypes.c_size_t, _P]),
     "agk_gemm_bf16_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, ctypes.c_int,
                                                         ctypes.c_int]),
+    "agk_gemm_bf16_launch_plan": (ctypes.c_int, [_I64, _I64, _I64, ctypes.c_int, _P]),
     "agk_transpose_bf16": (ctypes.c_int, [_P, _I64, _P, _I64, _I64, _I64, _P]),
     "agk_rmsnorm_launch_plan": (ctypes.c_int, [_I64, _I64, ctypes.c_int, ctypes.c_int, _P]),
     "agk_set_exchange_wait_limit": (ctypes.c_int, [ctypes.c_int]),
@@ -323,6 +324,14 @@ def transpose_bf16(src, dst=None, stream=None):
     return dst
 
 
+def gemm_bf16_launch_plan(M: int, N: int, K: int, cus: int = 0) -> dict:
+    """The kernel gemm_bf16 takes for an M x N x K product (diagnostic; cus: compute units, 0 for
+    the current device's).  halves: tiles that run as two 256 x 128 halves."""
+    out = (ctypes.c_int64 * 5)()
+    _check(lib().agk_gemm_bf16_launch_plan(M, N, K, cus, out), "agk_gemm_bf16_launch_plan")
+    return dict(zip(("shape", "tile_m", "tile_n", "grid_x", "halves"), out))
+
+
 def gemm_bf16(a, b, c=None, trans_a: bool = False, trans_b: bool = False, out_dtype=None,
               kscale=None, rowscale=None, accumulate: bool = False, workspace="auto",
               stream=None):
@@ -361,7 +370,7 @@ def gemm_f32_launch_plan(M: int, N: int, trans_a: bool = False, trans_b: bool = 
     out = (ctypes.c_int64 * 5)()
     _check(lib().agk_gemm_f32_launch_plan(M, N, int(trans_a), int(trans_b), cus, out),
            "agk_gemm_f32_launch_plan")
-    return dict(zip(("shape", "tile_m", "tile_n", "blocks", "lanes"), out))
+    return dict(zip(("shape", "tile_m", "tile_n", "grid_x", "grid_y"), out))
 
 
 def gemm_f32(a, b, c=None, trans_a: bool = False, trans_b: bool = False, accumulate=False,

@@ -50,6 +50,7 @@
 #include "agk_rmsnorm.h"
 #include "gemm_common.hpp"
 #include "gemm_ring.hpp"
+#include "rowcommon.hpp"
 
 namespace agk_gemm {
 
@@ -817,12 +818,23 @@ int launch_direct(bool f32, const GemmCall& c) {
 //   4096 x 4096 x 1032             36      -              38-77
 //   8192 x 4096 x 4096            204      -              225-489
 // Each round also costs about four steps (first loads, epilogue).
-inline int pick_shape(int M, int N, int K, int cus) {
-    if (K < BK) return kRingSmallK;
+// A shape whose workgroups are more than a grid holds is passed over (columns of
+// 8 by rows in the billions; the direct kernel has the largest tiles).
+inline int pick_shape(int64_t M, int64_t N, int64_t K, int cus) {
+    auto tiles_of = [&](const RingCost& s) {
+        return ((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+    };
+    if (K < BK) {  // the direct kernel needs a whole k-tile
+        int best = kRingSmallK;
+        for (const RingCost& s : kRingCosts)
+            if (s.id == best && !agk::grid_fits(tiles_of(s), 256)) best = kRingLargest;
+        return best;
+    }
     int best = 0;
     double best_cost = 0.0;
     for (const RingCost& s : kRingCosts) {
-        const double tiles = static_cast<double>((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        if (s.id != 0 && !agk::grid_fits(tiles_of(s), 256)) continue;
+        const double tiles = static_cast<double>(tiles_of(s));
         const double slots = static_cast<double>(cus) * s.per_cu;
         const double rounds = static_cast<double>(static_cast<int64_t>(tiles / slots));
         const double fill = tiles / slots - rounds;
@@ -927,6 +939,28 @@ int gemm_impl(const void* A, int64_t lda, int a_trans, const void* B, int64_t ld
 }
 
 }  // namespace agk_gemm
+
+extern "C" int agk_gemm_bf16_launch_plan(int64_t M, int64_t N, int64_t K, int cus,
+                                         int64_t* plan) {
+    using namespace agk_gemm;
+    constexpr int64_t kMax = 0x7fffffffLL;
+    if (!plan || M < 1 || N < 1 || K < 1 || M > kMax || N > kMax || K > kMax) return AGK_EINVAL;
+    if (cus <= 0) cus = device_cus();
+    const int shape = pick_shape(M, N, K, cus);
+    for (const RingCost& s : kRingCosts) {
+        if (s.id != shape) continue;
+        const int64_t tiles = ((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        if (tiles > kMax) return AGK_EINVAL;
+        const int full = direct_full_tiles(static_cast<int>(tiles), cus);
+        plan[0] = shape;
+        plan[1] = s.bm;
+        plan[2] = s.bn;
+        plan[3] = shape == 0 ? full + 2 * (tiles - full) : tiles;
+        plan[4] = shape == 0 ? tiles - full : 0;
+        return AGK_OK;
+    }
+    return AGK_EINVAL;
+}
 
 extern "C" int agk_gemm_bf16(const void* A, int64_t lda, int a_trans, const void* B, int64_t ldb,
                              int b_trans, void* C, int64_t ldc, int c_dtype, int64_t M, int64_t N,

@@ -376,14 +376,17 @@ __device__ __forceinline__ void direct_mfma(const DirectStep& a, const DirectSte
 template <bool A_KC, bool B_KC>
 __global__ __launch_bounds__(kSplitWaves * 64, 2) void gemm_f32_split_kernel(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
-    float* __restrict__ C, int64_t ldc, int M, int N, int K, int accumulate, int tiles_n) {
+    float* __restrict__ C, int64_t ldc, int M, int N, int K, int accumulate, int tiles,
+    int tiles_n) {
     __shared__ float part[kSplitWaves][16][64];  // [wave][accumulator element][lane]
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int half = lane >> 5;
-    const int m0 = (static_cast<int>(blockIdx.x) / tiles_n) * 32;
-    const int n0 = (static_cast<int>(blockIdx.x) % tiles_n) * 32;
+    const int tile = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+    if (tile >= tiles) return;  // workgroup-uniform, before any barrier
+    const int m0 = (tile / tiles_n) * 32;
+    const int n0 = (tile % tiles_n) * 32;
     const int64_t ra = m0 + (lane & 31) < M ? m0 + (lane & 31) : M - 1;
     const int64_t rb = n0 + (lane & 31) < N ? n0 + (lane & 31) : N - 1;
     // the lane's row at k = 32 wave + 4 half, and what 32 kSplitWaves k further on are
@@ -483,6 +486,7 @@ inline int pick_f32(int64_t M, int64_t N, int cus) {
 struct F32Plan {
     int shape, tile;  // pick_f32's, and its tile's rows and columns
     int64_t tiles_m, tiles_n;
+    int64_t grid_x, grid_y;  // the split kernel's tiles may need a second dimension
 };
 
 // a_kc: A k-contiguous (not given transposed); b_kc: B k-contiguous (given as B^T).
@@ -492,9 +496,23 @@ inline F32Plan plan_f32(int64_t M, int64_t N, bool a_kc, bool b_kc, int cus) {
     // the tiled kernel loads four rows at a time of an operand whose rows are
     // contiguous: it needs four of them
     if ((!a_kc && M < 4) || (!b_kc && N < 4)) p.shape = 0;
-    p.tile = p.shape == 2 ? 128 : p.shape == 1 ? 64 : 32;
-    p.tiles_m = (M + p.tile - 1) / p.tile;
-    p.tiles_n = (N + p.tile - 1) / p.tile;
+    auto set = [&](int shape) {
+        p.shape = shape;
+        p.tile = shape == 2 ? 128 : shape == 1 ? 64 : 32;
+        p.tiles_m = (M + p.tile - 1) / p.tile;
+        p.tiles_n = (N + p.tile - 1) / p.tile;
+    };
+    set(p.shape);
+    p.grid_x = p.tiles_m * p.tiles_n;
+    p.grid_y = 1;
+    if (p.shape == 1 && !agk::grid_fits(p.grid_x, 256)) {
+        set(2);
+        p.grid_x = p.tiles_m * p.tiles_n;
+    } else if (p.shape == 0 && !agk::grid_fits(p.grid_x, 256)) {
+        constexpr int64_t kRow = 1 << 20;
+        p.grid_y = (p.grid_x + kRow - 1) / kRow;
+        p.grid_x = kRow;
+    }
     return p;
 }
 
@@ -509,8 +527,8 @@ extern "C" int agk_gemm_f32_launch_plan(int64_t M, int64_t N, int a_trans, int b
                                cus > 0 ? cus : agk_gemm::device_cus());
     plan[0] = p.shape;
     plan[1] = plan[2] = p.tile;
-    plan[3] = p.tiles_m * p.tiles_n;
-    plan[4] = 256;
+    plan[3] = p.grid_x;
+    plan[4] = p.grid_y;
     return AGK_OK;
 }
 
@@ -538,7 +556,7 @@ extern "C" int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const floa
     const bool a_kc = a_trans == 0, b_kc = b_trans != 0;
     const F32Plan p = plan_f32(M, N, a_kc, b_kc, agk_gemm::device_cus());
     if (p.tiles_m * p.tiles_n > kMax) return AGK_EINVAL;
-    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n));
+    const dim3 grid(static_cast<unsigned>(p.grid_x), static_cast<unsigned>(p.grid_y));
     const int acc = accumulate != 0;
     const int tm = static_cast<int>(p.tiles_m), tn = static_cast<int>(p.tiles_n);
 #define AGK_F32(AK, BKC)                                                                      \
@@ -553,7 +571,7 @@ extern "C" int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const floa
             break;                                                                            \
         default:                                                                              \
             hipLaunchKernelGGL((gemm_f32_split_kernel<AK, BKC>), grid, dim3(kSplitWaves * 64), \
-                               0, st, A, lda, B, ldb, C, ldc, m, n, k, acc, tn);              \
+                               0, st, A, lda, B, ldb, C, ldc, m, n, k, acc, tm * tn, tn);     \
     }
     if (a_kc && b_kc) AGK_F32(true, true)
     else if (a_kc) AGK_F32(true, false)

@@ -31,7 +31,8 @@ namespace agk_gemm {
 #define AGK_RING_SHAPES(X)                                                              \
     X(1, 256, 128, 2, 3) X(2, 192, 128, 2, 3) X(3, 128, 192, 2, 3) X(4, 128, 256, 2, 3) \
     X(5, 128, 128, 2, 3) X(6, 128, 64, 2, 3) X(7, 64, 128, 2, 3) X(8, 64, 64, 2, 4)
-constexpr int kRingSmallK = 8;  // fewer than 64 k: one tail tile, nothing to stream
+constexpr int kRingSmallK = 8;   // fewer than 64 k: one tail tile, nothing to stream
+constexpr int kRingLargest = 1;  // the same where 64 x 64 tiles are too many for a grid
 
 template <int BM_, int BN_, int WVM, int NST>
 struct RingShape {

@@ -242,8 +242,8 @@ int agk_gemm_f32(const float* A, int64_t lda, int a_trans, const float* B, int64
 
 /* The kernel agk_gemm_f32 takes for an M x N product on a device of `cus` compute
  * units (0 or less: the current device): plan[5] = {0: K shared by a workgroup's
- * waves, 1 or 2: tiles staged through LDS; rows and columns of a tile; workgroups;
- * lanes per workgroup}.  Launches nothing; used by the tests.               */
+ * waves, 1 or 2: tiles staged through LDS; rows and columns of a tile; the grid's x
+ * and y in workgroups of 256 lanes}.  Launches nothing; used by the tests.   */
 int agk_gemm_f32_launch_plan(int64_t M, int64_t N, int a_trans, int b_trans, int cus,
                              int64_t* plan);
 
@@ -306,6 +306,13 @@ int agk_gemm_bf16(const void* A, int64_t lda, int a_trans, const void* B, int64_
                   int b_trans, void* C, int64_t ldc, int c_dtype, int64_t M, int64_t N,
                   int64_t K, const float* kscale, const float* rowscale, int accumulate,
                   void* workspace, size_t workspace_bytes, agk_stream_t stream);
+
+/* The kernel agk_gemm_bf16 takes without a k-scale, operands' leading dimensions
+ * within 2^31 bytes per tile, on a device of `cus` compute units (0 or less: the
+ * current device): plan[5] = {0: the 256 x 256 kernel, else the id of a ring shape;
+ * rows and columns of a tile; workgroups of 256 lanes; tiles that run as two
+ * halves}.  Launches nothing; used by the tests.                            */
+int agk_gemm_bf16_launch_plan(int64_t M, int64_t N, int64_t K, int cus, int64_t* plan);
 
 /* The linear layer's forward, Y = X W^T + bias, bf16 in and out with fp32
  * accumulation: linear_nodeops (cgadimpl/src/ops/linalg.cpp:21-33,

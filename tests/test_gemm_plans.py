@@ -16,3 +16,26 @@ def test_f32_tile_of_few_rows():
     """An operand whose rows are contiguous needs four of them for the staged tiles."""
     for M, N, ta, tb in ((3, 1 << 20, True, False), (1 << 20, 3, False, False)):
         assert agk.gemm_f32_launch_plan(M, N, trans_a=ta, trans_b=tb, cus=256)["shape"] == 0
+
+
+MOST_LANES = 2 ** 32 - 1  # along a grid dimension
+
+
+@pytest.mark.parametrize("M,N,K", [(2 ** 30 + 8, 8, 8), (2 ** 30 + 8, 8, 64), (2 ** 30 + 64, 64, 56),
+                                   (300_000, 300_000, 8), (300_000, 300_000, 64),
+                                   (8, 2 ** 31 - 512, 64), (2 ** 31 - 512, 8, 8)])
+def test_bf16_grids_fit_a_launch(M, N, K):
+    p = agk.gemm_bf16_launch_plan(M, N, K, cus=256)
+    assert p["grid_x"] * 256 <= MOST_LANES, p
+    assert p["grid_x"] >= -(-M // p["tile_m"]) * -(-N // p["tile_n"])
+    assert K >= 64 or p["shape"] != 0  # the 256 x 256 kernel starts from a whole k-tile
+
+
+@pytest.mark.parametrize("M,N,ta", [(8, 2 ** 29 + 32, False), (1, 2 ** 31 - 1, False),
+                                    (2, 2 ** 30 + 7, True), (64, 2 ** 30 + 64, False),
+                                    (40, 2 ** 30 + 64, True)])
+def test_f32_grids_fit_a_launch(M, N, ta):
+    p = agk.gemm_f32_launch_plan(M, N, trans_a=ta, cus=256)
+    assert p["grid_x"] * 256 <= MOST_LANES and p["grid_y"] <= 65535, p
+    assert p["grid_x"] * p["grid_y"] >= -(-M // p["tile_m"]) * -(-N // p["tile_n"])
+    assert not (ta and M < 4) or p["shape"] == 0

@@ -54,3 +54,42 @@ def test_ragged_rows_by_the_million(cuda):
     for w, z in zip(_windows(rows, 2 ** 23 - 4096), probe):
         ref = z * (z.square().mean(-1, keepdim=True) + 1e-6).rsqrt()
         assert ((x[w].double() - ref).abs() <= 1e-5 * ref.abs()).all().item()
+
+
+@pytest.mark.gpu
+def test_f32_outer_product_of_2_29_columns(cuda):
+    """32 x 32 tiles of 256 lanes: 2^29 columns are 2^32 lanes."""
+    import torch
+    N = 2 ** 29 + 40
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(3)
+    a = torch.randn(2, 1, generator=gen, device=cuda)
+    b = torch.empty(1, N, device=cuda).normal_(generator=gen)
+    print("gemm_f32", 2, N, 1, flush=True)
+    c = agk.gemm_f32(a, b)
+    torch.cuda.synchronize()
+    for w in _windows(N, 2 ** 29):
+        assert torch.equal(c[:, w], a * b[:, w])
+
+
+@pytest.mark.gpu
+def test_bf16_product_of_2_30_rows(cuda):
+    """64 x 64 tiles of 256 lanes: 2^30 rows are 2^32 lanes."""
+    import torch
+    M = 2 ** 30 + 64
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(4)
+    a = torch.empty(M, 8, device=cuda, dtype=torch.bfloat16)
+    pattern = torch.randn(8184, 8, generator=gen, device=cuda).bfloat16()
+    whole = M // 8184 * 8184
+    a[:whole].view(-1, 8184, 8).copy_(pattern.expand(M // 8184, 8184, 8))
+    a[whole:].copy_(pattern[:M - whole])
+    b = torch.randn(8, 8, generator=gen, device=cuda).bfloat16()
+    print("gemm_bf16", M, 8, 8, flush=True)
+    c = agk.gemm_bf16(a, b)
+    torch.cuda.synchronize()
+    want = agk.gemm_bf16(pattern, b)  # the ordinary grid
+    assert torch.equal(c[:whole].view(-1, 8184, 8), want.expand(M // 8184, 8184, 8))
+    assert torch.equal(c[whole:], want[:M - whole])
+    ref = pattern.float() @ b.float()
+    assert ((want.float() - ref).abs().max() / ref.abs().max()).item() <= 8e-3
