@@ -300,6 +300,13 @@ __device__ __forceinline__ int64_t view_col(int64_t slot, int64_t cols) {
     return c + W > cols ? cols - W : c;
 }
 
+// A slot of the full operand or of gy.  STREAM: past the caches.
+template <class S, bool STREAM>
+__device__ __forceinline__ u32x4 view_load(const typename S::T* p) {
+    if constexpr (STREAM) return load16_any_stream<S>(p);
+    else return load16_any<S>(p);
+}
+
 // y (+)= r for one slot, leaving out the first `dup` elements when adding.
 template <class S>
 __device__ __forceinline__ void view_store(typename S::T* y, float (&r)[S::kVec], int dup,
@@ -328,28 +335,53 @@ __device__ __forceinline__ void view_store(typename S::T* y, float (&r)[S::kVec]
 // 1 184 / 167; bf16 2 x 2048 x 4001 by 2 x 1 x 4001 78 / 16; f32 355 / 352.  With the
 // backward kernels below, both gradients: bf16 411 / 257, 587 / 274, 129 / 64; f32
 // 742 / 545, 794 / 573, 130 / 71.
+//
+// Workgroup `id` takes one row block and chunk (view_block).  Rows of 8 chunks and
+// more: chunk c runs on XCD c % 8 (workgroup L runs on XCD L % 8), for one row block
+// after the other, so that c's part of `other` is read into one XCD's L2 once.
 constexpr int kViewSlots = 4;
+constexpr uint32_t kViewXcds = 8;
 
-template <class S, int TPR, bool SCALAR>
+struct ViewBlocks {
+    uint32_t nrow, nchunk;  // row blocks, chunks of a row
+    __host__ __device__ bool wide() const { return nchunk >= kViewXcds; }
+    __host__ __device__ uint32_t total() const {  // with the padding
+        return nrow * (wide() ? (nchunk + kViewXcds - 1) / kViewXcds * kViewXcds : nchunk);
+    }
+};
+
+__device__ __forceinline__ void view_block(const ViewBlocks& b, uint32_t id, uint32_t& row,
+                                           uint32_t& chunk) {
+    const uint32_t q = b.wide() ? id / kViewXcds : id;
+    row = q % b.nrow;
+    chunk = q / b.nrow;
+    if (b.wide()) chunk = chunk * kViewXcds + id % kViewXcds;
+}
+
+template <class S, int TPR, bool SCALAR, bool STREAM>
 __global__ __launch_bounds__(kBcastBlock) void bcast_rows_mul_kernel(
     const typename S::T* __restrict__ full, const typename S::T* __restrict__ other,
-    typename S::T* __restrict__ y, int64_t rows, int64_t cols, int64_t group, int accumulate) {
+    typename S::T* __restrict__ y, int64_t rows, int64_t cols, int64_t group, int accumulate,
+    ViewBlocks blocks) {
     constexpr int W = S::kVec, NV = kViewSlots, RPB = kBcastBlock / TPR;
     const int t = threadIdx.x % TPR;
     const int64_t nslot = (cols + W - 1) / W;
-    for (int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + threadIdx.x / TPR; row < rows;
-         row += static_cast<int64_t>(gridDim.x) * RPB) {
-        const typename S::T* fr = full + row * cols;
-        typename S::T* yr = y + row * cols;
-        const typename S::T* orow = SCALAR ? other + row : other + row / group * cols;
-        const float os = SCALAR ? S::get(orow) : 0.0f;
-        for (int64_t s0 = static_cast<int64_t>(blockIdx.y) * (TPR * NV) + t; s0 < nslot;
-             s0 += static_cast<int64_t>(gridDim.y) * (TPR * NV)) {
+    const uint32_t total = blocks.total();
+    for (uint32_t id = blockIdx.x; id < total; id += gridDim.x) {
+        uint32_t rb, chunk;
+        view_block(blocks, id, rb, chunk);
+        const int64_t row = static_cast<int64_t>(rb) * RPB + threadIdx.x / TPR;
+        const int64_t s0 = static_cast<int64_t>(chunk) * (TPR * NV) + t;
+        if (row < rows && s0 < nslot) {
+            const typename S::T* fr = full + row * cols;
+            typename S::T* yr = y + row * cols;
+            const typename S::T* orow = SCALAR ? other + row : other + row / group * cols;
+            const float os = SCALAR ? S::get(orow) : 0.0f;
             u32x4 fv[NV], ov[SCALAR ? 1 : NV];
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
                 const int64_t s = s0 + k * TPR < nslot ? s0 + k * TPR : nslot - 1;
-                fv[k] = load16_any_stream<S>(fr + view_col<W>(s, cols));
+                fv[k] = view_load<S, STREAM>(fr + view_col<W>(s, cols));
                 if constexpr (!SCALAR) ov[k] = load16_any<S>(orow + view_col<W>(s, cols));
             }
 #pragma unroll
@@ -379,7 +411,7 @@ __global__ __launch_bounds__(kBcastBlock) void bcast_rows_mul_kernel(
 // BATCH of them in flight (loads past the group's end repeat its last row), and
 // their sums are added in lane order: an order fixed by the sizes.  HBM-bound at gy
 // + full + dfull; narrow tiles of 1024 lanes where wide ones would leave CUs idle.
-template <class S, int TW, int LANES, int BATCH>
+template <class S, int TW, int LANES, int BATCH, bool STREAM>
 __global__ __launch_bounds__(LANES) void bcast_group_grad_kernel(
     const typename S::T* __restrict__ gy, const typename S::T* __restrict__ full,
     const typename S::T* __restrict__ other, typename S::T* __restrict__ dfull,
@@ -406,8 +438,8 @@ __global__ __launch_bounds__(LANES) void bcast_group_grad_kernel(
         for (int e = 0; e < W; ++e) acc[e] = 0.0;
         u32x4 gv[BATCH], fv[BATCH];
         auto load = [&](int u, int64_t r) {
-            gv[u] = load16_any_stream<S>(gy + base + r * cols);
-            fv[u] = load16_any_stream<S>(full + base + r * cols);
+            gv[u] = view_load<S, STREAM>(gy + base + r * cols);
+            fv[u] = view_load<S, STREAM>(full + base + r * cols);
         };
         auto use = [&](int u, int64_t r) {
             float a[W], b[W];
@@ -642,6 +674,14 @@ inline bool grad_view_fits(const RowsView& v) {
     return v.kind == RowsView::kGroup;
 }
 
+// Full operands of this many bytes and more are loaded past the caches: with y they
+// exceed the 256 MiB Infinity Cache, where smaller ones may still lie from the
+// kernel that wrote them, and stay for the one that reads them next.  Measured on
+// MI355X by a scalar per row, ordinary / streaming loads (us, operands in the cache
+// where they fit; from HBM): 20 MB 5.7 / 8.8; 8.3 / 10.2, 100 MB 33 / 39; 32 / 40,
+// 200 MB 64 / 76; 64 / 77, 400 MB 134 / 126; 135 / 126.
+constexpr int64_t kStreamBytes = 256LL << 20;
+
 template <class S>
 int launch_rows_mul(const void* full, const void* other, void* y, const RowsView& v,
                     int accumulate, hipStream_t st) {
@@ -649,24 +689,31 @@ int launch_rows_mul(const void* full, const void* other, void* y, const RowsView
     const int64_t nslot = row_slots(v.cols, S::kVec);
     const int64_t need = (nslot + kViewSlots - 1) / kViewSlots;
     const int tpr = need <= 16 ? 16 : need <= 64 ? 64 : need <= 128 ? 128 : 256;
-    const int64_t bx = (v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr);
-    const int64_t by = (nslot + tpr * kViewSlots - 1) / (tpr * kViewSlots);
-    const dim3 grid(capped_blocks(bx, kBcastBlock), static_cast<unsigned>(by < 65535 ? by : 65535));
-#define AGK_ROWS_MUL(TPR)                                                                         \
+    // (a workgroup moves at least 256 bytes: the counts fit 32 bits)
+    ViewBlocks blocks;
+    blocks.nrow = static_cast<uint32_t>((v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr));
+    blocks.nchunk = static_cast<uint32_t>((nslot + tpr * kViewSlots - 1) / (tpr * kViewSlots));
+    const dim3 grid(capped_blocks(blocks.total(), kBcastBlock));
+    const bool stream = view_elems(v) * static_cast<int64_t>(sizeof(T)) >= kStreamBytes;
+#define AGK_ROWS_MUL(TPR, SCALAR, STREAM)                                                         \
+    hipLaunchKernelGGL((bcast_rows_mul_kernel<S, TPR, SCALAR, STREAM>), grid, dim3(kBcastBlock),  \
+                       0, st, static_cast<const T*>(full), static_cast<const T*>(other),          \
+                       static_cast<T*>(y), v.rows, v.cols, v.group, accumulate, blocks)
+#define AGK_ROWS_MUL_TPR(TPR)                                                                     \
     do {                                                                                          \
-        if (v.kind == RowsView::kScalar)                                                          \
-            hipLaunchKernelGGL((bcast_rows_mul_kernel<S, TPR, true>), grid, dim3(kBcastBlock), 0, \
-                               st, static_cast<const T*>(full), static_cast<const T*>(other),     \
-                               static_cast<T*>(y), v.rows, v.cols, v.group, accumulate);          \
-        else                                                                                      \
-            hipLaunchKernelGGL((bcast_rows_mul_kernel<S, TPR, false>), grid, dim3(kBcastBlock),   \
-                               0, st, static_cast<const T*>(full), static_cast<const T*>(other),  \
-                               static_cast<T*>(y), v.rows, v.cols, v.group, accumulate);          \
+        if (v.kind == RowsView::kScalar) {                                                        \
+            if (stream) AGK_ROWS_MUL(TPR, true, true);                                            \
+            else AGK_ROWS_MUL(TPR, true, false);                                                  \
+        } else {                                                                                  \
+            if (stream) AGK_ROWS_MUL(TPR, false, true);                                           \
+            else AGK_ROWS_MUL(TPR, false, false);                                                 \
+        }                                                                                         \
     } while (0)
-    if (tpr == 16) AGK_ROWS_MUL(16);
-    else if (tpr == 64) AGK_ROWS_MUL(64);
-    else if (tpr == 128) AGK_ROWS_MUL(128);
-    else AGK_ROWS_MUL(256);
+    if (tpr == 16) AGK_ROWS_MUL_TPR(16);
+    else if (tpr == 64) AGK_ROWS_MUL_TPR(64);
+    else if (tpr == 128) AGK_ROWS_MUL_TPR(128);
+    else AGK_ROWS_MUL_TPR(256);
+#undef AGK_ROWS_MUL_TPR
 #undef AGK_ROWS_MUL
     return check_launch();
 }
@@ -686,36 +733,52 @@ int launch_rows_grad(const void* gy, const void* full, const void* other, void* 
         const int tpr = nslot <= 32 ? 16 : 64;
         const int64_t bx = (v.rows + kBcastBlock / tpr - 1) / (kBcastBlock / tpr);
         const dim3 grid(capped_blocks(bx, kBcastBlock));
-        if (tpr == 16)
-            hipLaunchKernelGGL((bcast_row_grad_kernel<S, 16>), grid, dim3(kBcastBlock), 0, st, g, f,
-                               o, df, dother, v.rows, v.cols, acc_full, acc_other);
-        else
-            hipLaunchKernelGGL((bcast_row_grad_kernel<S, 64>), grid, dim3(kBcastBlock), 0, st, g, f,
-                               o, df, dother, v.rows, v.cols, acc_full, acc_other);
+#define AGK_ROW_GRAD(TPR)                                                                       \
+    hipLaunchKernelGGL((bcast_row_grad_kernel<S, TPR>), grid, dim3(kBcastBlock), 0, st, \
+                       g, f, o, df, dother, v.rows, v.cols, acc_full, acc_other)
+        if (tpr == 16) AGK_ROW_GRAD(16);
+        else AGK_ROW_GRAD(64);
+#undef AGK_ROW_GRAD
         return check_launch();
     }
     const int64_t groups = v.rows / v.group;
     // One row lane for short groups; else whole kilobytes per row (four row
-    // lanes), or narrower tiles of 64 or 256 row lanes where those would leave CUs
-    // without a workgroup and the group has the rows.  Measured on MI355X, both
-    // gradients (us, 4- / 16- / 64-slot tiles): f32 8 x 2048 x 1024 86 / 50 / -, bf16
-    // 42 / 51 / -; f32 2 x 2048 x 4001 126 / 71 / -; bf16 20 groups' rows of 117520
-    // - / 32 / 16; f32 2 x 2048 x 64 15 / 28 / - (the two passes this replaces: 76,
-    // 73, 130, 15, 32).
+    // lanes), or narrower tiles of 16 to 256 row lanes where those would leave CUs
+    // without a workgroup.  Measured on MI355X, both gradients (us, 4- / 16- / 64-slot
+    // tiles): f32 8 x 2048 x 1024 86 / 50 / -, bf16 42 / 51 / -; f32 2 x 2048 x 4001 126 /
+    // 71 / -; bf16 20 groups' rows of 117520 - / 32 / 16; f32 2 x 2048 x 64 15 / 28 / -
+    // (the two passes this replaces: 76, 73, 130, 15, 32); bf16 sums alone 40 x 73 x 513
+    // to 40 x 513 - / 4.7 (256 lanes) / 7.7.
     auto tiles = [&](int64_t tw) { return (nslot + tw - 1) / tw; };
     int tw = v.group <= 8 ? 256 : 64;
-    if (v.group >= 128 && tiles(64) * groups < 256)
+    if (v.group > 8 && tiles(64) * groups < 256)
         tw = v.group >= 512 && tiles(16) * groups < 100 ? 4 : 16;
     if (tiles(tw) > 0x7fffffffLL) return AGK_EINVAL;
     const dim3 grid(static_cast<unsigned>(tiles(tw)),
                     static_cast<unsigned>(groups < 65535 ? groups : 65535));
-#define AGK_GROUP_GRAD(TW, LANES, BATCH)                                                         \
-    hipLaunchKernelGGL((bcast_group_grad_kernel<S, TW, LANES, BATCH>), grid, dim3(LANES), 0, st, \
-                       g, f, o, df, dother, groups, v.group, v.cols, acc_full, acc_other)
-    if (tw == 256) AGK_GROUP_GRAD(256, 256, 8);
-    else if (tw == 64) AGK_GROUP_GRAD(64, 256, 8);
-    else if (tw == 16) AGK_GROUP_GRAD(16, 1024, 4);
-    else AGK_GROUP_GRAD(4, 1024, 4);
+    // Loads stream past the caches unless tiles share 128-byte lines, which then stay
+    // for the neighbour.  Measured on MI355X, both gradients, ordinary / streaming loads
+    // (us, operands from HBM): f32 2 x 97465 x 513 by 2 x 513 (odd widths, all sizes of 400
+    // MB) 724 / 906, 2 x 64-column rows of 200 MB 339 / 370, but 8 x 24366 x 513 by 24366 x
+    // 513 241 / 221.
+    const uintptr_t at = reinterpret_cast<uintptr_t>(gy) | reinterpret_cast<uintptr_t>(full) |
+                         static_cast<uintptr_t>(v.cols * static_cast<int64_t>(sizeof(T)));
+    const bool stream = tw == 256 || (tw >= 16 && at % 128 == 0);
+#define AGK_GROUP_GRAD(TW, LANES, BATCH, STREAM)                                              \
+    hipLaunchKernelGGL((bcast_group_grad_kernel<S, TW, LANES, BATCH, STREAM>), grid,          \
+                       dim3(LANES), 0, st, g, f, o, df, dother, groups, v.group, v.cols,      \
+                       acc_full, acc_other)
+#define AGK_GROUP_GRAD_TW(TW, LANES, BATCH)                                                   \
+    do {                                                                                      \
+        if (stream) AGK_GROUP_GRAD(TW, LANES, BATCH, true);                                   \
+        else AGK_GROUP_GRAD(TW, LANES, BATCH, false);                                         \
+    } while (0)
+    if (tw == 256) AGK_GROUP_GRAD_TW(256, 256, 8);
+    else if (tw == 64) AGK_GROUP_GRAD_TW(64, 256, 8);
+    else if (tw == 16 && v.group < 128) AGK_GROUP_GRAD_TW(16, 256, 8);
+    else if (tw == 16) AGK_GROUP_GRAD_TW(16, 1024, 4);
+    else AGK_GROUP_GRAD_TW(4, 1024, 4);
+#undef AGK_GROUP_GRAD_TW
 #undef AGK_GROUP_GRAD
     return check_launch();
 }
@@ -831,6 +894,24 @@ inline RowsView product_view(int nd, const int64_t* osize, const Aligned& al, co
     return v;
 }
 
+// Whether the rows x cols kernel takes a product: not tiny ones off the 16-byte grid,
+// where the element-wise kernel's shorter start counts, nor, on it, rows of many chunks
+// in tiny tensors, or by one vector in many rows of large ones.  Measured on MI355X
+// (us, general / rows x cols): bf16 8 x 6 x 513 by 6 x 513 2.4 / 2.9, f32 8 x 3 x 4096 by
+// 3 x 4096 2.2 / 2.7 (2 x 610 x 4096 by 610 x 4096 6.7 / 4.7), f32 40 x 305 x 4096 by 305 x
+// 4096 55 / 59, bf16 40 x 1220 x 4096 by 1220 x 4096 135 / 149 (8 rows: 167 / 164).
+template <class S>
+inline bool rows_mul_fits(const RowsView& v, const void* full, const void* other, const void* y) {
+    constexpr int64_t kTiny = 1 << 16, kTinyWide = 1 << 18, kLarge = 128LL << 20;
+    const int64_t n = view_elems(v);
+    if (v.cols % S::kVec != 0 || !aligned16(full) || !aligned16(other) || !aligned16(y))
+        return n >= kTiny;
+    if (v.kind != RowsView::kGroup || v.cols < kViewXcds * kBcastBlock * kViewSlots * S::kVec)
+        return true;
+    return n >= kTinyWide && (v.group != v.rows || v.rows < 16 ||
+                              n * static_cast<int64_t>(sizeof(typename S::T)) < kLarge);
+}
+
 template <class S>
 int bcast_bwd_one(const void* gy, const void* other, const Aligned& t, const Aligned& o,
                   const Aligned& gyal, int nd, const int64_t* osize, void* d, int accumulate,
@@ -840,7 +921,8 @@ int bcast_bwd_one(const void* gy, const void* other, const Aligned& t, const Ali
         const void *full = nullptr, *bc = nullptr;
         const int dtype = S::kVec == 4 ? AGK_F32 : AGK_BF16;
         const RowsView v = product_view(nd, osize, gyal, o, gy, other, d, dtype, &full, &bc);
-        if (v.kind != RowsView::kNone) return launch_rows_mul<S>(full, bc, d, v, accumulate, st);
+        if (v.kind != RowsView::kNone && rows_mul_fits<S>(v, full, bc, d))
+            return launch_rows_mul<S>(full, bc, d, v, accumulate, st);
         const BcastGeom g = make_geom(nd, osize, gyal, o);
         return launch_bcast_mul<S>(gy, other, d, g, accumulate, st);
     }
@@ -917,7 +999,9 @@ extern "C" int agk_mul_bcast_fwd(const void* a, const int64_t* a_shape, int a_nd
     const int acc = accumulate != 0;
     const void *full = nullptr, *other = nullptr;
     const RowsView v = product_view(nd, osize, al, bl, a, b, y, dtype, &full, &other);
-    if (v.kind != RowsView::kNone)
+    if (v.kind != RowsView::kNone &&
+        (dtype == AGK_F32 ? rows_mul_fits<F32>(v, full, other, y)
+                          : rows_mul_fits<BF16>(v, full, other, y)))
         return dtype == AGK_F32 ? launch_rows_mul<F32>(full, other, y, v, acc, st)
                                 : launch_rows_mul<BF16>(full, other, y, v, acc, st);
     const BcastGeom g = make_geom(nd, osize, al, bl);

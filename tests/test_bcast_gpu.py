@@ -192,7 +192,13 @@ VIEW_SHAPES = [((5, 37, 61), (5, 1, 61)), ((3, 9, 8), (3, 1, 8)), ((2, 300, 129)
                ((300, 17), (1, 17)), ((3, 1000, 1031), (3, 1, 1031)), ((2, 64, 4096), (2, 1, 4096)),
                ((33, 2051), (1, 2051)), ((7, 33, 5), (7, 33, 1)), ((4100, 40), (4100, 1)),
                ((2, 3, 20001), (2, 3, 1)), ((1500, 300), (1500, 1)), ((1030,), (1,)),
-               ((40, 3), (40, 1)), ((2, 3, 4, 32), (2, 1, 4, 32)), ((70000, 9), (70000, 1))]
+               ((40, 3), (40, 1)), ((2, 3, 4, 32), (2, 1, 4, 32)), ((70000, 9), (70000, 1)),
+               # rows of 8 chunks and more (an odd and a whole number of them), by one vector and
+               # by a scalar per row; a group of 70 rows in few tiles; tiny and large tensors,
+               # where the general kernels take over and where loads pass the caches by
+               ((5, 80001), (1, 80001)), ((3, 131072), (131072,)), ((3, 90003), (3, 1)),
+               ((20, 70, 33), (20, 1, 33)), ((2, 70, 515), (2, 1, 515)), ((3, 5, 4096), (5, 4096)),
+               ((16, 2200000), (2200000,)), ((70001, 1030), (70001, 1)), ((9, 4, 2000001), (9, 4, 1))]
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
