@@ -217,6 +217,7 @@ struct BwdCtx {
     uint32_t row_bytes, x_bytes, old_bytes, dx_bytes, dr_bytes, roff;
     uint32_t off[NV];
     float inv_cols;
+    bool same;       // RAG: rows of whole slots
     int klast, dup;  // RAG: the index of the row's last slot, and what it overlaps in this lane
 
     // First row of the wave's rows at `step` (clamped into range) and how many exist.
@@ -266,19 +267,66 @@ __device__ __forceinline__ void stored_product(float (&f)[S::kVec], const float 
     for (int e = 0; e < W; ++e) asm("" : "+v"(f[e]));
 }
 
+// A lane's dgamma sums.  Aligned rows add in fp32.  Ragged rows (FP64) add in fp64,
+// because their 256 workgroups take up to four times the rows of the looped kernel's,
+// whose fp32 sums were that much shorter.  (Relative error of dgamma, looped / fp32 sums
+// here / fp64: f32 20000 x 4099 1.1e-7 / 1.7e-7 / 0.7e-7, 60001 x 2051 1.6e-7 / 2.7e-7 /
+// 0.7e-7, bf16 1200 x 95 0.9e-7 / 1.7e-7 / 0.8e-7; sums of bf16 columns 2.5e-8 in each, so
+// those stay in fp32.)  It costs up to 5 % of the VJP and 12 % of fp32 column sums.  Rows
+// of whole slots that only start off a 16-byte boundary (`same`) add in fp32, for the bits
+// of aligned rows.  The widest shape, 16 sums per lane, has no registers for them in fp64:
+// they live in LDS, a column of it per lane (128 KiB).
+template <class S, int KIND, bool RAG>
+constexpr bool fp64_sums() {
+    return RAG && !(KIND == kBwdColSum && std::is_same<S, BF16>::value);
+}
+
+template <bool FP64, int NV, int W>
+struct BwdSums {
+    static constexpr bool kLds = FP64 && NV == 4;
+    static constexpr int kStride = 1024;
+    using T = std::conditional_t<FP64, double, float>;
+    T v[kLds ? 1 : NV][kLds ? 1 : W];
+    T* lds;  // kLds: this lane's first sum; the next one is kStride further on
+
+    __device__ __forceinline__ T& at(int k, int e) {
+        if constexpr (kLds) return lds[(k * W + e) * kStride];
+        else return v[k][e];
+    }
+    __device__ __forceinline__ float get(int k, int e) { return static_cast<float>(at(k, e)); }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int k = 0; k < NV; ++k)
+#pragma unroll
+            for (int e = 0; e < W; ++e) at(k, e) = 0;
+    }
+    // SAME: fp32 sums whatever T is (which holds them exactly)
+    template <bool SAME>
+    __device__ __forceinline__ void add(int k, int e, float a) {
+        if constexpr (SAME) at(k, e) = get(k, e) + a;
+        else at(k, e) += a;
+    }
+    template <bool SAME>
+    __device__ __forceinline__ void add_product(int k, int e, float a, float b) {
+        if constexpr (SAME) at(k, e) = __builtin_fmaf(a, b, get(k, e));
+        else if constexpr (FP64) at(k, e) += static_cast<double>(a) * static_cast<double>(b);  // exact
+        else at(k, e) += a * b;
+    }
+};
+
 template <class S, int TPR, int NV, int G, bool ACC, int KIND, bool RAG = false>
 __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIND, RAG>& c,
                                             BwdSet<S, NV, ACC>& b,
                                             int64_t step, int parity, const u32x4 (&gv)[NV],
-                                            bool has_gamma, float (&dg)[NV][S::kVec],
+                                            bool has_gamma, BwdSums<fp64_sums<S, KIND, RAG>(), NV, S::kVec>& dg,
                                             float (*red)[TPR > 64 ? G * (TPR / 64) : 1]) {
     constexpr int W = S::kVec;
+    constexpr bool kFp64 = fp64_sums<S, KIND, RAG>();
     const float r = b.r;
     float s = 0.0f;
     constexpr bool MUL = KIND == kBwdMul;
     constexpr bool COMP = KIND == kBwdRmsMul;
     if constexpr (KIND == kBwdColSum) {
-        (void)c;
         (void)step;
         (void)parity;
         (void)red;
@@ -288,8 +336,13 @@ __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIN
         for (int k = 0; k < NV; ++k) {
             float fd[W];
             S::unpack(b.dv[k], fd);
+            if (kFp64 && c.same) {
 #pragma unroll
-            for (int e = 0; e < W; ++e) dg[k][e] += fd[e];
+                for (int e = 0; e < W; ++e) dg.template add<true>(k, e, fd[e]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < W; ++e) dg.template add<false>(k, e, fd[e]);
+            }
         }
         return;
     }
@@ -389,19 +442,17 @@ __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIN
         } else {
             bstore16_stream(rdx, c.off[k], S::pack(o));
         }
-        if constexpr (MUL) {
+        if constexpr (!MUL) {
 #pragma unroll
-            for (int e = 0; e < W; ++e) dg[k][e] += fd[e] * fx[e];
-        } else if constexpr (COMP) {
-            float h[W];
+            for (int e = 0; e < W; ++e) fx[e] = fx[e] * r;
+            if constexpr (COMP) S::unpack(S::pack(fx), fx);
+        }
+        if (kFp64 && c.same) {
 #pragma unroll
-            for (int e = 0; e < W; ++e) h[e] = fx[e] * r;
-            S::unpack(S::pack(h), h);
-#pragma unroll
-            for (int e = 0; e < W; ++e) dg[k][e] += fd[e] * h[e];
+            for (int e = 0; e < W; ++e) dg.template add_product<true>(k, e, fd[e], fx[e]);
         } else {
 #pragma unroll
-            for (int e = 0; e < W; ++e) dg[k][e] += fd[e] * (fx[e] * r);
+            for (int e = 0; e < W; ++e) dg.template add_product<false>(k, e, fd[e], fx[e]);
         }
     }
 }
@@ -411,7 +462,7 @@ __device__ __forceinline__ void bwd_process(const BwdCtx<S, TPR, NV, G, ACC, KIN
 template <class S, int TPR, int NV, int G, int NSET, bool ACC, int KIND, bool RAG = false>
 __device__ __forceinline__ void bwd_segment(const BwdCtx<S, TPR, NV, G, ACC, KIND, RAG>& c, int64_t steps,
                                             const u32x4 (&gv)[NV], bool has_gamma,
-                                            float (&dg)[NV][S::kVec],
+                                            BwdSums<fp64_sums<S, KIND, RAG>(), NV, S::kVec>& dg,
                                             float (*red)[TPR > 64 ? G * (TPR / 64) : 1]) {
     if constexpr (NSET == 1) {
         BwdSet<S, NV, ACC> A;
@@ -462,9 +513,9 @@ __device__ __forceinline__ void bwd_segment(const BwdCtx<S, TPR, NV, G, ACC, KIN
 // Writes one partial row of dgamma: the G groups' sums (each group's in its
 // own LDS row) added in group order, column by column.  Ends with a barrier
 // so the LDS rows can be written again.
-template <class S, int TPR, int NV, int G, bool RAG = false>
+template <class S, int TPR, int NV, int G, bool RAG = false, bool FP64 = RAG>
 __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int cols, int t,
-                                                  int grp, const float (&dg)[NV][S::kVec],
+                                                  int grp, BwdSums<FP64, NV, S::kVec>& dg,
                                                   float* lds_part) {
     constexpr int W = S::kVec;
     if constexpr (G == 1) {
@@ -473,7 +524,7 @@ __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int 
             const int col = slot_col<RAG, W>(t + k * TPR, cols);
             if (col < cols) {
 #pragma unroll
-                for (int e = 0; e < W; ++e) prow[col + e] = dg[k][e];
+                for (int e = 0; e < W; ++e) prow[col + e] = dg.get(k, e);
             }
         }
     } else {
@@ -482,11 +533,33 @@ __device__ __forceinline__ void bwd_write_partial(float* __restrict__ prow, int 
             const int col = slot_col<RAG, W>(t + k * TPR, cols);
             if (col < cols) {
 #pragma unroll
-                for (int e = 0; e < W; ++e) lds_part[grp * cols + col + e] = dg[k][e];
+                for (int e = 0; e < W; ++e)
+                    lds_part[grp * cols + col + e] = dg.get(k, e);
             }
         }
         __syncthreads();
-        for (int c2 = threadIdx.x; c2 < cols; c2 += TPR * G) {
+        if constexpr (RAG) if (cols % W != 0) {  // uniform
+            // P lanes per column, each adding every P-th group; then a fixed tree
+            constexpr int CP = TPR * NV * W, P = TPR * G / CP > 1 ? TPR * G / CP : 1;
+            __shared__ double sums[P > 1 ? TPR * G : 1];
+            for (int c2 = threadIdx.x % CP; c2 < cols; c2 += TPR * G) {
+                double v = 0.0;
+                for (int q = threadIdx.x / CP % P; q < G; q += P) v += lds_part[q * cols + c2];
+                if constexpr (P > 1) sums[threadIdx.x] = v;
+                else prow[c2] = static_cast<float>(v);
+            }
+            if constexpr (P > 1) {
+                const int p = threadIdx.x / CP, c2 = threadIdx.x % CP;
+                for (int h = P / 2; h > 0; h /= 2) {
+                    __syncthreads();
+                    if (p < h && c2 < cols) sums[threadIdx.x] += sums[threadIdx.x + h * CP];
+                }
+                if (p == 0 && c2 < cols) prow[c2] = static_cast<float>(sums[c2]);
+            }
+            __syncthreads();
+            return;
+        }
+        for (int c2 = threadIdx.x; c2 < cols; c2 += TPR * G) {  // in group order
             float v = lds_part[c2];
             for (int q = 1; q < G; ++q) v += lds_part[q * cols + c2];
             prow[c2] = v;
@@ -530,6 +603,7 @@ __device__ __forceinline__ void bwd_setup(BwdCtx<S, TPR, NV, G, ACC, KIND, RAG>&
     c.roff = static_cast<uint32_t>(sub) * 4u;
     c.inv_cols = 1.0f / static_cast<float>(cols);
     if constexpr (RAG) {
+        c.same = cols % W == 0;
         const int last = (cols + W - 1) / W - 1;  // the row's last slot
         c.klast = last / TPR;
         c.dup = t == last % TPR ? (last + 1) * W - cols : 0;
@@ -564,16 +638,20 @@ __device__ __forceinline__ void bwd_resident_body(
     u32x4 gv[NV];
     bwd_setup(c, gv, x, gamma, inv_rms, dy, dx, dr, rows, cols, blockIdx.x, gridDim.x);
     const bool has_gamma = gamma != nullptr;
-    float dg[NV][W];
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-#pragma unroll
-        for (int e = 0; e < W; ++e) dg[k][e] = 0.0f;
+    constexpr bool kFp64 = fp64_sums<S, KIND, RAG>();
+    using Sums = BwdSums<kFp64, NV, W>;
+    Sums dg;
+    if constexpr (Sums::kLds) {
+        static_assert(TPR * G == Sums::kStride, "a column of LDS per lane");
+        __shared__ double sums[NV * W * Sums::kStride];
+        dg.lds = sums + threadIdx.x;  // no other lane's: no barrier
+    }
+    dg.clear();
 
     const int64_t steps = c.first < rows ? (rows - c.first + c.stride - 1) / c.stride : 0;
     bwd_segment<S, TPR, NV, G, NSET, ACC, KIND, RAG>(c, steps, gv, has_gamma, dg, red);
     if (partials)
-        bwd_write_partial<S, TPR, NV, G, RAG>(partials + static_cast<int64_t>(blockIdx.x) * cols, cols,
+        bwd_write_partial<S, TPR, NV, G, RAG, kFp64>(partials + static_cast<int64_t>(blockIdx.x) * cols, cols,
                                          t, grp, dg, lds_part);
 }
 
@@ -665,11 +743,8 @@ __global__ __launch_bounds__(TPR * G) void bwd_fewrows(
         BwdCtx<S, TPR, NV, G, ACC, KIND> c;
         u32x4 gv[NV];
         bwd_setup(c, gv, x, gamma, inv_rms, dy, dx, dr, rows, cols, blockIdx.x, nrow_blocks);
-        float dg[NV][W];  // unused: dgamma comes from the column workgroups
-#pragma unroll
-        for (int k = 0; k < NV; ++k)
-#pragma unroll
-            for (int e = 0; e < W; ++e) dg[k][e] = 0.0f;
+        BwdSums<false, NV, W> dg;  // unused: dgamma comes from the column workgroups
+        dg.clear();
         BwdSet<S, NV, ACC> A;
         c.issue(A, 0);
         bwd_process(c, A, 0, 0, gv, gamma != nullptr, dg, red);
@@ -1107,6 +1182,14 @@ constexpr int rms_mul_sets(int nv, int sets) {
     return (nv == 1 && sets == 2) ? 3 : bwd_sets<S>(nv, sets);
 }
 
+// Ragged rows that accumulate into dx hold the old dx and fp64 sums besides: two sets
+// for bf16 (three would spill).
+template <class S, bool ACC>
+constexpr int rms_mul_ragged_sets(int nv, int sets) {
+    return (std::is_same<S, BF16>::value && ACC && nv == 1) ? bwd_sets<S>(nv, sets)
+                                                           : rms_mul_sets<S>(nv, sets);
+}
+
 template <class S>
 inline Plan bwd_plan(int64_t nslot) {
     Plan p;
@@ -1426,7 +1509,8 @@ int launch_rms_mul_bwd_resident(const Plan& p, int64_t nblk, const void* x, cons
     if constexpr (bwd_shape_enabled<S>(a, b)) {                                            \
         if (p.tpr == a && p.nv == b && p.g == c) {                                         \
             if (p.rag)                                                                     \
-                hipLaunchKernelGGL((rms_mul_bwd_resident<S, a, b, c, rms_mul_sets<S>(b, d), \
+                hipLaunchKernelGGL((rms_mul_bwd_resident<S, a, b, c,                       \
+                                                         rms_mul_ragged_sets<S, ACC>(b, d), \
                                                          ACC, true>),                      \
                                    dim3(static_cast<unsigned>(nblk)), dim3(a * c), lds, st, \
                                    xp, gp, inv_rms, gyp, dxp, drp, partials, rows, cols);  \

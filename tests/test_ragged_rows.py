@@ -47,7 +47,7 @@ def _check(x, g, dy, y, inv, dx, dg, label):
 
 
 @pytest.mark.parametrize("dtype,cols", CASES, ids=str)
-@pytest.mark.parametrize("rows", [1, 37, 600])
+@pytest.mark.parametrize("rows", [1, 37, 600, 1700])
 def test_layer_matches_fp64(cuda, dtype, cols, rows):
     import torch
     print(f"{dtype} {rows}x{cols}", flush=True)
@@ -80,11 +80,11 @@ def test_layer_matches_fp64(cuda, dtype, cols, rows):
 
 @pytest.mark.parametrize("dtype,cols", CASES, ids=str)
 @pytest.mark.parametrize("accumulate", [False, True])
-def test_composition_equals_its_two_calls(cuda, dtype, cols, accumulate):
+@pytest.mark.parametrize("rows", [600, 900])
+def test_composition_equals_its_two_calls(cuda, dtype, cols, accumulate, rows):
     """agk_rms_mul_bwd against the multiply's VJP then the RMSNorm VJP of dr, bit for bit, and
     the column sums of a linear layer's bias."""
     import torch
-    rows = 600
     x, g, gy = device_inputs((rows, cols), dtype, cols, cuda)
     r, inv = agk.rmsnorm_fwd(x, None, EPS)
     y = agk.mul_rowbcast_fwd(r, g)
@@ -155,7 +155,7 @@ def test_infinities_and_nans_stay_where_they_belong(cuda, dtype, cols):
     """An infinite or NaN dy or x in the overlapped columns (which two slots hold): the same
     NaN / infinity pattern as the formula in fp32, other rows and columns untouched."""
     import torch
-    x, g, dy = device_inputs((600, cols), dtype, cols, cuda)
+    x, g, dy = device_inputs((700, cols), dtype, cols, cuda)
     _, _, clean_dx, clean_dg, _ = _ref(x, g, dy)
     dy[3, cols - 3] = float("inf")
     dy[5, cols - 1] = float("nan")
@@ -169,7 +169,7 @@ def test_infinities_and_nans_stay_where_they_belong(cuda, dtype, cols):
     want = r * (gy - xf * s)
     assert torch.equal(torch.isnan(dx), torch.isnan(want))
     assert torch.equal(torch.isinf(dx), torch.isinf(want))
-    rows = [i for i in range(600) if i not in (3, 5, 7)]
+    rows = [i for i in range(700) if i not in (3, 5, 7)]
     bar = (1e-5 + (2.0 ** -8 if dtype == "bf16" else 0.0)) * clean_dx.abs().amax()
     assert ((dx[rows].double() - clean_dx[rows]).abs() <= bar).all().item()
     bad = [cols - 9, cols - 3, cols - 1]
@@ -183,8 +183,10 @@ ROWOP_COLS = {"f32": [4, 5, 9, 61, 253, 515, 1001, 4099, 8195, 16383],
               "bf16": [8, 9, 121, 1001, 4099, 8195, 16391, 32767]}
 
 
-@pytest.mark.parametrize("dtype,cols", [(d, c) for d in ROWOP_COLS for c in ROWOP_COLS[d]], ids=str)
-@pytest.mark.parametrize("rows", [1, 541])
+# rows 4100: enough for the ragged form at every width that is looped in few rows
+@pytest.mark.parametrize("dtype,cols,rows", [(d, c, r) for d in ROWOP_COLS for c in ROWOP_COLS[d]
+                                             for r in (1, 541, 4100) if r < 4100 or c < 1025],
+                         ids=str)
 def test_row_ops_match_fp64(cuda, dtype, cols, rows):
     """LayerNorm, softmax and log-sum-exp, the RMSNorm JVP, with masked logits in the overlapped
     columns.  Bars: 1e-5 of the row's scale (fp32 sums and the hardware exponential's
@@ -255,3 +257,27 @@ def test_row_ops_match_fp64(cuda, dtype, cols, rows):
     agk.softmax_fwd(in_place, y=in_place)
     torch.cuda.synchronize()
     assert torch.equal(in_place, agk.softmax_fwd(z))
+
+
+@pytest.mark.parametrize("dtype,rows,cols", [("f32", 60001, 131), ("f32", 30000, 2051),
+                                             ("f32", 5000, 9001), ("bf16", 60001, 95),
+                                             ("bf16", 9000, 4099)], ids=str)
+def test_column_gradients_of_many_rows(cuda, dtype, rows, cols):
+    """dgamma, the row-vector multiply's db and the column sums: fp64 sums in 256 partial rows,
+    each rounded to fp32, and the total rounded again.  A rounding is at most 2^-24 relative,
+    0.42 of that in the root mean square, so the two together stay under 2^-24 of the result in
+    the 2-norm over the columns; dgamma's terms hold one rounding more each (x times inv_rms).
+    fp32 sums of the same rows are two to four times further off."""
+    import torch
+    x, g, dy = device_inputs((rows, cols), dtype, rows + cols, cuda)
+    _, inv = agk.rmsnorm_fwd(x, None, EPS)
+    _, dg = agk.rmsnorm_bwd(x, g, inv, dy, want_dx=False)
+    _, db = agk.mul_rowbcast_bwd(dy, x, g, want_da=False)
+    s = agk.sum_rows(x)
+    torch.cuda.synchronize()
+    x64, d64 = x.double(), dy.double()
+    for got, terms, roundings in ((dg, d64 * (x64 * inv.double().view(-1, 1)), 1), (db, d64 * x64, 0),
+                                  (s, x64, 0)):
+        want = terms.sum(0)
+        bound = 2.0 ** -24 * (want.norm() + roundings * terms.norm())
+        assert (got.double() - want).norm() <= bound
