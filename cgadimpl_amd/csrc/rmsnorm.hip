@@ -84,7 +84,7 @@ __global__ __launch_bounds__(TPR * G) void rms_fwd_resident(
     for (int k = 0; k < NV; ++k) {
         const int col = slot_col<RAG, W>(t + k * TPR, cols);
         xv[k] = (active && col < cols)
-                    ? (RAG ? load16_any_stream<S>(xr + col) : load16_stream<S>(xr + col))
+                    ? (RAG ? load16_any<S>(xr + col) : load16_stream<S>(xr + col))
                     : u32x4{0u, 0u, 0u, 0u};
     }
     [[maybe_unused]] u32x4 gv[EARLY_G ? NV : 1];
@@ -1210,10 +1210,34 @@ inline Plan bwd_plan(int64_t nslot) {
     return p;
 }
 
+// Rows below which the looped kernels stay off the 16-byte grid: a workgroup per row
+// then has the latency-bound call to itself, and the ragged form's several rows per
+// workgroup leave CUs idle.  kRagFwd: the forward (the row-vector multiply has a rule of
+// its own besides); kRagBwd: the VJPs of RMSNorm, of the row-vector multiply and of the
+// two together, whose results are each other's bits, so one line serves them; kRagSum:
+// the column sums.  Measured on MI355X (graph replays, us, looped / ragged):
+//   forward: f32 520 x 191 2.7 / 2.7; bf16 520 x 191 2.7 / 3.3, 1200 x 191 3.0 / 3.3, 800 x
+//     383 3.2 / 3.5;
+//   RMSNorm VJP: f32 520 x 191 6.2 / 6.2, 520 x 1001 9.5 / 7.6, 64 x 2051 12.6 / 8.8; bf16
+//     520 x 191 6.2 / 6.9, 520 x 767 8.2 / 8.8, 800 x 767 9.6 / 8.6; with dr bf16 800 x 767
+//     10.1 / 10.9; the multiply's f32 64 x 4099 8.1 / 9.2, 520 x 4099 15.6 / 13.5;
+//   column sums: f32 520 x 95 5.5 / 5.8, 520 x 1001 7.8 / 5.9, 20 x 4099 5.4 / 6.0, 150 x
+//     4099 8.1 / 7.2; bf16 150 x 1535 5.6 / 6.0.
+enum : int { kRagFwd, kRagBwd, kRagSum };
+template <class S>
+inline int64_t ragged_min_rows(int kind, int64_t cols) {
+    constexpr bool f32 = std::is_same<S, F32>::value;
+    if (cols > 1024) return kind == kRagSum ? 100 : 0;
+    if (kind == kRagSum) return cols > 256 ? 513 : 641;
+    if (f32) return 513;
+    return kind == kRagBwd ? 641 : cols > 448 ? 513 : cols > 256 ? 1000 : 1600;
+}
+
 // p (the shape for row_slots(cols, w) slots) in its ragged form; none for rows
-// of less than one slot, or few short ones.
-inline Plan ragged(Plan p, int64_t rows, int64_t cols, int w) {
-    if (p.tpr == 0 || cols < w || few_short_rows(rows, cols)) return Plan{};
+// of less than one slot, or too few.
+template <class S>
+inline Plan ragged(Plan p, int kind, int64_t rows, int64_t cols) {
+    if (p.tpr == 0 || cols < S::kVec || rows < ragged_min_rows<S>(kind, cols)) return Plan{};
     p.rag = true;
     return p;
 }
@@ -1221,8 +1245,9 @@ inline Plan ragged(Plan p, int64_t rows, int64_t cols, int w) {
 // The ragged form of the forward's shape; none where its workgroups, one per g
 // rows, are more than a grid holds (wide rows by the million: the looped kernel's
 // 256 lanes per row still fit).
-inline Plan ragged_fwd_plan(int64_t rows, int64_t cols, int w) {
-    const Plan p = ragged(fwd_plan(row_slots(cols, w), rows), rows, cols, w);
+template <class S>
+inline Plan ragged_fwd_plan(int64_t rows, int64_t cols) {
+    const Plan p = ragged<S>(fwd_plan(row_slots(cols, S::kVec), rows), kRagFwd, rows, cols);
     if (p.tpr != 0 && !grid_fits((rows + p.g - 1) / p.g, p.tpr * p.g)) return Plan{};
     return p;
 }
@@ -1313,7 +1338,7 @@ int launch_fwd(const void* x, const void* gamma, void* y, float* inv_rms, int64_
     }
     // Rows off the 16-byte grid: the same shape in its ragged form.  In place
     // (y = x) too: a row's loads end in its sum, which comes before its stores.
-    if (!vec) p = ragged_fwd_plan(rows, cols, S::kVec);
+    if (!vec) p = ragged_fwd_plan<S>(rows, cols);
     return launch_fwd_plan<S>(p, x, gamma, y, inv_rms, rows, cols, eps, st);
 }
 
@@ -1338,7 +1363,7 @@ int launch_mul_fwd(const void* a, const void* b, void* y, int64_t rows, int cols
     const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(T));
     if (!vec && (rows >= kLargeRows || bytes >= (1LL << 28)) && disjoint(a, y, bytes) &&
         disjoint(b, cols * static_cast<int64_t>(sizeof(T)), y, bytes))
-        p = ragged_fwd_plan(rows, cols, S::kVec);
+        p = ragged_fwd_plan<S>(rows, cols);
     if (p.tpr == 0) {
         if (rows > 0x7fffffffLL) return AGK_EINVAL;
         const int64_t chunk = mul_chunk(rows, cols, vec ? S::kVec : 1);
@@ -1484,12 +1509,12 @@ inline Plan bwd_plan_for(const void* x, const void* gamma, const void* dy, const
 // [4099, 1030] against the looped kernels: forward 8.6 us from 11.8, backward
 // 12.9 from 40.1, its finalize 3.5 from 4.6 (a quarter of the partial rows).
 template <class S>
-inline Plan ragged_bwd_plan(const void* x, const void* dy, const void* dx, const void* dr,
-                            int64_t rows, int cols) {
+inline Plan ragged_bwd_plan(int kind, const void* x, const void* dy, const void* dx,
+                            const void* dr, int64_t rows, int cols) {
     const int64_t bytes = rows * cols * static_cast<int64_t>(sizeof(typename S::T));
     for (const void* o : {dx, dr})
         if (!disjoint(o, x, bytes) || !disjoint(o, dy, bytes)) return Plan{};
-    const Plan p = ragged(bwd_plan<S>(row_slots(cols, S::kVec)), rows, cols, S::kVec);
+    const Plan p = ragged<S>(bwd_plan<S>(row_slots(cols, S::kVec)), kind, rows, cols);
     if (p.tpr != 0 && p.g > 1 && static_cast<int64_t>(p.g) * cols * 4 > 64 * 1024) return Plan{};
     return p;
 }
@@ -1591,7 +1616,7 @@ int launch_bwd(const void* x, const void* gamma, const float* inv_rms, const voi
         nblk = bwd_num_blocks(rows);
     }
     if (p.tpr == 0) {
-        p = ragged_bwd_plan<S>(x, dy, dx, dr, rows, cols);
+        p = ragged_bwd_plan<S>(kRagBwd, x, dy, dx, dr, rows, cols);
         if (p.tpr != 0) nblk = bwd_resident_blocks(rows);
     }
     if (p.tpr != 0 && !p.rag && rows <= kFewRowsMax) {
@@ -2068,8 +2093,8 @@ int agk_mul_rowbcast_bwd(const void* gy, const void* a, const void* b, void* da,
     Plan p = dtype == AGK_F32 ? bwd_plan_for<F32>(a, b, gy, da, rows, c, nblk, rpb)
                               : bwd_plan_for<BF16>(a, b, gy, da, rows, c, nblk, rpb);
     if (p.tpr == 0) {
-        p = dtype == AGK_F32 ? ragged_bwd_plan<F32>(a, gy, da, nullptr, rows, c)
-                             : ragged_bwd_plan<BF16>(a, gy, da, nullptr, rows, c);
+        p = dtype == AGK_F32 ? ragged_bwd_plan<F32>(kRagBwd, a, gy, da, nullptr, rows, c)
+                             : ragged_bwd_plan<BF16>(kRagBwd, a, gy, da, nullptr, rows, c);
         if (p.tpr != 0) nblk = bwd_resident_blocks(rows);
     }
     if (nblk > 0x7fffffffLL) return AGK_EINVAL;
@@ -2138,8 +2163,8 @@ int agk_sum_rows(const void* x, float* out, void* workspace, size_t workspace_by
     Plan p = dtype == AGK_F32 ? bwd_plan_for<F32>(x, nullptr, x, nullptr, rows, c, nblk, rpb)
                               : bwd_plan_for<BF16>(x, nullptr, x, nullptr, rows, c, nblk, rpb);
     if (p.tpr == 0) {
-        p = dtype == AGK_F32 ? ragged_bwd_plan<F32>(x, x, nullptr, nullptr, rows, c)
-                             : ragged_bwd_plan<BF16>(x, x, nullptr, nullptr, rows, c);
+        p = dtype == AGK_F32 ? ragged_bwd_plan<F32>(kRagSum, x, x, nullptr, nullptr, rows, c)
+                             : ragged_bwd_plan<BF16>(kRagSum, x, x, nullptr, nullptr, rows, c);
         if (p.tpr != 0) nblk = bwd_resident_blocks(rows);
     }
     if (nblk > 0x7fffffffLL) return AGK_EINVAL;

@@ -173,14 +173,6 @@ __device__ __forceinline__ void drop_dup(float (&f)[W], int dup) {
     for (int e = 0; e < W; ++e) f[e] = e < dup ? 0.0f : f[e];
 }
 
-// Few short ragged rows keep the looped kernels: a workgroup per row then has
-// the whole latency-bound call to itself, and the ragged form's several rows per
-// workgroup leave CUs idle.  Measured on MI355X (graph replays, us, looped /
-// ragged): backward 64 x 515 f32 8.7 / 9.2, bf16 8.8 / 10.0; 300 x 515 bf16 7.4 /
-// 8.7; 1000 x 515 10.5 / 8.0; 64 x 2051 13.1 / 9.3; layernorm 300 x 1001 f32 4.0-4.2
-// / 4.5, 300 x 2051 5.5-5.7 / 4.6-4.7.
-inline bool few_short_rows(int64_t rows, int64_t cols) { return rows <= 512 && cols <= 1024; }
-
 // Slots of a row, the last one perhaps partly filled.
 inline int64_t row_slots(int64_t cols, int w) { return (cols + w - 1) / w; }
 

@@ -63,6 +63,7 @@ struct RowArgs {
     float* ws1 = nullptr;        // per-row fp32 output 1, [rows]
     float eps = 0.0f;
     int acc = 0;                 // out += f instead of out = f
+    bool stream = true;          // ragged rows: loaded past the caches (stream_rows)
 };
 
 // ---- reductions ----------------------------------------------------------------
@@ -203,12 +204,23 @@ struct Resident {
         const int64_t off = (active ? row : 0) * static_cast<int64_t>(cols);
         const T* x = static_cast<const T*>(p.in0) + off;
         const T* y = NIN == 2 ? static_cast<const T*>(p.in1) + off : nullptr;
+        if constexpr (RAG) {
+            if (!p.stream) {
+                load_slots([](const T* q) { return load16_any<S>(q); }, x, y);
+                return;
+            }
+        }
+        load_slots([](const T* q) { return load_row(q); }, x, y);
+    }
+
+    template <class L>
+    __device__ __forceinline__ void load_slots(L load, const T* x, const T* y) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const int col = slot_col<RAG, W>(t + k * TPR, cols);
             const bool ok = active && col < cols;
-            a[k] = ok ? load_row(x + col) : u32x4{0u, 0u, 0u, 0u};
-            if constexpr (NIN == 2) b[k] = ok ? load_row(y + col) : u32x4{0u, 0u, 0u, 0u};
+            a[k] = ok ? load(x + col) : u32x4{0u, 0u, 0u, 0u};
+            if constexpr (NIN == 2) b[k] = ok ? load(y + col) : u32x4{0u, 0u, 0u, 0u};
         }
     }
 
@@ -1129,14 +1141,51 @@ inline bool fits_buffer(int cols) {
 //   f32 4000 x 16383 (looped 16-byte kernel before): backward 163 -> 139, softmax
 //     forward 85 -> 93, log-sum-exp forward 39 -> 42; bf16 4000 x 30001: backward
 //     143 -> 168, softmax forward 75 -> 101, log-sum-exp forward 37 -> 57.
+// Of many wide rows of two fp32 inputs, those that fill little more than half of the
+// widest shape's slots stay looped too: layernorm backward f32 64 x 8193 4.6 / 4.0, 1200 x
+// 8193 21.8 / 21.4, 3000 x 8193 47.7 / 54.8.
 template <class Op, class S>
-inline bool prefers_looped_vec(const RowArgs& p, int cols) {
+inline bool prefers_looped_vec(const RowArgs& p, int64_t rows, int cols) {
     if (cols < kVecMinCols || !fits_buffer<S>(cols) || !same_offset<typename S::T>(p)) return false;
-    return Op::kIn == 1 || (std::is_same<S, BF16>::value && row_slots(cols, S::kVec) > 2048);
+    const int64_t nslot = row_slots(cols, S::kVec);
+    return Op::kIn == 1 ||
+           (std::is_same<S, BF16>::value ? nslot > 2048 : rows > 1500 && nslot <= 2560);
+}
+
+// Few short ragged rows keep the looped kernel: a workgroup per row then has the
+// latency-bound call to itself, and the ragged form's several rows per workgroup leave
+// CUs idle.  Measured on MI355X (graph replays, us, looped / ragged; the lines lie where
+// the two meet):
+//   f32, two inputs (layernorm backward): 520 x 191 2.6 / 2.9, 1200 x 515 3.6 / 3.9, 1200 x
+//     1001 4.3 / 4.2, 2000 x 515 4.2 / 4.1; one: 520 x 767 3.6 / 3.7, 800 x 767 3.8 / 3.8;
+//   bf16, two inputs: 520 x 191 2.6 / 3.6, 2000 x 383 3.6 / 3.9, 3000 x 383 4.4 / 4.0, 1200 x
+//     767 3.7 / 4.0, 1200 x 1001 4.1 / 4.1; one (layernorm forward): 520 x 191 2.9 / 3.5,
+//     1200 x 383 3.6 / 3.8, 2000 x 383 4.3 / 3.9, 800 x 767 3.8 / 3.7.
+template <class Op, class S>
+inline bool few_short_rows(int64_t rows, int64_t cols) {
+    if (cols > 1024) return false;
+    if (rows <= 512) return true;
+    if (std::is_same<S, F32>::value) return Op::kIn == 2 && rows <= 1200;
+    return Op::kIn == 2 ? rows <= 4000 && rows * cols <= 1100000
+                        : rows <= 1800 && rows * cols <= 700000;
+}
+
+// Whether ragged rows pass the caches on their way in: from 256 MiB of inputs, what the
+// Infinity Cache holds.  Smaller ones may still lie there, and rows off the 128-byte
+// lines share lines with their neighbours.  Measured on MI355X (graph replays, us,
+// streaming / ordinary loads, means over widths of 131-16383): softmax backward on
+// tensors of 16 MB f32 10.5 / 8.3, bf16 11.9 / 8.5, 60 MB 32.7 / 29.7, 34.9 / 29.3, 200
+// MB 101 / 106, 114 / 116; layernorm forward 60 MB 24.2 / 22.2, 27.7 / 24.8, 500 MB
+// level.
+template <class Op, class S>
+inline bool stream_rows(int64_t rows, int64_t cols) {
+    return Op::kIn * rows * cols * static_cast<int64_t>(sizeof(typename S::T)) >= 256LL << 20;
 }
 
 template <class Op, class S>
-int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
+int launch(const RowArgs& args, int64_t rows, int cols, hipStream_t st) {
+    RowArgs p = args;
+    p.stream = stream_rows<Op, S>(rows, cols);
     const bool vec = (cols % S::kVec) == 0 && aligned16(p.in0) && aligned_or_null(p.in1) &&
                      aligned_or_null(p.out) && aligned_or_null(p.col0) &&
                      aligned_or_null(p.col1);
@@ -1147,8 +1196,8 @@ int launch(const RowArgs& p, int64_t rows, int cols, hipStream_t st) {
         const Plan q{pl.tpr / 2, 4, pl.tpr >= 512 ? 1 : 512 / pl.tpr, false};
         if (has_shape(kFwdShapes, q)) pl = q;
     }
-    if (!vec && cols >= S::kVec && !few_short_rows(rows, cols) &&
-        !prefers_looped_vec<Op, S>(p, cols)) {
+    if (!vec && cols >= S::kVec && !few_short_rows<Op, S>(rows, cols) &&
+        !prefers_looped_vec<Op, S>(p, rows, cols)) {
         pl = fwd_plan(row_slots(cols, S::kVec), rows);
         pl.rag = true;
         // not where the looped kernel's 256 lanes per row fit a grid and these don't
