@@ -741,48 +741,16 @@ int dispatch_ks(bool has_ks, int c_dtype, const void* A, int64_t lda, const void
 
 namespace agk_gemm {
 
-// Tile orders measured on MI355X for the products of the RMSNorm + linear
-// layer at its headline size (M = 8192 rows, K = 4096, N = 11008), with
-// random bf16 operands; every other shape takes kGroupM.  The best group size
-// depends on the shape in ways no simple rule captured (the same y layout
-// with K = 8192 is fastest at 4, with 16384 rows at 2), so only shapes that
-// were measured are listed.  Microseconds per product, group size 2 / 4 / 8:
-//   y  = h W     (32 x 43 tiles, 64 k-steps, A k-contiguous, B k-strided):
-//                 531-537 / 551-561 / 549-558
-//   dh = dy W^T  (32 x 16 tiles, 172 k-steps, both k-contiguous):
-//                 565-570 / 506-516 / 493-499
-// (dW = h^T dy, 16 x 43 tiles, measured 524-550 at every group size: 4.)
-// The order changes only which workgroup computes which tile: results are
-// bit-identical.
-struct TunedOrder {
-    int tiles_m, tiles_n, nk;
-    bool a_tr, b_tr;
-    int group_m;
-};
-constexpr TunedOrder kTunedOrders[] = {
-    {32, 43, 64, false, true, 2},     // y
-    {32, 16, 172, false, false, 8},   // dh
-};
-
-inline int tuned_group_m(int tiles_m, int tiles_n, int nk, bool a_tr, bool b_tr) {
-    for (const TunedOrder& t : kTunedOrders)
-        if (t.tiles_m == tiles_m && t.tiles_n == tiles_n && t.nk == nk && t.a_tr == a_tr &&
-            t.b_tr == b_tr)
-            return t.group_m;
-    return kGroupM;
-}
-
 template <bool A_TR, bool B_TR>
 int launch_direct(bool f32, const GemmCall& c) {
     const int tiles_m = (c.M + BM - 1) / BM, tiles_n = (c.N + BN - 1) / BN;
-    const int gm = tuned_group_m(tiles_m, tiles_n, c.K / BK, A_TR, B_TR);
     const int tiles = tiles_m * tiles_n;
     const int full = direct_full_tiles(tiles, device_cus());
     const dim3 grid(full + 2 * (tiles - full)), block(kDirectThreads);
 #define AGK_DIRECT(F32, TAIL, S)                                                               \
     hipLaunchKernelGGL((gemm_nt_direct_kernel<F32, A_TR, B_TR, TAIL, Stores::S>), grid, block, \
                        0, c.st, c.A, c.lda, c.B, c.ldb, c.C, c.ldc, c.M, c.N, c.K, c.rowscale, \
-                       c.colbias, c.accumulate, tiles_m, tiles_n, gm, full)
+                       c.colbias, c.accumulate, tiles_m, tiles_n, kGroupM, full)
     const bool tail = c.K % BK != 0;
     if constexpr (!A_TR && !B_TR) {  // the layout of agk_linear_bf16
         if (!f32 && c.colbias != nullptr && c.rowscale == nullptr && !c.accumulate) {
