@@ -777,15 +777,20 @@ int launch_direct(bool f32, const GemmCall& c) {
 // lower the clock): light for a round of few workgroups, full for a full one,
 // light + (full - light) * fill^2 between.  The two times per shape were
 // measured on MI355X (random bf16, k-contiguous operands, K = 4096: 512 and
-// 8192 rows by 4096 columns); with them the rule came within 10 % of the best
-// shape's time at every product of the sweep:
+// 8192 rows by 4096 columns).  What a round costs besides its k-steps is left out,
+// so K decides only below one k-tile.  Against every shape's time at 1179 products of
+// 64 to 8192 rows, 128 to 11008 columns and K of 64 to 4096, in the three layouts of a
+// layer's products (both k-contiguous, B strided, A and B strided with fp32 output), the
+// rule's shape takes 3.5 % more than the best one on average, and 21 % in one of twenty;
+// costs with a fixed part per round, fitted to them, came to 1.4 % and 9 % but were up to
+// 45 % slower at single sizes.
 //   rows x columns x K (us)   256x256  ring shape taken   other shapes
 //   512 x 4096 x 4096              58      22 (128x64)    22-42
 //   1032 x 4096 x 4096             65      39 (192x128)   39-73
+//   1032 x 4096 x 64               6.5     8.0 (192x128)  6.3-8.1
 //   2048 x 4096 x 4096             84      57 (128x256)   59-137
 //   4096 x 4096 x 1032             36      -              38-77
 //   8192 x 4096 x 4096            204      -              225-489
-// Each round also costs about four steps (first loads, epilogue).
 // A shape whose workgroups are more than a grid holds is passed over (columns of
 // 8 by rows in the billions; the direct kernel has the largest tiles).
 inline int pick_shape(int64_t M, int64_t N, int64_t K, int cus) {
@@ -806,8 +811,8 @@ inline int pick_shape(int64_t M, int64_t N, int64_t K, int cus) {
         const double slots = static_cast<double>(cus) * s.per_cu;
         const double rounds = static_cast<double>(static_cast<int64_t>(tiles / slots));
         const double fill = tiles / slots - rounds;
-        const double step = rounds * s.full + (fill > 0 ? s.light + (s.full - s.light) * fill * fill : 0.0);
-        const double cost = step * (static_cast<double>(K) / BK + 4.0);
+        const double cost =
+            rounds * s.full + (fill > 0 ? s.light + (s.full - s.light) * fill * fill : 0.0);
         if (s.id == 0 || cost < best_cost) {
             best = s.id;
             best_cost = cost;

@@ -100,6 +100,53 @@ def test_gemm_against_torch(cuda, M, N, K, ta, tb, ws):
 # k-tiles than the ring has stages.
 SHAPE_CASES = [(456, 5376), (688, 5392), (336, 5624), (1168, 4864), (5416, 664), (5808, 1032),
                (392, 4840), (72, 136), (3392, 2320)]
+# The launch plan's shape of each of them on 256 compute units (test_gemm_plans.py).
+SHAPE_IDS = [5, 2, 6, 4, 3, 1, 7, 8, 0]
+# (shape, tiles in halves, M, N, K): each shape, and the 256 x 256 kernel where its last round of
+# few tiles runs as two 256 x 128 halves each, at one k-tile, with a tail and at several.
+PLAN_CASES = ([(i, False, M, N, K) for i, (M, N) in zip(SHAPE_IDS, SHAPE_CASES) for K in (72, 256)]
+              + [(0, True, 7880, 2824, K) for K in (64, 72, 200)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,halves,M,N,K", PLAN_CASES)
+def test_gemm_every_plan(cuda, shape, halves, M, N, K):
+    """Every kernel and tile shape: the four layouts' fp32 products against a float64 one (the
+    bar of fp32 sums of exact products, K 2^-24 |a| |b| per element) and equal to each other, the
+    bf16 product their rounding, accumulation, a row scale and the bias in the store."""
+    import torch
+    plan = agk.gemm_bf16_launch_plan(M, N, K)
+    print(f"gemm {M}x{N}x{K} {plan}", flush=True)
+    assert (plan["shape"], plan["halves"] > 0) == (shape, halves)
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(M + 3 * N + 7 * K)
+    a = torch.randn(M, K, generator=gen, device=cuda).bfloat16()
+    b = torch.randn(N, K, generator=gen, device=cuda).bfloat16()
+    A, B = a.double(), b.double()
+    want = A @ B.t()
+    bound = K * 2.0 ** -24 * (A.abs() @ B.abs().t())
+    first = None
+    for ta, tb in ((0, 1), (0, 0), (1, 1), (1, 0)):
+        aa, bb = a.t().contiguous() if ta else a, b if tb else b.t().contiguous()
+
+        def product(**kw):
+            return agk.gemm_bf16(aa, bb, trans_a=bool(ta), trans_b=bool(tb), **kw)
+
+        c = product(out_dtype=torch.float32)
+        half = product(out_dtype=torch.bfloat16)
+        if first is None:
+            first = c
+            assert ((c.double() - want).abs() <= bound).all().item(), (ta, tb)
+        assert torch.equal(c, first) and torch.equal(half, c.bfloat16()), (ta, tb)
+        base = torch.full((M, N), 0.5, device=cuda)
+        product(c=base, accumulate=True)
+        assert torch.equal(base, c + 0.5), (ta, tb)
+        rs = torch.rand(M, generator=gen, device=cuda) + 0.5
+        assert torch.equal(product(out_dtype=torch.float32, rowscale=rs), c * rs[:, None]), (ta, tb)
+    bias = torch.randn(N, generator=gen, device=cuda).bfloat16()
+    y = agk.linear_bf16(a, b, bias)
+    torch.cuda.synchronize()
+    assert torch.equal(y, (first.bfloat16().float() + bias.float()).bfloat16())
 
 
 @pytest.mark.gpu

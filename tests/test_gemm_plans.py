@@ -2,6 +2,7 @@
 import pytest
 
 import cgadimpl_amd as agk
+from test_gemm import PLAN_CASES, SHAPE_IDS
 
 
 @pytest.mark.parametrize("M,N,shape", [(1024, 1024, {256: 1, 32: 2}), (2048, 2048, {256: 2, 32: 2}),
@@ -39,3 +40,13 @@ def test_f32_grids_fit_a_launch(M, N, ta):
     assert p["grid_x"] * 256 <= MOST_LANES and p["grid_y"] <= 65535, p
     assert p["grid_x"] * p["grid_y"] >= -(-M // p["tile_m"]) * -(-N // p["tile_n"])
     assert not (ta and M < 4) or p["shape"] == 0
+
+
+def test_bf16_cases_reach_every_shape():
+    """The GPU tests' sizes take the shapes they stand for, on 256 compute units, and leave none
+    out."""
+    assert sorted(SHAPE_IDS) == list(range(9))
+    for shape, halves, M, N, K in PLAN_CASES:
+        p = agk.gemm_bf16_launch_plan(M, N, K, cus=256)
+        assert (p["shape"], p["halves"] > 0) == (shape, halves), (M, N, K, p)
+        assert M % p["tile_m"] or N % p["tile_n"], (M, N, K, p)  # ragged last tiles
