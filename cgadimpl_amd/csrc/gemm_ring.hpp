@@ -258,9 +258,9 @@ __global__ __launch_bounds__(256, SH::kPerCu) void gemm_ring_kernel(
     constexpr int NST = SH::kStages;
     __shared__ __attribute__((aligned(16))) uint16_t st0[SH::kElems];
     __shared__ __attribute__((aligned(16))) uint16_t st1[SH::kElems];
-    __shared__ __attribute__((aligned(16))) uint16_t st2[NST > 2 ? SH::kElems : 8];
+    __shared__ __attribute__((aligned(16))) uint16_t st2[SH::kElems];
     __shared__ __attribute__((aligned(16))) uint16_t st3[NST > 3 ? SH::kElems : 8];
-    static_assert(NST >= 2 && NST <= 4, "ring of two to four stages");
+    static_assert(NST == 3 || NST == 4, "ring of three or four stages");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -298,14 +298,14 @@ __global__ __launch_bounds__(256, SH::kPerCu) void gemm_ring_kernel(
 
     // The K % 64 tail goes first, through the last stage, whose own loads are
     // issued by step 0.
-    uint16_t* const last = NST == 2 ? st1 : NST == 3 ? st2 : st3;
+    uint16_t* const last = NST == 3 ? st2 : st3;
     const int k_left = K - r.nk * BK;
     if (k_left) {
         stage_k_tail<A_TR, SH::kBM>(last, a0, lda, rows_a, r.nk * BK, K);
         stage_k_tail<B_TR, SH::kBN>(last + SH::kBM * BK, b0, ldb, rows_b, r.nk * BK, K);
     }
     ring_issue<SH>(r, o, st0, 0, wave);
-    if constexpr (NST > 2) ring_issue<SH>(r, o, st1, 1, wave);
+    ring_issue<SH>(r, o, st1, 1, wave);
     if constexpr (NST > 3) ring_issue<SH>(r, o, st2, 2, wave);
     if (k_left) {
         stage_barrier<(NST - 1) * SH::kLoads>();  // the tail's LDS writes, every wave
@@ -320,13 +320,7 @@ __global__ __launch_bounds__(256, SH::kPerCu) void gemm_ring_kernel(
                                      wave)
         AGK_RING(true, st0, last, 0);
         int t = 1;
-        if constexpr (NST == 2) {
-            for (; t + 1 < r.nk; t += 2) {
-                AGK_RING(false, st1, st0, t);
-                AGK_RING(false, st0, st1, t + 1);
-            }
-            if (t < r.nk) AGK_RING(false, st1, st0, t);
-        } else if constexpr (NST == 3) {
+        if constexpr (NST == 3) {
             for (; t + 2 < r.nk; t += 3) {
                 AGK_RING(false, st1, st0, t);
                 AGK_RING(false, st2, st1, t + 1);
