@@ -15,7 +15,13 @@
 // The host merges adjacent axes that both operands walk contiguously (and
 // drops extent-1 output axes), so a launch sees at most 8 axes, usually 2-3.
 //
-// Otherwise:
+// The broadcasts that training code writes most -- a full operand times a vector
+// per group of rows ([B, T, D] * [B, 1, D], [B, T, D] * [T, D]) or a scalar per row
+// ([B, T, D] * [B, T, 1]) -- have kernels of their own over a rows x cols view of
+// the full operand (RowsView): 16-byte accesses at any element alignment
+// (rowcommon.hpp, ragged rows), and a backward that reads gy and the full operand
+// once for both gradients.  The general kernels take every other pair, products that
+// they are faster for (rows_mul_fits) and outputs that lie over the operands:
 //
 // Forward / full-shape gradient (y (+)= a * b): one workgroup row per run of
 // the innermost output axis; its base offsets into a and b are decomposed once
@@ -34,14 +40,6 @@
 //    (short sums) or one 256-lane workgroup (long sums) per output element;
 //    lane l takes positions l, l + lanes, ... of the reduced index space in
 //    row-major order, and the lanes' partials meet in a fixed tree in LDS.
-
-//
-// The broadcasts that training code writes most -- a full operand times a vector
-// per group of rows ([B, T, D] * [B, 1, D], [B, T, D] * [T, D]) or a scalar per row
-// ([B, T, D] * [B, T, 1]) -- have kernels of their own over a rows x cols view of
-// the full operand (RowsView): 16-byte accesses at any element alignment
-// (rowcommon.hpp, ragged rows), and a backward that reads gy and the full operand
-// once for both gradients.
 
 #include <hip/hip_runtime.h>
 

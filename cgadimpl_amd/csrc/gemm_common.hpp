@@ -1,6 +1,6 @@
-// gemm_common.hpp -- what the bf16 product kernels (gemm.hip, gemm_ring.hpp) share: types and conversions, the LDS layouts of staged
-// operands, the order of the tiles over the XCDs, the epilogue and the
-// description of one product.
+// gemm_common.hpp -- what the bf16 product kernels (gemm.hip, gemm_ring.hpp)
+// share: types and conversions, the LDS layouts of staged operands, the order of
+// the tiles over the XCDs, the epilogue and the description of one product.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -4,9 +4,9 @@ the row, overlapping the one before it).
 
 Every lanes-per-row and slots-per-lane shape at odd widths, against float64 on
 the same inputs: y and inv_rms per element, dx against its row's scale, dgamma
-against the sum of its terms' magnitudes (fp32 sums of `rows` terms in any order:
-at most rows * 2^-24 of it, and the two-stage sum far less).  bf16 results carry
-one rounding (2^-9 relative) more.
+against the sum of its terms' magnitudes (fp32 sums of `rows` terms in any order err
+by at most rows * 2^-24 of it; column sums here add in fp64, fp32 only over aligned
+rows).  bf16 results carry one rounding (2^-9 relative) more.
 """
 import pytest
 
