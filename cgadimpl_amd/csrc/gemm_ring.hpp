@@ -9,8 +9,12 @@
 // through a ring of NST LDS stages filled by `buffer_load_dwordx4 ... lds`:
 // while tile t is multiplied the loads of tiles t + 1 .. t + NST - 1 are in
 // flight.  With tiles this small a k-step's MFMAs (0.1-0.3 us) are far shorter
-// than a load's latency (1-2 us), so what bounds the product is how many bytes
-// are in flight per CU; the deeper ring, or two workgroups per CU, gives them.
+// than a load's latency (1-2 us); the deeper ring, or two workgroups per CU, keeps
+// the bytes in flight that cover it.  Measured on MI355X: 1032 x 4096 x 4096 in 192 x
+// 128 tiles, the waves wait for 16 % of their cycles and the matrix cores of the 192
+// CUs with a tile are busy 44 % of the time at 2.4 GHz (the idle CUs and the lower
+// clock are the rest); 16 x 11008 x 4096 in 64 x 64 tiles, 57 % waiting, the weights read
+// at 5.2 TB/s.
 //
 // Step t: the fragments run one 16-deep substep ahead of the MFMAs, across the
 // barrier, as in the direct kernel.  At the end of the step each wave waits
